@@ -109,6 +109,7 @@ struct Plan {
     int upper_rows = 0;
     uint16_t qmask[kMaxK] = {};  // positions QEDGE(l)[1:]
     uint16_t smask[kMaxK] = {};  // positions s in SYM(l), s > 0
+    uint16_t above[kMaxK] = {};  // positions s with x_s < x_l in every candidate tuple (closure of smask)
 };
 
 std::unique_ptr<Plan> plan_from_edges(const uint32_t *src, const uint32_t *dst, uint64_t ne,

@@ -216,6 +216,9 @@ std::unique_ptr<Plan> plan_from_edges(const uint32_t *src, const uint32_t *dst, 
                 for (int b = 1; b < s; b++)
                     if (gt[s][b]) gt[l][b] = true;
             }
+    for (int l = 1; l < p->L; l++)
+        for (int s = 1; s < l; s++)
+            if (gt[l][s]) p->above[l] |= (uint16_t)(1u << s);
     bool upper = p->uses_bitmap != 0;
     for (int l = 2; l < p->L; l++)
         for (int q = 1; q < l; q++) {

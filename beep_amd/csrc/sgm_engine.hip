@@ -25,7 +25,7 @@ static_assert(sizeof(RootRec) == kRootRecBytes, "per-root record size");
 hipError_t launch_lds_batches(int lg, int cus, hipStream_t st, const KGraph &g, const KPlan &pl,
                               const RootRec *recs, const uint32_t *bf, const uint32_t *bc,
                               uint32_t b0, uint32_t b1, unsigned long long *cursor, const KOut &out,
-                              int *grid_out, bool dense = false);
+                              bool dense = false);
 hipError_t launch_hub_hash(int grid, hipStream_t st, const KGraph &g, const HubRec *hubs,
                            const uint32_t *hor, uint64_t g0, uint64_t g1, uint64_t *kv,
                            const unsigned long long *dl);
@@ -446,6 +446,44 @@ ScratchNeeds scratch_needs(const Prep &pp, const Plan &p, const beep_opts &o, in
     return n;
 }
 
+// Reduces level l (rows qm, bounds sm, all of them positions below `top`) to
+// what has to be applied on top of the set C_b of an earlier level b < l that
+// the walk holds: b's rows and bounds are part of l's, so C_l is a subset of
+// C_b but for b's exclusions, which l has too.  Of the rest, a bound or an
+// exclusion of x_s is dropped where another constraint implies it: x_l above
+// x_t >= x_s, or, over bitmaps without mirrored bits, x_l in the row of x_q
+// (whose bits lie above x_q) with x_q >= x_s; and the row of x_s does not hold
+// x_s itself.
+struct LevelWork {
+    uint32_t rq, rs, rx, base;
+};
+static LevelWork reduce_level(const Plan &p, int l, uint32_t qm, uint32_t sm, int top)
+{
+    LevelWork w{qm, 0, 0, 0};
+    for (int b = 2; b < l && b <= p.L - 2 && b <= top; b++) {
+        if ((p.qmask[b] & ~qm) || (p.smask[b] & ~sm)) continue;
+        const int left = __builtin_popcount(qm & ~(uint32_t)p.qmask[b]);
+        if (!w.base || left < __builtin_popcount(w.rq) || (left == __builtin_popcount(w.rq) && b > (int)w.base)) {
+            w.base = (uint32_t)b;
+            w.rq = qm & ~(uint32_t)p.qmask[b];
+        }
+    }
+    auto implied = [&](int s) {  // x_l > x_s without a bound on x_s
+        for (int t = 1; t < top; t++) {
+            if (((sm >> t) & 1u) && ((p.above[t] >> s) & 1u)) return true;
+            if (p.upper_rows && ((qm >> t) & 1u) && (t == s || ((p.above[t] >> s) & 1u))) return true;
+        }
+        return false;
+    };
+    for (int s = 1; s < top; s++) {
+        const bool in_base = w.base && ((p.smask[w.base] >> s) & 1u);
+        if (((sm >> s) & 1u) && !in_base && !implied(s)) w.rs |= 1u << s;
+        const bool apart = ((sm >> s) & 1u) || ((qm >> s) & 1u) || (w.base && s < (int)w.base) || implied(s);
+        if (!apart) w.rx |= 1u << s;
+    }
+    return w;
+}
+
 static KPlan make_kplan(const Plan &p, int emit, int build_mode)
 {
     KPlan k{};
@@ -461,6 +499,27 @@ static KPlan make_kplan(const Plan &p, int emit, int build_mode)
         k.qmask[l] = p.qmask[l];
         k.smask[l] = p.smask[l];
     }
+    k.nested = p.upper_rows && p.L >= 4 ? 1 : 0;
+    for (int l = 2; l < p.L; l++) {
+        if (p.qmask[l]) k.reads_rows = 1;
+        // a summed last level leaves its constraint on x_{L-2} to the sum
+        const bool summed = k.tail && l == p.L - 1;
+        const LevelWork w = reduce_level(p, l, p.qmask[l], summed ? p.smask[l] & ~(1u << (l - 1)) : p.smask[l],
+                                         summed ? l - 1 : l);
+        k.lev[l] = w.rq | w.rs << 16;
+        k.lev[kMaxLevels + l] = w.rx | w.base << 16;
+        if (w.rq != 1u << (l - 1) || w.rs || w.rx || (l > 2 && (int)w.base != l - 1)) k.nested = 0;
+    }
+    k.tail_gt = k.tail && ((p.smask[p.L - 1] >> (p.L - 2)) & 1u) ? 1 : 0;
+    if (emit == BEEP_EMIT_NONE && p.L == 3) k.closed = kClosedC;
+    if (k.tail && p.L == 4) {
+        if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 2u << 16) k.closed = k.tail_gt ? kClosedPairs : kClosedOrdered;
+        if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 1u << 1 && !k.tail_gt) k.closed = kClosedRow;
+    }
+    // levels an item walks below x_2: none (one pass over the row's words, or
+    // the count itself), one, two, or more
+    const int walked = p.L - (k.tail ? 1 : 0) - (k.pair ? 2 : 0) - 3;
+    k.chunk = walked <= 0 || (k.nested && p.L == 4) ? kNoSplit : walked == 1 ? 64u : walked == 2 ? 8u : 2u;
     return k;
 }
 
@@ -565,7 +624,7 @@ int enqueue_lds_classes(const Prep &pp, const LaunchCfg &c, const Scratch &s, hi
         if (cls >= 32) throw Error(BEEP_ERANGE, "too many lane classes");
         unsigned long long *cur = s.ctr + kCtrLds + (uint64_t)cls * kCurWords;
         HIP_CHECK(launch_lds_batches(lg, pp.dev->cus, streams[cls % nst], c.kg, c.kp, R.recs, R.batch_first,
-                                     R.batch_count, b, e, cur, c.out, nullptr));
+                                     R.batch_count, b, e, cur, c.out));
         if (cls_done) {
             HIP_CHECK(hipEventRecord(cls_done[cls], streams[cls % nst]));
             cls_lg[cls] = (uint8_t)lg;
@@ -674,7 +733,7 @@ void enqueue_query(const Prep &pp, const LaunchCfg &c, const Scratch &s, Lane &l
         // for 7 workgroups per CU
         HIP_CHECK(hipEventRecord(lane.cls_start[i], sk));
         HIP_CHECK(launch_lds_batches(lc.lg, pp.dev->cus, sk, c.kg, c.kp, R.recs, R.batch_first, R.batch_count,
-                                     lc.b0, lc.b1, cur, c.out, nullptr, !hubs));
+                                     lc.b0, lc.b1, cur, c.out, !hubs));
         HIP_CHECK(hipEventRecord(lane.cls_done[i], sk));
         lane.cls_lg[i] = (uint8_t)lc.lg;
         if (n == 0) {
@@ -818,7 +877,6 @@ struct Batch {
     MultiQuery *dqs = nullptr;
     MultiWork *dwork = nullptr;
     uint32_t nwork = 0;
-    uint32_t nlev = 1;
     // lane classes: work records [cls_w0, cls_w1) of width cls_lg, one launch
     // and one striped cursor (kCurWords words) each
     std::vector<int> cls_lg;
@@ -850,7 +908,7 @@ struct Batch {
 };
 
 hipError_t launch_lds_multi(int cus, hipStream_t st, const MultiQuery *qs, const MultiWork *work, uint32_t nwork,
-                            unsigned long long *cursor, uint32_t nlev, int lg, int *grid_out);
+                            unsigned long long *cursor, uint32_t stack_words, int levels, int lg);
 
 Batch *batch_create(Prep *const *preps, const Plan *const *plans, const beep_opts *opts, int n)
 {
@@ -879,7 +937,6 @@ Batch *batch_create(Prep *const *preps, const Plan *const *plans, const beep_opt
             b->cfgs.push_back(make_launch(pp, *plans[i], opts[i], b->scr.back(), d.cus));
             const LaunchCfg &c = b->cfgs.back();
             qs[i] = MultiQuery{c.kg, c.kp, d.roots.recs, d.roots.batch_first, d.roots.batch_count, c.out};
-            b->nlev = std::max<uint32_t>(b->nlev, (uint32_t)c.nlev);
             for (uint32_t bi = 0; c.kp.L >= 3 && bi < (uint32_t)pp.batches.size(); bi++) {
                 const LdsBatch &lb = pp.batches[bi];
                 uint64_t cost = 0;
@@ -952,9 +1009,15 @@ static void batch_capture(Batch &b)
     }
     for (int k = 0; k < ncls; k++) {
         hipStream_t sk = b.branch[n + k];
+        uint32_t words = 1;
+        int levels = 3;
+        for (const LaunchCfg &c : b.cfgs) {
+            words = std::max(words, lds_stack_words(c.kp, b.cls_lg[k]));
+            levels = std::max(levels, (int)c.kp.L);
+        }
         HIP_CHECK(hipStreamWaitEvent(sk, b.fork, 0));
         HIP_CHECK(launch_lds_multi(d0.cus, sk, b.dqs, b.dwork + b.cls_w0[k], b.cls_w1[k] - b.cls_w0[k],
-                                   b.cursor + (uint64_t)k * kCurWords, b.nlev, b.cls_lg[k], nullptr));
+                                   b.cursor + (uint64_t)k * kCurWords, words, levels, b.cls_lg[k]));
         HIP_CHECK(hipEventRecord(b.done[n + k], sk));
     }
     for (int i = 0; i < n + ncls; i++) HIP_CHECK(hipStreamWaitEvent(b.s0, b.done[i], 0));

@@ -244,17 +244,17 @@ __device__ __forceinline__ bool claim_striped(unsigned long long *cur, uint64_t 
     return false;
 }
 
+// Hash of an empty prefix of a tuple of `len` vertices.
+__device__ __forceinline__ uint64_t hash_seed(int len) { return 0x6a09e667f3bcc909ull ^ (uint64_t)len; }
+
 // Emits the tuples (u, A[x_1], ..., A[x_{l-1}], A[i]) for every bit i of word
-// w of the last level: hash accumulation and optional buffer append.
+// w of the last level: hash accumulation and optional buffer append.  h is the
+// hash of the first l entries.
 template <class XGet>
-__device__ __forceinline__ void emit_word(const KOut &out, const KPlan &pl, int l, uint32_t u,
-                                          const uint32_t *A, uint64_t t, uint32_t w, XGet xget,
-                                          uint64_t &hs, uint64_t &hx)
+__device__ __forceinline__ void emit_bits(const KOut &out, int l, uint32_t u, const uint32_t *A, uint64_t h,
+                                          uint64_t t, uint32_t w, XGet xget, uint64_t &hs, uint64_t &hx)
 {
     const int len = l + 1;
-    uint64_t h = 0x6a09e667f3bcc909ull ^ (uint64_t)len;
-    h = hash_step(h, 0, u);
-    for (int q = 1; q < l; q++) h = hash_step(h, q, A[xget(q)]);
     uint64_t base = 0;
     if (out.buf) base = atomicAdd(&out.acc[3], (unsigned long long)__popcll(t));
     uint64_t idx = 0;
@@ -275,6 +275,16 @@ __device__ __forceinline__ void emit_word(const KOut &out, const KPlan &pl, int 
     }
 }
 
+template <class XGet>
+__device__ __forceinline__ void emit_word(const KOut &out, const KPlan &pl, int l, uint32_t u,
+                                          const uint32_t *A, uint64_t t, uint32_t w, XGet xget,
+                                          uint64_t &hs, uint64_t &hx)
+{
+    uint64_t h = hash_step(hash_seed(l + 1), 0, u);
+    for (int q = 1; q < l; q++) h = hash_step(h, q, A[xget(q)]);
+    emit_bits(out, l, u, A, h, t, w, xget, hs, hx);
+}
+
 __device__ __forceinline__ bool use_search(uint32_t hlen, uint32_t d, uint32_t ratio)
 {
     return (uint64_t)hlen > (uint64_t)d * ratio;
@@ -284,37 +294,36 @@ __device__ __forceinline__ bool use_search(uint32_t hlen, uint32_t d, uint32_t r
 
 struct LdsLayout {
     uint32_t oE, oHBeg, oStk, oA, oPre, oHKey, oRoot, oHVal, oX, oJRoot, oMisc, bytes;
-    uint32_t ewords, nlev;
+    uint32_t ewords;
 };
 
 __host__ __device__ inline uint32_t align_up(uint32_t x, uint32_t a) { return (x + a - 1) / a * a; }
 
-// Layout of lane class lg's batches (the widest class serves every batch);
-// nlev + 3 >= L positions of x are kept per thread.
-__host__ inline LdsLayout make_lds_layout(int lg, uint32_t nlev)
+// Layout of lane class lg's batches; stack_words words of DFS stack and
+// `levels` positions of x are kept per thread.
+__host__ inline LdsLayout make_lds_layout(int lg, uint32_t stack_words, int levels)
 {
     const uint32_t sd = LdsBudget::sumdeg(lg), hs = LdsBudget::hash(lg), ew = LdsBudget::ewords(lg);
     LdsLayout L{};
     uint32_t o = 0;
     L.ewords = ew;
-    L.nlev = nlev;
     L.oE = o;       o += ew * 8;
     L.oHBeg = o;    o += sd * 8;
-    L.oStk = o;     o += nlev * kBlock * 8;
+    L.oStk = o;     o += stack_words * kBlock * 8;
     L.oRoot = o;    o += LdsBudget::kMaxRoots * (uint32_t)sizeof(RootRec);
     L.oA = o;       o += sd * 4;
     L.oPre = o;     o += align_up((sd + 1) * 4, 8);
     L.oHKey = o;    o += hs * 4;
     L.oMisc = o;    o += 32 * 4;
     L.oHVal = o;    o += hs * 2;
-    L.oX = o;       o += (nlev + 3) * kBlock * 2;
+    L.oX = o;       o += (uint32_t)levels * kBlock * 2;
     L.oJRoot = o;   o += sd;
     L.bytes = align_up(o, 16);
     return L;
 }
 
 // Misc slots
-enum { M_BATCH = 0, M_NEXT = 1, M_QM = 4, M_SM = 14 };
+enum { M_BATCH = 0, M_NEXT = 1, M_LEV = 4 };  // M_LEV: 2 kMaxLevels words (KPlan::lev); 28..31: scan
 
 // Block-wide exclusive scan of a[0..n) in place (n <= 4 * kBlock); a[n] = total.
 __device__ void block_excl_scan(uint32_t *a, uint32_t n, uint32_t *tmp4)
@@ -368,32 +377,458 @@ __device__ __forceinline__ LdsView lds_view(unsigned char *smem, const LdsLayout
     return v;
 }
 
-// Processes one LDS batch: stage rows, hash and bitmaps, then the DFS over
-// its (root, x_1) items.  PC > 0 fixes the group width at compile time; PC == 0
-// takes it from Prt.  The plan's level masks are in sMisc[M_QM..], [M_SM..].
-template <int PC>
-__device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v,
-                              const RootRec *__restrict__ recs, uint32_t first, uint32_t nr,
-                              const KOut &out, uint64_t dl, int Prt, uint64_t &cnt, uint64_t &hs,
-                              uint64_t &hx)
+// Rows whose index range holds item e: the largest j with pre[j] <= e (pre
+// ascends, pre[n] > e).
+__device__ __forceinline__ uint32_t find_row(const uint32_t *pre, uint32_t n, uint32_t e)
 {
-    const int P = PC > 0 ? PC : Prt;
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (pre[mid] <= e) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// The n lowest set bits of v (n <= popcount).
+__device__ __forceinline__ uint64_t low_bits(uint64_t v, uint32_t n)
+{
+    uint64_t r = v;
+    for (uint32_t i = 0; i < n; i++) r &= r - 1;
+    return v ^ r;
+}
+
+__device__ __forceinline__ bool whole_rows(const KPlan &pl)
+{
+    return pl.chunk == kNoSplit && !pl.closed && !pl.nested;
+}
+
+// DFS items of a batch, once its bitmaps are there: row j (x_1 = j of its root)
+// gives ceil(|C_2| / chunk) items, each the x_2 of `chunk` consecutive
+// candidates, so a row with many candidates under a deep plan is walked by
+// many lanes and an x_1 without candidates by none.  Leaves the rows' item
+// offsets in sPre (sPre[sumd] = the number of items, also returned).  Plans whose
+// count follows from |C_2| (KPlan::closed) are counted right here (no items),
+// and where an item is a whole x_1 the rows themselves are the items.
+//
+// Why: with one item per x_1, a lane's serial chain under a 6-clique's x_1 ran
+// 40 ms (R-MAT scale 17) while the GPU idled: mean/max workgroup time 0.07.
+__device__ uint32_t lds_items(const KPlan &pl, const LdsView &v, uint32_t sumd, uint64_t &cnt)
+{
+    const int L = pl.L;
+    if (whole_rows(pl)) return sumd;
+    const bool row1 = (pl.qmask[2] & 2u) != 0, above = (pl.smask[2] & 2u) != 0;
+    const uint32_t need = pl.nested ? (uint32_t)L - 2u : 1u;  // a clique's x_2..x_{L-1} all lie in C_2
+    for (uint32_t j = threadIdx.x; j < sumd; j += kBlock) {
+        const RootRec rr = v.sRoot[v.sJRoot[j]];
+        const uint32_t jl = j - rr.doff, d = rr.d, W = (d + 63) >> 6;
+        uint32_t c2 = 0;
+        // x_1..x_{L-1} are distinct row entries
+        if (!(pl.skip_split && jl < rr.split) && d + 1u >= (uint32_t)L) {
+            if (row1) {
+                const uint64_t *E = v.sE + rr.eoff + jl * W;
+                for (uint32_t w = above ? jl >> 6 : 0u; w < W; w++)
+                    c2 += (uint32_t)__popcll(above ? E[w] & gt_mask(jl, w) : E[w]);
+            } else {
+                c2 = above ? d - 1u - jl : d - 1u;
+            }
+        }
+        if (pl.closed) cnt += c2 ? closed_count(pl.closed, c2, d) : 0ull;
+        else v.sPre[j] = c2 < need ? 0u : pl.chunk == kNoSplit ? 1u : (c2 + pl.chunk - 1u) / pl.chunk;
+    }
+    if (pl.closed) return 0;
+    __syncthreads();
+    block_excl_scan(v.sPre, sumd, v.sMisc + 28);
+    return v.sPre[sumd];
+}
+
+// Plans whose levels nest (KPlan::nested, cliques): every lane walks items of
+// its own and holds all WT words of the current level's set in registers, so a
+// step is one row read, WT ANDs and popcounts and no cross-lane traffic.
+// E[x] holds bits above x only, so the candidates not yet taken are the whole
+// set as far as the next level is concerned: one set per level is kept, in
+// registers for the current level and in the LDS stack above it.
+//
+// Lanes of a wave are at different depths.  Each round first brings every lane
+// that ran out of candidates to its next last-level set (climb, claim,
+// descend), then steps all lanes through their sets until half of the lanes
+// that still have work are out of candidates: the two phases' instructions are
+// then paid by at least half of the lanes they serve.
+template <int WT, bool EMIT>
+__device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uint32_t items, const KOut &out,
+                            uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
+{
+    const int tid = threadIdx.x;
+    const int L = pl.L;
+    uint64_t *stk = v.sStk + tid;  // word k of level l's set: stk[((l - 3) * WT + k) * kBlock]
+    uint16_t *sX = v.sX;
+    auto xget = [&](int q) -> uint32_t { return sX[q * kBlock + tid]; };
+    uint64_t S[WT];
+#pragma unroll
+    for (int k = 0; k < WT; k++) S[k] = 0ull;
+    int l = 3;             // S = what is left of C_{l-1}; x_{l-1} is taken next
+    uint32_t left = 0;     // x_2's of the item not yet taken
+    bool live = true;
+    const uint64_t *E = v.sE;
+    const uint32_t *A = v.sA;
+    uint32_t W = 1, u = 0;
+    uint32_t rounds = 0;
+    uint64_t hpre = 0;  // EMIT: hash of u, x_1..x_{L-3}
+    auto any = [&]() -> bool {
+        uint64_t o = S[0];
+#pragma unroll
+        for (int k = 1; k < WT; k++) o |= S[k];
+        return o != 0ull;
+    };
+    // takes the smallest candidate out of S (not empty)
+    auto take = [&]() -> uint32_t {
+        uint32_t k0 = 0;
+        uint64_t c = S[0];
+#pragma unroll
+        for (int k = 1; k < WT; k++)
+            if (c == 0ull) {
+                c = S[k];
+                k0 = k;
+            }
+#pragma unroll
+        for (int k = 0; k < WT; k++)
+            if ((uint32_t)k == k0) S[k] = c & (c - 1ull);
+        return (k0 << 6) + (uint32_t)__builtin_ctzll(c);
+    };
+    for (;;) {
+        // ---- bring every lane to a last-level set
+        while (live && !(l == L - 1 && any())) {
+            if (l > 3 && !any()) {  // climb
+                --l;
+#pragma unroll
+                for (int k = 0; k < WT; k++) S[k] = stk[((l - 3) * WT + k) * kBlock];
+            } else if (l == 3 && (left == 0 || !any())) {  // claim
+                // one LDS atomic for the lanes that claim together
+                const uint64_t m = __ballot(1);
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                uint32_t first = 0;
+                if (rank == 0) first = atomicAdd(&v.sMisc[M_NEXT], (uint32_t)__popcll(m));
+                const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + rank;
+                if (item >= items) {
+                    live = false;
+#pragma unroll
+                    for (int k = 0; k < WT; k++) S[k] = 0ull;
+                } else {
+                    const uint32_t row = find_row(v.sPre, sumd, item);
+                    const RootRec rr = v.sRoot[v.sJRoot[row]];
+                    const uint32_t jl = row - rr.doff;
+                    W = (rr.d + 63) >> 6;
+                    E = v.sE + rr.eoff;
+                    uint32_t skip = 0;
+                    left = 0xffffffffu;
+                    if (pl.chunk != kNoSplit) {
+                        skip = (item - v.sPre[row]) * pl.chunk;
+                        left = pl.chunk;
+                    }
+#pragma unroll
+                    for (int k = 0; k < WT; k++) {
+                        uint64_t c = (uint32_t)k < W ? E[jl * W + k] : 0ull;
+                        if (skip) {
+                            const uint32_t pc = (uint32_t)__popcll(c);
+                            const uint32_t drop = skip < pc ? skip : pc;
+                            c ^= low_bits(c, drop);
+                            skip -= drop;
+                        }
+                        S[k] = c;
+                    }
+                    if (EMIT) {
+                        A = v.sA + rr.doff;
+                        u = rr.u;
+                        sX[1 * kBlock + tid] = (uint16_t)jl;
+                        if (L == 4) hpre = hash_step(hash_step(hash_seed(L), 0, u), 1, A[jl]);
+                    }
+                }
+            } else {  // descend: l < L - 1 and a candidate is left
+                const uint32_t x = take();
+                if (l == 3) left--;
+                uint64_t t[WT];
+                uint32_t pc = 0;
+#pragma unroll
+                for (int k = 0; k < WT; k++) {
+                    t[k] = S[k] & E[x * W + k];  // past the row's words S is 0
+                    pc += (uint32_t)__popcll(t[k]);
+                }
+                if (pc >= (uint32_t)(L - l)) {  // enough for x_l..x_{L-1}
+#pragma unroll
+                    for (int k = 0; k < WT; k++) {
+                        stk[((l - 3) * WT + k) * kBlock] = S[k];
+                        S[k] = t[k];
+                    }
+                    ++l;
+                    if (EMIT) {
+                        sX[(l - 2) * kBlock + tid] = (uint16_t)x;
+                        if (l == L - 1) {
+                            hpre = hash_step(hash_seed(L), 0, u);
+                            for (int q = 1; q < L - 2; q++) hpre = hash_step(hpre, q, A[xget(q)]);
+                        }
+                    }
+                }
+            }
+        }
+        const uint32_t alive = (uint32_t)__popcll(__ballot(live));
+        if (alive == 0) break;
+        if ((++rounds & 255u) == 0u && past(dl)) {
+            mark_stop(out);
+            break;
+        }
+        // ---- last level: add |S n E[x]| for every x in S
+        for (;;) {
+            const bool on = any();
+            if (2u * (uint32_t)__popcll(__ballot(on)) < alive + 1u) break;
+            if (on) {
+                const uint32_t x = take();
+                const uint64_t *Ex = E + x * W;
+                uint32_t pc = 0;
+#pragma unroll
+                for (int k = 0; k < WT; k++) {
+                    const uint64_t t = S[k] & Ex[k];
+                    pc += (uint32_t)__popcll(t);
+                    if (EMIT && t) {
+                        if (out.buf) sX[(L - 2) * kBlock + tid] = (uint16_t)x;
+                        emit_bits(out, L - 1, u, A, hash_step(hpre, L - 2, A[x]), t, (uint32_t)k, xget, hs, hx);
+                    }
+                }
+                cnt += pc;
+            }
+        }
+    }
+}
+
+// DFS over the items of a batch, P lanes an item: lane i of the group owns word
+// i of every set, the next candidate is one ballot over the group's words, and
+// the sets of the levels above are kept in the thread's LDS stack.
+template <int P>
+__device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uint32_t items, const KOut &out,
+                           uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
+{
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int lx = lane & (P - 1);
     const int pbase = lane & ~(P - 1);
     const int L = pl.L;
+    uint64_t *sStk = v.sStk;
+    uint32_t *sMisc = v.sMisc;
+    uint16_t *sX = v.sX;
+    auto xget = [&](int q) -> uint32_t { return sX[q * kBlock + tid]; };
+    uint32_t spins = 0;
+    for (;;) {
+        uint32_t item = 0;
+        if (lx == 0) {
+            if (past(dl)) {
+                item = 0xffffffffu;
+                mark_stop(out);
+            } else {
+                item = atomicAdd(&sMisc[M_NEXT], 1u);
+            }
+        }
+        item = __shfl(item, 0, P);
+        if (item >= items) break;
+        const bool whole = whole_rows(pl);
+        const uint32_t row = whole ? item : find_row(v.sPre, sumd, item);
+        const RootRec rr = v.sRoot[v.sJRoot[row]];
+        const uint32_t jl = row - rr.doff;
+        if (whole && ((pl.skip_split && jl < rr.split) || rr.d + 1u < (uint32_t)L)) continue;
+        const uint32_t skip = whole ? 0u : (item - v.sPre[row]) * pl.chunk;
+        const uint32_t d = rr.d, W = (d + 63) >> 6;
+        const uint64_t *E = v.sE + rr.eoff;
+        const uint32_t *A = v.sA + rr.doff;
+        const uint32_t w = (uint32_t)lx;
+        const bool own = w < W;
+        sX[1 * kBlock + tid] = (uint16_t)jl;
+
+        // C_l from the set of its base level (KPlan::lev)
+        auto level_word = [&](int l) -> uint64_t {
+            const uint32_t a = sMisc[M_LEV + l], b = sMisc[M_LEV + kMaxLevels + l];
+            uint64_t t = b >> 16 ? sStk[((b >> 16) - 2) * kBlock + tid] : valid_mask(w, d);
+            uint32_t m = b & 0xffffu;
+            while (m) {
+                const int s = __builtin_ctz(m);
+                m &= m - 1;
+                t &= ~bit_at(xget(s), w);
+            }
+            m = a >> 16;
+            while (m) {
+                const int s = __builtin_ctz(m);
+                m &= m - 1;
+                t &= gt_mask(xget(s), w);
+            }
+            m = a & 0xffffu;
+            while (m && t) {  // no row reads once the word is empty
+                const int q = __builtin_ctz(m);
+                m &= m - 1;
+                t &= E[xget(q) * W + w];
+            }
+            return t;
+        };
+
+        // Summed last level (pl.tail): F = the part of C_{L-1} fixed by
+        // x_1..x_{L-3}; for x_{L-2} = x, |C_{L-1}| = |F n (x, inf)| when
+        // L-2 is in smask[L-1], else |F \ {x}|.  Summed over x in S = C_{L-2}:
+        //   sum_w [ |S_w| (|F| - |F_{<=w}|) + pairs_w(S, F) ]  or  |S||F| - |S n F|
+        // with one group prefix sum of |F_w|.
+        auto tail_sum = [&](int l) -> uint64_t {
+            const uint64_t S = own ? sStk[(l - 3) * kBlock + tid] : 0ull;
+            const uint64_t F = own ? level_word(l) : 0ull;
+            const uint32_t sc = (uint32_t)__popcll(S);
+            uint32_t fin = (uint32_t)__popcll(F);
+            for (int o = 1; o < P; o <<= 1) {
+                const uint32_t y = __shfl_up(fin, o, P);
+                if (lx >= o) fin += y;
+            }
+            const uint32_t ftot = __shfl(fin, P - 1, P);
+            if (pl.tail_gt) return (uint64_t)sc * (ftot - fin) + pairs_in_word(S, F);
+            return (uint64_t)sc * ftot - (uint64_t)__popcll(S & F);
+        };
+
+        // Paired last levels (pl.pair), l = L-2 = b: S = C_{l-1} = C_a with
+        // x_1..x_{a-1} fixed; adds C(|S n E[x_b]|, 2) over x_b in B, the
+        // candidates of level b without its constraints on x_a.  Only an x_b
+        // adjacent to some member of S can add anything, so B is first cut to
+        // the union of their rows.
+        auto pair_sum = [&](int l) -> uint64_t {
+            const uint64_t S = own ? sStk[(l - 3) * kBlock + tid] : 0ull;
+            uint64_t U = 0;
+            for (uint64_t rem = S;;) {
+                const uint64_t bal = __ballot(rem != 0ull);
+                const uint64_t mine = (P == 64) ? bal : ((bal >> pbase) & ((1ull << P) - 1ull));
+                if (mine == 0ull) break;
+                const int f = __builtin_ctzll(mine);
+                const uint64_t vf = __shfl(rem, f, P);
+                const uint32_t xs = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
+                if (lx == f) rem &= rem - 1ull;
+                if (own) U |= E[xs * W + w];
+            }
+            uint64_t B = 0;
+            if (own) {
+                B = valid_mask(w, d) & U;
+                uint32_t qm = pl.qmask[l] & ~(1u << (l - 1));
+                while (qm) {
+                    const int q = __builtin_ctz(qm);
+                    qm &= qm - 1;
+                    B &= E[xget(q) * W + w];
+                }
+                for (int s = 1; s < l - 1; s++) B &= ~bit_at(xget(s), w);
+                uint32_t sm = pl.smask[l];
+                while (sm) {
+                    const int s = __builtin_ctz(sm);
+                    sm &= sm - 1;
+                    B &= gt_mask(xget(s), w);
+                }
+            }
+            uint64_t sum = 0;
+            for (;;) {
+                const uint64_t bal = __ballot(B != 0ull);
+                const uint64_t mine = (P == 64) ? bal : ((bal >> pbase) & ((1ull << P) - 1ull));
+                if (mine == 0ull) break;
+                const int f = __builtin_ctzll(mine);
+                const uint64_t vf = __shfl(B, f, P);
+                const uint32_t xb = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
+                if (lx == f) B &= B - 1ull;  // lane f's lowest bit is x_b
+                uint32_t pc = own ? (uint32_t)__popcll(S & E[xb * W + w]) : 0u;
+                for (int o = 1; o < P; o <<= 1) pc += __shfl_xor(pc, o, P);
+                if (lx == 0) sum += (uint64_t)pc * (pc - 1u) / 2u;
+            }
+            return sum;
+        };
+
+        const uint64_t t2 = own ? level_word(2) : 0ull;
+        if (L == 3) {
+            cnt += (uint64_t)__popcll(t2);
+            if (pl.emit && t2) emit_word(out, pl, 2, rr.u, A, t2, w, xget, hs, hx);
+            continue;
+        }
+        sStk[tid] = t2;
+        // the item's x_2: the candidates of rank [skip, skip + chunk) in C_2
+        uint64_t x2s = t2;
+        if (pl.chunk != kNoSplit) {
+            const uint32_t pc = (uint32_t)__popcll(t2);
+            uint32_t before = pc;
+            for (int o = 1; o < P; o <<= 1) {
+                const uint32_t y = __shfl_up(before, o, P);
+                if (lx >= o) before += y;
+            }
+            before -= pc;
+            uint32_t drop = skip > before ? skip - before : 0u;
+            uint32_t end = skip + pl.chunk > before ? skip + pl.chunk - before : 0u;
+            if (drop > pc) drop = pc;
+            if (end > pc) end = pc;
+            x2s = end > drop ? low_bits(t2, end) & ~low_bits(t2, drop) : 0ull;
+        }
+        int l = 3;
+        uint32_t pos = 0;
+        for (;;) {
+            if (++spins == kClockEvery) {
+                spins = 0;
+                if (past(dl)) break;  // the next claim records the stop
+            }
+            if (pl.tail && l == L - 1) {  // every x_{L-2} of C_{L-2} at once
+                cnt += tail_sum(l);
+                if (l == 3) break;
+                --l;
+                pos = (uint32_t)xget(l - 1) + 1u;
+                continue;
+            }
+            if (pl.pair && l == L - 2) {  // levels L-3..L-1 at once
+                cnt += pair_sum(l);
+                if (l == 3) break;
+                --l;
+                pos = (uint32_t)xget(l - 1) + 1u;
+                continue;
+            }
+            uint64_t vv = l == 3 ? x2s : own ? sStk[(l - 3) * kBlock + tid] : 0ull;
+            const uint32_t pw = pos >> 6;
+            if (w < pw) vv = 0ull;
+            else if (w == pw) vv &= (~0ull << (pos & 63u));
+            const uint64_t bal = __ballot(vv != 0ull);
+            const uint64_t mine = (P == 64) ? bal : ((bal >> pbase) & ((1ull << P) - 1ull));
+            if (mine == 0ull) {
+                if (l == 3) break;
+                --l;
+                pos = (uint32_t)xget(l - 1) + 1u;
+                continue;
+            }
+            const int f = __builtin_ctzll(mine);
+            const uint64_t vf = __shfl(vv, f, P);
+            const uint32_t xi = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
+            sX[(l - 1) * kBlock + tid] = (uint16_t)xi;
+            const uint64_t t = own ? level_word(l) : 0ull;
+            if (l == L - 1) {
+                cnt += (uint64_t)__popcll(t);
+                if (pl.emit && t) emit_word(out, pl, l, rr.u, A, t, w, xget, hs, hx);
+                pos = xi + 1u;
+            } else {
+                sStk[(l - 2) * kBlock + tid] = t;
+                ++l;
+                pos = 0;
+            }
+        }
+    }
+}
+
+// Processes one LDS batch: stage rows, hash and bitmaps, then the DFS over
+// its items (lds_items).  The plan's level records are in sMisc[M_LEV..].
+// WALK fixes the walk at compile time where the launch serves one plan (the
+// walks need different registers); kWalkAny picks it per plan.
+enum { kWalkAny = 0, kWalkGroup = 1, kWalkLane = 2, kWalkLaneEmit = 3, kWalkNone = 4 };
+template <int PC, int WALK>
+__device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v,
+                              const RootRec *__restrict__ recs, uint32_t first, uint32_t nr,
+                              const KOut &out, uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
+{
+    const int tid = threadIdx.x;
+    const int L = pl.L;
     uint64_t *sE = v.sE;
     uint64_t *sHBeg = v.sHBeg;
-    uint64_t *sStk = v.sStk;
     RootRec *sRoot = v.sRoot;
     uint32_t *sA = v.sA, *sPre = v.sPre, *sHKey = v.sHKey, *sMisc = v.sMisc;
-    uint16_t *sHVal = v.sHVal, *sX = v.sX;
+    uint16_t *sHVal = v.sHVal;
     uint8_t *sJRoot = v.sJRoot;
-    auto xget = [&](int q) -> uint32_t { return sX[q * kBlock + tid]; };
     // bitmaps are built only when some level intersects with a bitmap row
-    bool needE = false;
-    for (int l = 2; l < L; l++) needE |= sMisc[M_QM + l] != 0u;
+    const bool needE = pl.reads_rows != 0;
     const uint64_t t_build = wall_clock64();
 
     if (tid < (int)nr) sRoot[tid] = recs[first + tid];
@@ -566,199 +1001,25 @@ __device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v
 
     if (tid == 0) prof_add(out, 3, blockIdx.x, t_build);  // staging + bitmap build
 
-    // DFS over (root, x_1) items
-    uint32_t spins = 0;
-    for (;;) {
-        uint32_t item = 0;
-        if (lx == 0) {
-            if (past(dl)) {
-                item = 0xffffffffu;
-                mark_stop(out);
-            } else {
-                item = atomicAdd(&sMisc[M_NEXT], 1u);
-            }
-        }
-        item = __shfl(item, 0, P);
-        if (item >= sumd) break;
-        const RootRec rr = sRoot[sJRoot[item]];
-        const uint32_t jl = item - rr.doff;
-        if (pl.skip_split && jl < rr.split) continue;
-        if (L < 3) continue;
-        const uint32_t d = rr.d, W = (d + 63) >> 6;
-        const uint64_t *E = sE + rr.eoff;
-        const uint32_t *A = sA + rr.doff;
-        const uint32_t w = (uint32_t)lx;
-        const bool own = w < W;
-        sX[1 * kBlock + tid] = (uint16_t)jl;
-
-        auto level_word = [&](int l) -> uint64_t {  // masks first; no row reads once empty
-            uint64_t t = valid_mask(w, d);
-            for (int s = 1; s < l; s++) t &= ~bit_at(xget(s), w);
-            uint32_t sm = sMisc[M_SM + l];
-            while (sm) {
-                const int s = __builtin_ctz(sm);
-                sm &= sm - 1;
-                t &= gt_mask(xget(s), w);
-            }
-            uint32_t qm = sMisc[M_QM + l];
-            while (qm && t) {
-                const int q = __builtin_ctz(qm);
-                qm &= qm - 1;
-                t &= E[xget(q) * W + w];
-            }
-            return t;
-        };
-
-        // Summed last level (pl.tail): F = the part of C_{L-1} fixed by
-        // x_1..x_{L-3}; for x_{L-2} = x, |C_{L-1}| = |F n (x, inf)| when
-        // L-2 is in smask[L-1], else |F \ {x}|.  Summed over x in S = C_{L-2}:
-        //   sum_w [ |S_w| (|F| - |F_{<=w}|) + pairs_w(S, F) ]  or  |S||F| - |S n F|
-        // with one group prefix sum of |F_w|.
-        auto tail_sum = [&](int l) -> uint64_t {
-            const int lv = l - 1;
-            const uint64_t S = own ? sStk[(l - 3) * kBlock + tid] : 0ull;
-            uint64_t F = 0;
-            if (own) {
-                F = valid_mask(w, d);
-                uint32_t qm = sMisc[M_QM + l];
-                while (qm) {
-                    const int q = __builtin_ctz(qm);
-                    qm &= qm - 1;
-                    F &= E[xget(q) * W + w];
-                }
-                for (int s = 1; s < lv; s++) F &= ~bit_at(xget(s), w);
-                uint32_t sm = sMisc[M_SM + l] & ~(1u << lv);
-                while (sm) {
-                    const int s = __builtin_ctz(sm);
-                    sm &= sm - 1;
-                    F &= gt_mask(xget(s), w);
-                }
-            }
-            const uint32_t sc = (uint32_t)__popcll(S);
-            uint32_t fin = (uint32_t)__popcll(F);
-            for (int o = 1; o < P; o <<= 1) {
-                const uint32_t y = __shfl_up(fin, o, P);
-                if (lx >= o) fin += y;
-            }
-            const uint32_t ftot = __shfl(fin, P - 1, P);
-            if ((sMisc[M_SM + l] >> lv) & 1u) return (uint64_t)sc * (ftot - fin) + pairs_in_word(S, F);
-            return (uint64_t)sc * ftot - (uint64_t)__popcll(S & F);
-        };
-
-        // Paired last levels (pl.pair), l = L-2 = b: S = C_{l-1} = C_a with
-        // x_1..x_{a-1} fixed; adds C(|S n E[x_b]|, 2) over x_b in B, the
-        // candidates of level b without its constraints on x_a.  Only an x_b
-        // adjacent to some member of S can add anything, so B is first cut to
-        // the union of their rows.
-        auto pair_sum = [&](int l) -> uint64_t {
-            const uint64_t S = own ? sStk[(l - 3) * kBlock + tid] : 0ull;
-            uint64_t U = 0;
-            for (uint64_t rem = S;;) {
-                const uint64_t bal = __ballot(rem != 0ull);
-                const uint64_t mine = (P == 64) ? bal : ((bal >> pbase) & ((1ull << P) - 1ull));
-                if (mine == 0ull) break;
-                const int f = __builtin_ctzll(mine);
-                const uint64_t vf = __shfl(rem, f, P);
-                const uint32_t xs = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
-                if (lx == f) rem &= rem - 1ull;
-                if (own) U |= E[xs * W + w];
-            }
-            uint64_t B = 0;
-            if (own) {
-                B = valid_mask(w, d) & U;
-                uint32_t qm = sMisc[M_QM + l] & ~(1u << (l - 1));
-                while (qm) {
-                    const int q = __builtin_ctz(qm);
-                    qm &= qm - 1;
-                    B &= E[xget(q) * W + w];
-                }
-                for (int s = 1; s < l - 1; s++) B &= ~bit_at(xget(s), w);
-                uint32_t sm = sMisc[M_SM + l];
-                while (sm) {
-                    const int s = __builtin_ctz(sm);
-                    sm &= sm - 1;
-                    B &= gt_mask(xget(s), w);
-                }
-            }
-            uint64_t sum = 0;
-            for (;;) {
-                const uint64_t bal = __ballot(B != 0ull);
-                const uint64_t mine = (P == 64) ? bal : ((bal >> pbase) & ((1ull << P) - 1ull));
-                if (mine == 0ull) break;
-                const int f = __builtin_ctzll(mine);
-                const uint64_t vf = __shfl(B, f, P);
-                const uint32_t xb = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
-                if (lx == f) B &= B - 1ull;  // lane f's lowest bit is x_b
-                uint32_t pc = own ? (uint32_t)__popcll(S & E[xb * W + w]) : 0u;
-                for (int o = 1; o < P; o <<= 1) pc += __shfl_xor(pc, o, P);
-                if (lx == 0) sum += (uint64_t)pc * (pc - 1u) / 2u;
-            }
-            return sum;
-        };
-
-        const uint64_t t2 = own ? level_word(2) : 0ull;
-        if (L == 3) {
-            cnt += (uint64_t)__popcll(t2);
-            if (pl.emit && t2) emit_word(out, pl, 2, rr.u, A, t2, w, xget, hs, hx);
-            continue;
-        }
-        sStk[tid] = t2;
-        int l = 3;
-        uint32_t pos = 0;
-        for (;;) {
-            if (++spins == kClockEvery) {
-                spins = 0;
-                if (past(dl)) break;  // the next claim records the stop
-            }
-            if (pl.tail && l == L - 1) {  // every x_{L-2} of C_{L-2} at once
-                cnt += tail_sum(l);
-                if (l == 3) break;
-                --l;
-                pos = (uint32_t)xget(l - 1) + 1u;
-                continue;
-            }
-            if (pl.pair && l == L - 2) {  // levels L-3..L-1 at once
-                cnt += pair_sum(l);
-                if (l == 3) break;
-                --l;
-                pos = (uint32_t)xget(l - 1) + 1u;
-                continue;
-            }
-            uint64_t vv = own ? sStk[(l - 3) * kBlock + tid] : 0ull;
-            const uint32_t pw = pos >> 6;
-            if (w < pw) vv = 0ull;
-            else if (w == pw) vv &= (~0ull << (pos & 63u));
-            const uint64_t bal = __ballot(vv != 0ull);
-            const uint64_t mine = (P == 64) ? bal : ((bal >> pbase) & ((1ull << P) - 1ull));
-            if (mine == 0ull) {
-                if (l == 3) break;
-                --l;
-                pos = (uint32_t)xget(l - 1) + 1u;
-                continue;
-            }
-            const int f = __builtin_ctzll(mine);
-            const uint64_t vf = __shfl(vv, f, P);
-            const uint32_t xi = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
-            sX[(l - 1) * kBlock + tid] = (uint16_t)xi;
-            const uint64_t t = own ? level_word(l) : 0ull;
-            if (l == L - 1) {
-                cnt += (uint64_t)__popcll(t);
-                if (pl.emit && t) emit_word(out, pl, l, rr.u, A, t, w, xget, hs, hx);
-                pos = xi + 1u;
-            } else {
-                sStk[(l - 2) * kBlock + tid] = t;
-                ++l;
-                pos = 0;
-            }
-        }
+    if (L < 3) return;
+    const uint32_t items = lds_items(pl, v, sumd, cnt);
+    if (WALK == kWalkNone || items == 0) {
+        __syncthreads();  // the next batch reuses the LDS arrays
+        return;
     }
+    constexpr int WT = PC <= 8 ? PC : 1, kLg = WT == 8 ? 3 : WT >> 1;
+    const int walk = WALK != kWalkAny ? WALK
+                     : PC <= 8 && lds_lane_walk(pl, kLg) ? (pl.emit ? kWalkLaneEmit : kWalkLane) : kWalkGroup;
+    if (PC <= 8 && walk == kWalkLane) clique_walk<WT, false>(pl, v, sumd, items, out, dl, cnt, hs, hx);
+    else if (PC <= 8 && walk == kWalkLaneEmit) clique_walk<WT, true>(pl, v, sumd, items, out, dl, cnt, hs, hx);
+    else group_walk<PC>(pl, v, sumd, items, out, dl, cnt, hs, hx);
     __syncthreads();
 }
 
 // MinWaves > 1: the compiler keeps the registers to that many waves per SIMD
 // (7 workgroups per CU instead of 5 for the narrow classes, at the cost of a
 // few bytes of spill); used when no hub kernels of the query share the CUs.
-template <int P, int MinWaves>
+template <int P, int MinWaves, int WALK>
 __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, KPlan pl,
                                                            const RootRec *__restrict__ recs,
                                                            const uint32_t *__restrict__ batch_first,
@@ -770,10 +1031,7 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
     extern __shared__ __align__(16) unsigned char smem[];
     const LdsView v = lds_view(smem, lay);
     const int tid = threadIdx.x;
-    if (tid < kMaxLevels) {
-        v.sMisc[M_QM + tid] = pl.qmask[tid];
-        v.sMisc[M_SM + tid] = pl.smask[tid];
-    }
+    if (tid < 2 * kMaxLevels) v.sMisc[M_LEV + tid] = pl.lev[tid];
     uint64_t cnt = 0, hs = 0, hx = 0;
     const uint64_t dl = out.dl[1];
     const uint64_t t_start = wall_clock64();
@@ -793,7 +1051,7 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
         __syncthreads();
         const uint32_t b = v.sMisc[M_BATCH];
         if (b >= b1) break;
-        process_batch<P>(g, pl, v, recs, batch_first[b], batch_count[b], out, dl, P, cnt, hs, hx);
+        process_batch<P, WALK>(g, pl, v, recs, batch_first[b], batch_count[b], out, dl, cnt, hs, hx);
     }
     flush_acc(out, cnt, hs, hx);
     if (tid == 0) prof_add(out, 0, blockIdx.x, t_start);
@@ -801,8 +1059,9 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
 
 // One persistent launch over the LDS batches of several prepared queries.
 // Work records are ordered heaviest first; a workgroup takes the next record,
-// loads that query's plan and graph and runs the batch with the record's
-// group width, then flushes its counts to that query's counters.
+// loads that query's plan and graph and runs the batch, then flushes its counts
+// to that query's counters.  One launch per lane class (P lanes an item).
+template <int P>
 __global__ __launch_bounds__(kBlock) void lds_multi_kernel(const MultiQuery *__restrict__ qs,
                                                            const MultiWork *__restrict__ work,
                                                            uint32_t nwork, unsigned long long *cursor,
@@ -819,21 +1078,18 @@ __global__ __launch_bounds__(kBlock) void lds_multi_kernel(const MultiQuery *__r
                                    ? (uint32_t)bb : nwork;
         }
         __syncthreads();
-        const uint32_t wi = v.sMisc[M_BATCH];
+        const uint32_t wi = (uint32_t)__builtin_amdgcn_readfirstlane((int)v.sMisc[M_BATCH]);
         if (wi >= nwork) break;
         const MultiWork w = work[wi];
         const MultiQuery &q = qs[w.query];
-        const KPlan pl = q.pl;
-        if (tid < kMaxLevels) {
-            v.sMisc[M_QM + tid] = pl.qmask[tid];
-            v.sMisc[M_SM + tid] = pl.smask[tid];
-        }
+        const KPlan &pl = q.pl;
+        if (tid < 2 * kMaxLevels) v.sMisc[M_LEV + tid] = pl.lev[tid];
         __syncthreads();
         uint64_t cnt = 0, hs = 0, hx = 0;
         const uint64_t dl = q.out.dl[1];
         const uint64_t t_start = wall_clock64();
-        process_batch<0>(q.g, pl, v, q.recs, q.batch_first[w.batch], q.batch_count[w.batch], q.out, dl,
-                         1 << w.lanes_log2, cnt, hs, hx);
+        process_batch<P, kWalkAny>(q.g, pl, v, q.recs, q.batch_first[w.batch], q.batch_count[w.batch], q.out, dl, cnt, hs,
+                         hx);
         flush_acc(q.out, cnt, hs, hx);
         if (tid == 0) prof_add(q.out, 0, blockIdx.x, t_start);
     }
@@ -1522,6 +1778,20 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
         const HubRec h = hubs[hidx];
         const uint32_t jl = h.jbeg + (uint32_t)(item - h.ioff);
         if (L < 3) continue;
+        if (pl.closed) {  // the count follows from |C_2|: one pass over x_1's row, nothing staged
+            const uint32_t hw = (h.d + 63) >> 6;
+            const uint64_t *row = E + h.eoff + (uint64_t)(jl - h.rlo) * hw;
+            const bool rd = (sQM[2] & 2u) != 0, gt = (sSM[2] & 2u) != 0;
+            uint32_t c = 0;
+            for (uint32_t w = (gt ? jl >> 6 : 0u) + lane; w < hw; w += 64) {
+                uint64_t t = (rd ? row[w] : valid_mask(w, h.d)) & ~bit_at(jl, w);
+                if (gt) t &= gt_mask(jl, w);
+                c += (uint32_t)__popcll(t);
+            }
+            c = (uint32_t)wave_sum_u64(c);
+            if (lane == 0 && c) cnt += closed_count(pl.closed, c, h.d);
+            continue;
+        }
         bind(h, jl);
         const uint32_t lo2 = word_lo(2);
         if (L == 3) {
@@ -1636,17 +1906,6 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
 
 // ------------------------------------------------------------ launchers
 
-template <int P, int MinWaves>
-static hipError_t launch_lds_p(int grid, size_t lds, hipStream_t st, const KGraph &g, const KPlan &pl,
-                               const RootRec *recs, const uint32_t *bf, const uint32_t *bc,
-                               uint32_t b0, uint32_t b1, unsigned long long *cursor, const LdsLayout &lay,
-                               const KOut &out)
-{
-    hipLaunchKernelGGL((lds_batch_kernel<P, MinWaves>), dim3(grid), dim3(kBlock), lds, st, g, pl, recs, bf, bc,
-                       b0, b1, cursor, lay, out);
-    return hipGetLastError();
-}
-
 // Workgroups of a kernel per CU with `lds` bytes of dynamic LDS, and its
 // dynamic-LDS attribute raised to at least `lds`.  Both are host calls of
 // several microseconds on the launch path of every query, so they are made
@@ -1676,41 +1935,56 @@ struct LdsLaunchCache {
     }
 };
 
-template <int P, int MinWaves>
-static int occupancy_lds_p(size_t lds)
+constexpr int kBesideHubs = 3;
+
+template <int P, int MinWaves, int WALK>
+static hipError_t launch_lds_p(int cus, size_t lds, hipStream_t st, const KGraph &g, const KPlan &pl,
+                               const RootRec *recs, const uint32_t *bf, const uint32_t *bc,
+                               uint32_t b0, uint32_t b1, unsigned long long *cursor, const LdsLayout &lay,
+                               const KOut &out)
 {
     static LdsLaunchCache cache;
-    return cache.get((const void *)lds_batch_kernel<P, MinWaves>, lds);
-}
-
-// Dispatch on the DFS group width.
-hipError_t launch_lds_batches(int lg, int cus, hipStream_t st, const KGraph &g, const KPlan &pl,
-                              const RootRec *recs, const uint32_t *bf, const uint32_t *bc,
-                              uint32_t b0, uint32_t b1, unsigned long long *cursor, const KOut &out,
-                              int *grid_out, bool dense)
-{
-    const uint32_t nlev = pl.L > 3 ? (uint32_t)(pl.L - 3) : 1u;
-    LdsLayout lay = make_lds_layout(lg, nlev);
-    size_t lds = lay.bytes;
-    int occ = 1;
-    switch (lg) {
-#define BEEP_CASE(LG)                                                                              \
-    case LG:                                                                                       \
-        occ = dense ? occupancy_lds_p<(1 << LG), 7>(lds) : occupancy_lds_p<(1 << LG), 1>(lds);    \
-        break;
-        BEEP_CASE(0) BEEP_CASE(1) BEEP_CASE(2) BEEP_CASE(3) BEEP_CASE(4) BEEP_CASE(5) BEEP_CASE(6)
-#undef BEEP_CASE
-    default: return hipErrorInvalidValue;
-    }
+    int occ = cache.get((const void *)lds_batch_kernel<P, MinWaves, WALK>, lds);
+    // Beside hub kernels a class leaves them wave slots: with seven workgroups
+    // per CU the hub chain's second kernel started 245 us late (diamond, 1.1M
+    // vertices); the query takes 749 us with 3 per CU, 784 with 4, 809 with 5,
+    // 826 with 6.
+    if (MinWaves == 1 && occ > kBesideHubs) occ = kBesideHubs;
     int grid = occ * cus;
     if ((uint32_t)grid > b1 - b0) grid = (int)(b1 - b0);
     if (grid < 1) grid = 1;
-    if (grid_out) *grid_out = grid;
+    hipLaunchKernelGGL((lds_batch_kernel<P, MinWaves, WALK>), dim3(grid), dim3(kBlock), lds, st, g, pl, recs, bf,
+                       bc, b0, b1, cursor, lay, out);
+    return hipGetLastError();
+}
+
+// Dispatch on the DFS group width and the plan's walk.
+template <int LG>
+static hipError_t launch_lds_lg(int cus, hipStream_t st, const KGraph &g, const KPlan &pl, const RootRec *recs,
+                                const uint32_t *bf, const uint32_t *bc, uint32_t b0, uint32_t b1,
+                                unsigned long long *cursor, const KOut &out, bool dense)
+{
+    constexpr int P = 1 << LG;
+    const LdsLayout lay = make_lds_layout(LG, lds_stack_words(pl, LG), pl.L);
+#define BEEP_RUN(MW, WALK) launch_lds_p<P, MW, WALK>(cus, lay.bytes, st, g, pl, recs, bf, bc, b0, b1, cursor, lay, out)
+    if (pl.closed) return dense ? BEEP_RUN(7, kWalkNone) : BEEP_RUN(1, kWalkNone);
+    if constexpr (LG <= 3) {
+        if (lds_lane_walk(pl, LG)) {
+            if (pl.emit) return dense ? BEEP_RUN(LG == 3 ? 4 : 6, kWalkLaneEmit) : BEEP_RUN(1, kWalkLaneEmit);
+            return dense ? BEEP_RUN(7, kWalkLane) : BEEP_RUN(1, kWalkLane);
+        }
+    }
+    return dense ? BEEP_RUN(7, kWalkGroup) : BEEP_RUN(1, kWalkGroup);
+#undef BEEP_RUN
+}
+
+hipError_t launch_lds_batches(int lg, int cus, hipStream_t st, const KGraph &g, const KPlan &pl,
+                              const RootRec *recs, const uint32_t *bf, const uint32_t *bc,
+                              uint32_t b0, uint32_t b1, unsigned long long *cursor, const KOut &out, bool dense)
+{
     switch (lg) {
-#define BEEP_CASE(LG)                                                                                    \
-    case LG:                                                                                             \
-        return dense ? launch_lds_p<(1 << LG), 7>(grid, lds, st, g, pl, recs, bf, bc, b0, b1, cursor, lay, out) \
-                     : launch_lds_p<(1 << LG), 1>(grid, lds, st, g, pl, recs, bf, bc, b0, b1, cursor, lay, out);
+#define BEEP_CASE(LG) \
+    case LG: return launch_lds_lg<LG>(cus, st, g, pl, recs, bf, bc, b0, b1, cursor, out, dense);
         BEEP_CASE(0) BEEP_CASE(1) BEEP_CASE(2) BEEP_CASE(3) BEEP_CASE(4) BEEP_CASE(5) BEEP_CASE(6)
 #undef BEEP_CASE
     }
@@ -1763,19 +2037,29 @@ hipError_t launch_begin_sequence(unsigned long long *ctr, uint64_t n, uint64_t d
 }
 
 // One lane class's batches (lg: the widest of them) of several queries.
-hipError_t launch_lds_multi(int cus, hipStream_t st, const MultiQuery *qs, const MultiWork *work,
-                            uint32_t nwork, unsigned long long *cursor, uint32_t nlev, int lg, int *grid_out)
+template <int P>
+static hipError_t launch_lds_multi_p(int cus, hipStream_t st, const MultiQuery *qs, const MultiWork *work,
+                                     uint32_t nwork, unsigned long long *cursor, const LdsLayout &lay)
 {
-    LdsLayout lay = make_lds_layout(lg, nlev);
-    size_t lds = lay.bytes;
     static LdsLaunchCache cache;
-    const int occ = cache.get((const void *)lds_multi_kernel, lds);
-    int grid = occ * cus;
+    int grid = cache.get((const void *)lds_multi_kernel<P>, lay.bytes) * cus;
     if ((uint32_t)grid > nwork) grid = (int)nwork;
     if (grid < 1) grid = 1;
-    if (grid_out) *grid_out = grid;
-    hipLaunchKernelGGL(lds_multi_kernel, dim3(grid), dim3(kBlock), lds, st, qs, work, nwork, cursor, lay);
+    hipLaunchKernelGGL((lds_multi_kernel<P>), dim3(grid), dim3(kBlock), lay.bytes, st, qs, work, nwork, cursor, lay);
     return hipGetLastError();
+}
+
+hipError_t launch_lds_multi(int cus, hipStream_t st, const MultiQuery *qs, const MultiWork *work,
+                            uint32_t nwork, unsigned long long *cursor, uint32_t stack_words, int levels, int lg)
+{
+    const LdsLayout lay = make_lds_layout(lg, stack_words, levels);
+    switch (lg) {
+#define BEEP_CASE(LG) \
+    case LG: return launch_lds_multi_p<(1 << LG)>(cus, st, qs, work, nwork, cursor, lay);
+        BEEP_CASE(0) BEEP_CASE(1) BEEP_CASE(2) BEEP_CASE(3) BEEP_CASE(4) BEEP_CASE(5) BEEP_CASE(6)
+#undef BEEP_CASE
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_hub_hash(int grid, hipStream_t st, const KGraph &g, const HubRec *hubs,

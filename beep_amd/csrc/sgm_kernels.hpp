@@ -16,6 +16,8 @@ constexpr int kMaxLevels = 10;  // query positions (DEPTH)
 // one per 128-byte line of kLine u64 words.
 constexpr int kLine = 16, kStripes = 16;
 
+constexpr uint32_t kNoSplit = 1u << 20;  // KPlan::chunk: an item is a whole x_1
+
 // Query plan as the kernels consume it (by value).  Level l in [2, L) is
 // the candidate set C_l:
 //   C_l = {i in [0,d) \ {x_1..x_{l-1}} : E[x_q][i] = 1 for q in qmask[l],
@@ -53,7 +55,48 @@ struct KPlan {
     int32_t upper;
     uint32_t qmask[kMaxLevels];
     uint32_t smask[kMaxLevels];
+    // What is left to do for level l when the walk starts from an earlier
+    // level's set: C_l = C_base with the rows rq, the bounds rs and the
+    // exclusions rx applied (base 0: from all of [0, d)).  lev[l] holds
+    // rq | rs << 16, lev[kMaxLevels + l] holds rx | base << 16.
+    uint32_t lev[2 * kMaxLevels];
+    // Every level is C_l = C_{l-1} n E[x_{l-1}] over bitmaps without mirrored
+    // bits (cliques): one row per step, no bounds, no exclusions.
+    int32_t nested;
+    // x_2 candidates of one DFS item of the LDS batches (see lds_items).
+    uint32_t chunk;
+    int32_t reads_rows;  // some level intersects with a bitmap row
+    int32_t tail_gt;     // tail: L-2 is in smask[L-1]
+    // Count-only plans whose count below x_1 is a function of |C_2| = c and
+    // the root's row length d alone (diamond: c (c - 1) / 2); see closed_count.
+    int32_t closed;
 };
+
+// KPlan::closed: triangle-like plans (L = 3), or a summed level 3 whose set is
+// C_2 again (with or without x_3 > x_2), or all of the row but x_1 (and x_2).
+enum { kOpen = 0, kClosedC = 1, kClosedPairs = 2, kClosedOrdered = 3, kClosedRow = 4 };
+__host__ __device__ __forceinline__ uint64_t closed_count(int closed, uint64_t c, uint32_t d)
+{
+    return closed == kClosedC ? c
+           : closed == kClosedPairs ? c * (c - 1u) / 2u
+           : closed == kClosedOrdered ? c * (c - 1u)
+                                      : c * (d - 2u);
+}
+
+// Whether the LDS batches of lane class lg walk this plan one item per lane
+// (clique_walk), and the u64 words of LDS stack a thread then needs: the sets
+// of levels 3..L-2 of 1 << lg words each, against one word per level for the
+// lane groups (group_walk).  16 words (32 KB a workgroup) leave the widest
+// class one workgroup per CU fewer; plans deeper than that keep the groups.
+__host__ __device__ inline bool lds_lane_walk(const KPlan &pl, int lg)
+{
+    return pl.nested && lg <= 3 && ((pl.L - 4) << lg) <= 16;
+}
+__host__ __device__ inline uint32_t lds_stack_words(const KPlan &pl, int lg)
+{
+    const int group = pl.L > 3 ? pl.L - 3 : 1, lane = lds_lane_walk(pl, lg) ? (pl.L - 4) << lg : 0;
+    return (uint32_t)(group > lane ? group : lane);
+}
 
 // Per-vertex record read when the vertex appears in a root's row: where its
 // bitmap-build scan range starts in ocol and how long it is (one 16-byte

@@ -464,3 +464,28 @@ def test_golden_quirk_cases():
             if got != c["count"]:
                 bad.append((c["graph"], c["pattern"], c["mode"], emit, got, c["count"]))
     assert not bad, bad[:10]
+
+
+def _roots_over_core(core, seed):
+    """core + 8 roots, each adjacent to all `core` vertices of a random graph:
+    the roots' rows above their own key have exactly `core` entries."""
+    rng = np.random.default_rng(seed)
+    a = np.triu(rng.random((core, core)) < max(0.08, min(0.5, 16.0 / core)), 1)
+    u, v = np.nonzero(a)
+    edges = list(zip(u.tolist(), v.tolist())) + [(c, core + r) for r in range(core + 8) for c in range(core)]
+    pairs = sorted(set(edges) | {(y, x) for x, y in edges})
+    return B.Graph.from_edges([x for x, _ in pairs], [y for _, y in pairs])
+
+
+@pytest.mark.parametrize("core", [5, 63, 64, 65, 128, 129, 257, 512])
+@pytest.mark.parametrize("k", [4, 5, 6, 7])
+def test_clique_walk_row_widths(core, k):
+    """Cliques on rows at the edges of every lane class, counted and emitted."""
+    g = _roots_over_core(core, 5)
+    og = oracle_graph(g)
+    for emit in (B.EMIT_NONE, B.EMIT_HASH):
+        say("clique walk", core, k, emit)
+        r, o, _ = run_pair(g, og, _clique(k), B.SGC, emit=emit)
+        assert r["count"] == o["count"]
+        if emit:
+            assert (r["hash_sum"], r["hash_xor"]) == (o["hash_sum"], o["hash_xor"])
