@@ -207,10 +207,10 @@ struct LdsBudget {
     static constexpr uint32_t kMaxRoots = 128;     // roots per batch
     static constexpr uint32_t kMaxSumDeg = 512;    // largest sum of degrees per batch
     static constexpr uint32_t kMaxEWords = 4096;   // bitmap words (u64)
-    static constexpr uint32_t kMaxHash = 2048;     // largest hash slots per batch
     static constexpr int kMaxClass = 6;
     static constexpr uint32_t sumdeg(int lg) { return lg >= 3 ? kMaxSumDeg : kMaxSumDeg / 2; }
-    static constexpr uint32_t hash(int lg) { return 4 * sumdeg(lg); }
+    // slots of a row: a power of two >= 2d, so three per entry hold a full batch
+    static constexpr uint32_t hash(int lg) { return 3 * sumdeg(lg); }
     static constexpr uint32_t ewords(int lg)
     {
         return (sumdeg(lg) << (lg < 3 ? lg : 3)) < kMaxEWords ? (sumdeg(lg) << (lg < 3 ? lg : 3)) : kMaxEWords;
@@ -226,9 +226,23 @@ struct LdsBudget {
 };
 
 uint32_t hash_slots_for(uint32_t d);
-// Automatic LDS bitmap build: a row vertex whose larger-key range is longer
-// than kLookupRatio x the root's degree looks the root's neighbours up in the
-// range's lookup table instead of streaming the range.
+// Slots of a root's row in an LDS batch: the smallest power of two >= max(4, 2d).
+constexpr uint32_t lds_hash_log2(uint32_t d) { return d < 3 ? 2u : 32u - (uint32_t)__builtin_clz(2 * d - 1); }
+constexpr uint32_t lds_hash_slots(uint32_t d) { return 1u << lds_hash_log2(d); }
+// LDS bitmap build, row j of a root (vertex v): the number of row entries that
+// can pair with j and that the plan reads -- those on v's larger-key side (after
+// j in ascending rows, before it in descending ones), and with `kept` (only
+// rows from the split on are read) those of which one is kept.  0: the row has
+// nothing to find.
+constexpr uint32_t pair_partners(uint32_t j, uint32_t d, uint32_t split, int asc, int kept, int upper)
+{
+    if (!asc) return j;
+    if (kept && j < split) return upper || split >= d ? 0u : d - split;
+    return d - 1u - j;
+}
+// Automatic build: a larger-key range longer than kLookupRatio x the row's
+// partners is not streamed; the partners are looked up in the range's lookup
+// table instead.
 constexpr uint32_t kLookupRatio = 4;
 void build_tiers(Prep &pp);
 void class_figures(Prep &pp);

@@ -15,8 +15,7 @@
 
 namespace beep {
 
-// Hash slots of a root's row (LDS batches and hub arena): the smallest power
-// of two >= max(4, 4d), as the kernels' hash_slots_dev.
+// Hash slots of a hub's kept rows: the smallest power of two >= max(4, 4d).
 uint32_t hash_slots_for(uint32_t d)
 {
     uint32_t h = 4;
@@ -265,7 +264,7 @@ void build_work(Prep &pp_, const Plan &p, uint32_t sample_stride)
     pp->alg_bytes = bytes.load();
     // Work list.  With above_split plans a root keeps only its suffix of
     // larger keys (asc rows), which drops the skipped x_1 < split items and
-    // every bitmap entry they alone would use; roots left empty carry no work.
+    // every bitmap entry they alone would use; roots left too short carry no work.
     pp->reduced = p.above_split;
     pp->skip_split = p.skip_split;
     pp->rows_above_split = p.rows_above_split;
@@ -278,8 +277,10 @@ void build_work(Prep &pp_, const Plan &p, uint32_t sample_stride)
         };
         std::vector<uint32_t> idx;
         idx.reserve(pp->roots.size());
+        // a tuple takes L - 1 distinct row entries: shorter rows carry no work
+        const uint32_t least = (uint32_t)std::max(p.L - 1, 1);
         for (uint32_t r = 0; r < (uint32_t)pp->roots.size(); r++)
-            if (len_of(r)) idx.push_back(r);
+            if (len_of(r) >= least) idx.push_back(r);
         // roots are in degree-descending order already; only reduced lengths
         // need a (stable) sort
         if (pp->reduced)
@@ -289,7 +290,7 @@ void build_work(Prep &pp_, const Plan &p, uint32_t sample_stride)
             // length-sorted list) are kept every hub_sample_stride(), the rest
             // every sample_stride; the middle entry of every stride, so the
             // heaviest root alone does not stand for the ones after it.
-            auto fits_lds = [](uint32_t d) { return LdsBudget::fits(d, hash_slots_for(d)); };
+            auto fits_lds = [](uint32_t d) { return LdsBudget::fits(d, lds_hash_slots(d)); };
             size_t nh = 0;
             while (nh < idx.size() && !fits_lds(len_of(idx[nh]))) nh++;
             const uint32_t hs = hub_sample_stride(sample_stride);
@@ -320,7 +321,7 @@ void build_work(Prep &pp_, const Plan &p, uint32_t sample_stride)
 void build_tiers(Prep &pp)
 {
     auto deg = [&](uint32_t i) { return pp.wlen[i]; };
-    auto fits_lds = [&](uint32_t d) { return LdsBudget::fits(d, hash_slots_for(d)); };
+    auto fits_lds = [&](uint32_t d) { return LdsBudget::fits(d, lds_hash_slots(d)); };
     uint32_t nh = 0;
     while (nh < pp.wlen.size() && !fits_lds(deg(nh))) nh++;
     pp.n_hub = nh;
@@ -348,11 +349,11 @@ void build_tiers(Prep &pp)
             uint32_t d = deg(i);
             uint64_t w = (d + 63) / 64;
             if (b.count && (sd + d > cap || sw + d * w > LdsBudget::ewords((int)lg) ||
-                            sh + hash_slots_for(d) > LdsBudget::hash((int)lg) || lg_of(d) != lg))
+                            sh + lds_hash_slots(d) > LdsBudget::hash((int)lg) || lg_of(d) != lg))
                 break;
             sd += d;
             sw += d * w;
-            sh += hash_slots_for(d);
+            sh += lds_hash_slots(d);
             b.count++;
             i++;
         }
@@ -363,9 +364,8 @@ void build_tiers(Prep &pp)
 }
 
 // Work and compulsory bytes of each lane class's launch, with the automatic
-// build mode (a row vertex whose scan range is over kLookupRatio x the root's
-// degree looks the root's neighbours on its larger-key side up in the range's
-// lookup table, one 4-byte slot each).
+// build mode (pair_partners, kLookupRatio): a streamed range's entries, or one
+// 4-byte table slot per looked-up partner.
 void class_figures(Prep &pp)
 {
     const Variant &V = *pp.var;
@@ -383,17 +383,11 @@ void class_figures(Prep &pp)
             for (uint32_t j = 0; j < d; j++) {
                 const uint32_t v = V.ocol[rb + j];
                 const uint64_t hl = V.hlen[v];
-                bytes += 16;  // the row vertex's record
-                if (hl > (uint64_t)kLookupRatio * d) {
-                    // the root's neighbours on the larger-key side of v, one
-                    // table slot each
-                    const uint64_t c = V.asc ? d - 1 - j : j;
-                    units += c;
-                    bytes += 4ull * c;
-                } else {
-                    units += hl;
-                    bytes += 4ull * hl;
-                }
+                const uint64_t c = pair_partners(j, d, pp.reduced ? 0u : V.nlow[u], V.asc, pp.rows_above_split,
+                                                 pp.upper_rows);
+                const uint64_t n = c == 0 ? 0 : hl > kLookupRatio * c ? c : hl;
+                bytes += 16 + 4 * n;  // the row vertex's record
+                units += n;
             }
         }
         bu[bi] = units;

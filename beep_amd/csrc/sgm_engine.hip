@@ -266,7 +266,7 @@ void upload(Prep &pp, int device, int p_skip_split, uint64_t arena_budget)
                 r.hoff = hoff;
                 doff += r.d;
                 eoff += r.d * ((r.d + 63) / 64);
-                hoff += hash_slots_for(r.d);
+                hoff += lds_hash_slots(r.d);
                 recs.push_back(r);
             }
         }
@@ -516,6 +516,10 @@ static KPlan make_kplan(const Plan &p, int emit, int build_mode)
         if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 2u << 16) k.closed = k.tail_gt ? kClosedPairs : kClosedOrdered;
         if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 1u << 1 && !k.tail_gt) k.closed = kClosedRow;
     }
+    k.kept = p.rows_above_split;
+    // every pair found is one candidate x_2 of its smaller index, and the count
+    // is a sum over those: the build counts pairs and sets no bitmap
+    k.hits = p.upper_rows && (k.closed == kClosedC || k.closed == kClosedRow) && p.qmask[2] == 2u;
     // levels an item walks below x_2: none (one pass over the row's words, or
     // the count itself), one, two, or more
     const int walked = p.L - (k.tail ? 1 : 0) - (k.pair ? 2 : 0) - 3;
@@ -908,7 +912,7 @@ struct Batch {
 };
 
 hipError_t launch_lds_multi(int cus, hipStream_t st, const MultiQuery *qs, const MultiWork *work, uint32_t nwork,
-                            unsigned long long *cursor, uint32_t stack_words, int levels, int lg);
+                            unsigned long long *cursor, const LdsNeeds &need, int lg);
 
 Batch *batch_create(Prep *const *preps, const Plan *const *plans, const beep_opts *opts, int n)
 {
@@ -1009,15 +1013,11 @@ static void batch_capture(Batch &b)
     }
     for (int k = 0; k < ncls; k++) {
         hipStream_t sk = b.branch[n + k];
-        uint32_t words = 1;
-        int levels = 3;
-        for (const LaunchCfg &c : b.cfgs) {
-            words = std::max(words, lds_stack_words(c.kp, b.cls_lg[k]));
-            levels = std::max(levels, (int)c.kp.L);
-        }
+        LdsNeeds need;
+        for (const LaunchCfg &c : b.cfgs) need.add(c.kp, b.cls_lg[k]);
         HIP_CHECK(hipStreamWaitEvent(sk, b.fork, 0));
         HIP_CHECK(launch_lds_multi(d0.cus, sk, b.dqs, b.dwork + b.cls_w0[k], b.cls_w1[k] - b.cls_w0[k],
-                                   b.cursor + (uint64_t)k * kCurWords, words, levels, b.cls_lg[k]));
+                                   b.cursor + (uint64_t)k * kCurWords, need, b.cls_lg[k]));
         HIP_CHECK(hipEventRecord(b.done[n + k], sk));
     }
     for (int i = 0; i < n + ncls; i++) HIP_CHECK(hipStreamWaitEvent(b.s0, b.done[i], 0));

@@ -111,14 +111,6 @@ __device__ __forceinline__ void set_pair(uint64_t *E, uint32_t W, uint32_t j, ui
     if (!upper || j > i) atomicOr((unsigned long long *)&E[i * W + (j >> 6)], 1ull << (j & 63));
 }
 
-// smallest power of two >= max(4, 4d): at most a quarter of the slots are
-// taken, so a probe for an absent key rarely goes past its first slot
-__host__ __device__ __forceinline__ uint32_t hash_slots_dev(uint32_t d)
-{
-    if (d <= 1) return 4;
-    return 1u << (32 - __builtin_clz(4 * d - 1));
-}
-
 __device__ __forceinline__ uint64_t mix64(uint64_t z)
 {
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
@@ -152,6 +144,25 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
         if (lane >= o) v += y;
     }
     return v;
+}
+
+// Set bits of m below the lane.
+__device__ __forceinline__ uint32_t bits_below(uint64_t m)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+__device__ __forceinline__ uint32_t lane_u32(uint32_t v, uint32_t l)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
+}
+
+// Orders a wave's own LDS writes before its following reads by other lanes.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Deadline check: wall_clock64() is a constant-rate device clock.
@@ -285,45 +296,68 @@ __device__ __forceinline__ void emit_word(const KOut &out, const KPlan &pl, int 
     emit_bits(out, l, u, A, h, t, w, xget, hs, hx);
 }
 
-__device__ __forceinline__ bool use_search(uint32_t hlen, uint32_t d, uint32_t ratio)
-{
-    return (uint64_t)hlen > (uint64_t)d * ratio;
-}
-
 // ------------------------------------------------------------ LDS batches
 
+// Context of a row of an LDS batch that has build units (see find_pairs):
+// streamed rows: unit e is ocol[base + e]; looked-up rows: unit e looks the row
+// entry aoff + e up in the range whose hbeg | hlen << kRangeShift is `base`.
+struct RowCtx {
+    uint64_t base;
+    uint32_t aoff;
+    uint32_t info;  // row (9 bits) | looked up << 9 | filter word << 10 (10) | filter bits' log2 << 20
+};
+
+// Units of the tile of build work whose row starts are marked at once, and the
+// entries of a wave's queue of probable pairs.
+constexpr uint32_t kTile = 4096, kQueue = 128;
+
+// What the build needs (hash, filter, row contexts, marks, queues) and what the
+// walk needs (items, stack, x) share the space after `shared`.
 struct LdsLayout {
-    uint32_t oE, oHBeg, oStk, oA, oPre, oHKey, oRoot, oHVal, oX, oJRoot, oMisc, bytes;
-    uint32_t ewords;
+    uint32_t oE, oRoot, oA, oMisc, oJRoot;
+    uint32_t oCtx, oQ, oMark, oHKey, oFlt, oHVal;  // build
+    uint32_t oStk, oPre, oX;                       // walk
+    uint32_t bytes;
 };
 
 __host__ __device__ inline uint32_t align_up(uint32_t x, uint32_t a) { return (x + a - 1) / a * a; }
 
 // Layout of lane class lg's batches; stack_words words of DFS stack and
 // `levels` positions of x are kept per thread.
-__host__ inline LdsLayout make_lds_layout(int lg, uint32_t stack_words, int levels)
+__host__ inline LdsLayout make_lds_layout(int lg, const LdsNeeds &need)
 {
-    const uint32_t sd = LdsBudget::sumdeg(lg), hs = LdsBudget::hash(lg), ew = LdsBudget::ewords(lg);
+    const uint32_t sd = LdsBudget::sumdeg(lg), hs = LdsBudget::hash(lg);
     LdsLayout L{};
     uint32_t o = 0;
-    L.ewords = ew;
-    L.oE = o;       o += ew * 8;
-    L.oHBeg = o;    o += sd * 8;
-    L.oStk = o;     o += stack_words * kBlock * 8;
+    // past the last row's words, clique_walk reads up to 7 more
+    L.oE = o;       o += need.bitmap ? (LdsBudget::ewords(lg) + 8) * 8 : 0;
     L.oRoot = o;    o += LdsBudget::kMaxRoots * (uint32_t)sizeof(RootRec);
     L.oA = o;       o += sd * 4;
-    L.oPre = o;     o += align_up((sd + 1) * 4, 8);
-    L.oHKey = o;    o += hs * 4;
     L.oMisc = o;    o += 32 * 4;
-    L.oHVal = o;    o += hs * 2;
-    L.oX = o;       o += (uint32_t)levels * kBlock * 2;
+    L.oMark = o;    o += kTile / 8;
     L.oJRoot = o;   o += sd;
-    L.bytes = align_up(o, 16);
+    const uint32_t shared = align_up(o, 16);
+    o = shared;
+    if (need.rows) {
+        L.oCtx = o;     o += sd * (uint32_t)sizeof(RowCtx);
+        L.oQ = o;       o += (kBlock / 64) * kQueue * 8;
+        L.oHKey = o;    o += hs * 4;
+        L.oFlt = o;     o += hs / 2 * 4;
+        L.oHVal = o;    o += hs * 2;
+    }
+    const uint32_t build = o;
+    o = shared;
+    if (need.walk) {
+        L.oStk = o;     o += need.stack_words * kBlock * 8;
+        L.oPre = o;     o += align_up((sd + 1) * 4, 8);
+        L.oX = o;       o += (uint32_t)need.levels * kBlock * 2;
+    }
+    L.bytes = align_up(o > build ? o : build, 16);
     return L;
 }
 
 // Misc slots
-enum { M_BATCH = 0, M_NEXT = 1, M_LEV = 4 };  // M_LEV: 2 kMaxLevels words (KPlan::lev); 28..31: scan
+enum { M_BATCH = 0, M_NEXT = 1, M_LEV = 4 };  // M_LEV: 2 kMaxLevels words (KPlan::lev); 24..31: scans
 
 // Block-wide exclusive scan of a[0..n) in place (n <= 4 * kBlock); a[n] = total.
 __device__ void block_excl_scan(uint32_t *a, uint32_t n, uint32_t *tmp4)
@@ -353,9 +387,10 @@ __device__ void block_excl_scan(uint32_t *a, uint32_t n, uint32_t *tmp4)
 
 // LDS carve-up of one workgroup.
 struct LdsView {
-    uint64_t *sE, *sHBeg, *sStk;
+    uint64_t *sE, *sStk, *sMark, *sQ;
     RootRec *sRoot;
-    uint32_t *sA, *sPre, *sHKey, *sMisc;
+    RowCtx *sCtx;
+    uint32_t *sA, *sPre, *sHKey, *sFlt, *sMisc;
     uint16_t *sHVal, *sX;
     uint8_t *sJRoot;
 };
@@ -364,12 +399,15 @@ __device__ __forceinline__ LdsView lds_view(unsigned char *smem, const LdsLayout
 {
     LdsView v;
     v.sE = (uint64_t *)(smem + lay.oE);
-    v.sHBeg = (uint64_t *)(smem + lay.oHBeg);
     v.sStk = (uint64_t *)(smem + lay.oStk);
+    v.sMark = (uint64_t *)(smem + lay.oMark);
+    v.sQ = (uint64_t *)(smem + lay.oQ);
     v.sRoot = (RootRec *)(smem + lay.oRoot);
+    v.sCtx = (RowCtx *)(smem + lay.oCtx);
     v.sA = (uint32_t *)(smem + lay.oA);
     v.sPre = (uint32_t *)(smem + lay.oPre);
     v.sHKey = (uint32_t *)(smem + lay.oHKey);
+    v.sFlt = (uint32_t *)(smem + lay.oFlt);
     v.sMisc = (uint32_t *)(smem + lay.oMisc);
     v.sHVal = (uint16_t *)(smem + lay.oHVal);
     v.sX = (uint16_t *)(smem + lay.oX);
@@ -504,7 +542,7 @@ __device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, ui
             } else if (l == 3 && (left == 0 || !any())) {  // claim
                 // one LDS atomic for the lanes that claim together
                 const uint64_t m = __ballot(1);
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                const uint32_t rank = bits_below(m);
                 uint32_t first = 0;
                 if (rank == 0) first = atomicAdd(&v.sMisc[M_NEXT], (uint32_t)__popcll(m));
                 const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + rank;
@@ -809,10 +847,271 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
     }
 }
 
-// Processes one LDS batch: stage rows, hash and bitmaps, then the DFS over
-// its items (lds_items).  The plan's level records are in sMisc[M_LEV..].
-// WALK fixes the walk at compile time where the launch serves one plan (the
-// walks need different registers); kWalkAny picks it per plan.
+// Hash of a vertex for the LDS tables: the top bits of a 24-bit product (a
+// full-rate multiply; the 32-bit one runs at a quarter of the rate).
+__device__ __forceinline__ uint32_t lds_hash(uint32_t v) { return __umul24(v, 0x9E3779u); }
+
+// Stages a batch -- its roots, row vertices and each row's root -- and builds
+// the roots' bitmaps (or counts their pairs, KPlan::hits).  Returns the number
+// of rows.
+//
+// Each adjacent pair (v, w) of a root's row, key(v) < key(w), is found from v.
+// Row v's work units are the entries of v's larger-key range, each tested
+// against the root's row, or, where that range is longer than kLookupRatio
+// times the entries v can pair with, those entries, each looked up in the
+// range's table.  What bounds it is instruction issue (a wave64 VALU
+// instruction takes a SIMD four cycles), so the units cost as few as possible:
+//  * all rows' units are numbered through and a wave takes 64 consecutive ones,
+//    one a lane.  A unit's row is the number of row starts at or before it,
+//    one 64-bit mark word and one count per 64 units and a mask-and-count per
+//    lane; the row's context is one 16-byte LDS read;
+//  * a streamed entry is first tested against a filter of 16 to 32 bits per row
+//    entry.  The few per cent that pass (and the looked-up slots that are taken)
+//    go to a queue per wave, which is worked off 64 at a time: the exact probe
+//    and the bit setting run with full waves;
+//  * four loads a lane are in flight.
+// Before, each thread took 8 consecutive units and reloaded the row's context
+// wherever one of 64 lanes crossed into another row, and every lane waited for
+// the longest probe: 216 lane instructions per unit (4-clique, 1.1M vertices).
+__device__ uint32_t build_batch(const KGraph &g, const KPlan &pl, const LdsView &v, const RootRec *__restrict__ recs,
+                                uint32_t first, uint32_t nr, uint64_t &cnt)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const bool rows = pl.reads_rows != 0;
+    if (tid < (int)(LdsBudget::kMaxSumDeg / 64)) v.sMark[tid] = 0;
+    if (tid == 0) v.sMisc[M_NEXT] = 0;
+    RootRec mine{};
+    if (tid < (int)nr) {
+        mine = recs[first + tid];
+        v.sRoot[tid] = mine;
+    }
+    __syncthreads();
+    if (tid < (int)nr) atomicOr((unsigned long long *)&v.sMark[mine.doff >> 6], 1ull << (mine.doff & 63u));
+    const RootRec last = v.sRoot[nr - 1];
+    const uint32_t sumd = last.doff + last.d;
+    if (rows) {
+        const uint32_t ew = pl.hits ? 0u : last.eoff + last.d * ((last.d + 63) >> 6);
+        const uint32_t hsl = last.hoff + lds_hash_slots(last.d);
+        for (uint32_t i = tid; i < ew; i += kBlock) v.sE[i] = 0;
+        for (uint32_t i = tid; i < hsl; i += kBlock) v.sHKey[i] = 0;
+        for (uint32_t i = tid; i < hsl / 2; i += kBlock) v.sFlt[i] = 0;
+    }
+    __syncthreads();
+    // A thread holds at most kRowsPer rows; their row entries, then their
+    // vertex records, are loaded together.  A row's root is the number of
+    // roots that start at or before it.
+    constexpr int kRowsPer = (int)(LdsBudget::kMaxSumDeg / kBlock);
+    static_assert(LdsBudget::kMaxSumDeg % kBlock == 0, "rows per thread");
+    uint32_t rvx[kRowsPer], rro[kRowsPer];
+#pragma unroll
+    for (int q = 0; q < kRowsPer; q++) {
+        const uint32_t j = (uint32_t)tid + (uint32_t)q * kBlock;
+        rvx[q] = 0;
+        rro[q] = 0;
+        if ((uint32_t)q * kBlock >= sumd) continue;
+        const int wj = q * (kBlock / 64) + wv;
+        uint32_t before = 0;
+        for (int w = 0; w < wj; w++) before += (uint32_t)__popcll(v.sMark[w]);
+        const uint64_t m = v.sMark[wj];
+        if (j < sumd) {
+            const uint32_t r = before + bits_below(m) + (uint32_t)((m >> lane) & 1u) - 1u;
+            rro[q] = r;
+            rvx[q] = g.ocol[v.sRoot[r].rbeg + (j - v.sRoot[r].doff)];
+            v.sA[j] = rvx[q];
+            v.sJRoot[j] = (uint8_t)r;
+        }
+    }
+    if (!rows) {
+        __syncthreads();
+        return sumd;
+    }
+    VInfo rvi[kRowsPer];
+#pragma unroll
+    for (int q = 0; q < kRowsPer; q++)
+        if ((uint32_t)tid + (uint32_t)q * kBlock < sumd) rvi[q] = g.vinfo[rvx[q]];
+    uint32_t un[kRowsPer], inc[kRowsPer];
+    uint64_t act[kRowsPer];
+    RowCtx cx[kRowsPer];
+#pragma unroll
+    for (int q = 0; q < kRowsPer; q++) {
+        const uint32_t j = (uint32_t)tid + (uint32_t)q * kBlock;
+        un[q] = inc[q] = 0;
+        act[q] = 0;
+        if ((uint32_t)q * kBlock >= sumd) continue;
+        if (j < sumd) {
+            const RootRec rr = v.sRoot[rro[q]];
+            const uint32_t jl = j - rr.doff, vx = rvx[q], lh = lds_hash_log2(rr.d);
+            const uint32_t H = 1u << lh, h = lds_hash(vx);
+            if (!pl.kept || jl >= rr.split) {  // only kept entries are looked for
+                uint32_t s = h >> (32u - lh);
+                while (atomicCAS(&v.sHKey[rr.hoff + s], 0u, vx + 1u) != 0u) s = (s + 1) & (H - 1);
+                v.sHVal[rr.hoff + s] = (uint16_t)jl;
+                const uint32_t fb = h >> (28u - lh);  // 16 H filter bits
+                atomicOr(&v.sFlt[(rr.hoff >> 1) + (fb >> 5)], 1u << (fb & 31u));
+            }
+            // x_1..x_{L-1} are distinct row entries: shorter rows hold no tuple
+            const uint32_t c = rr.d + 1u < (uint32_t)pl.L
+                                   ? 0u : pair_partners(jl, rr.d, rr.split, g.asc, pl.kept, pl.upper);
+            const VInfo vi = rvi[q];
+            if (c) {
+                const bool look = (uint64_t)vi.hlen > (uint64_t)c * pl.bin_ratio;
+                un[q] = look ? c : vi.hlen;
+                cx[q].base = look ? vi.hbeg | ((uint64_t)vi.hlen << kRangeShift) : vi.hbeg;
+                cx[q].aoff = rr.doff + (g.asc ? rr.d - c : 0u);  // first partner
+                cx[q].info = j | (look ? 1u << 9 : 0u) | (rr.hoff >> 1) << 10 | (lh + 4u) << 20;
+            }
+        }
+        inc[q] = wave_incl_scan(un[q]);
+        act[q] = __ballot(un[q] != 0);
+        if (lane == 63) {
+            v.sMark[16 + q * (kBlock / 64) + wv] = (uint64_t)inc[q] | (uint64_t)__popcll(act[q]) << 32;
+        }
+    }
+    __syncthreads();
+    uint32_t total = 0, rows_before = 0;
+#pragma unroll
+    for (int q = 0; q < kRowsPer; q++) {
+        if ((uint32_t)q * kBlock >= sumd) continue;
+        uint32_t ub = total, rb = rows_before;
+        for (int w = 0; w < kBlock / 64; w++) {
+            const uint64_t t = v.sMark[16 + q * (kBlock / 64) + w];
+            if (w < wv) {
+                ub += (uint32_t)t;
+                rb += (uint32_t)(t >> 32);
+            }
+            total += (uint32_t)t;
+            rows_before += (uint32_t)(t >> 32);
+        }
+        if (un[q]) {
+            const uint32_t start = ub + inc[q] - un[q];
+            cx[q].aoff -= start;
+            if (!((cx[q].info >> 9) & 1u)) cx[q].base -= start;
+            v.sCtx[rb + bits_below(act[q])] = cx[q];
+        }
+        inc[q] = ub + inc[q] - un[q];  // the row's first unit
+    }
+
+    // exact probe of 64 queued units (lanes below n), and what a pair does
+    uint64_t *q = v.sQ + wv * kQueue;
+    auto settle = [&](uint32_t from, uint32_t n) {
+        wave_lds_sync();
+        if ((uint32_t)lane < n) {
+            const uint64_t ent = q[from + lane];
+            const uint32_t lo = (uint32_t)ent, info = (uint32_t)(ent >> 32);
+            const uint32_t j = info & 511u;
+            const RootRec rr = v.sRoot[v.sJRoot[j]];
+            const uint32_t jl = j - rr.doff;
+            uint32_t i = 0;
+            bool hit = false;
+            if ((info >> 9) & 1u) {  // looked up: lo = the partner's row, top bit = found in its first slot
+                const uint32_t p = lo & 0x7fffffffu;
+                i = p - rr.doff;
+                hit = (lo >> 31) != 0;
+                if (!hit) {
+                    const VInfo vi = g.vinfo[v.sA[j]];
+                    const uint32_t a = v.sA[p] + 1u, size = 2 * vi.hlen;
+                    const uint32_t *t = g.htab + 2 * vi.hbeg;
+                    uint32_t s = lookup_slot(a - 1u, size);
+                    for (;;) {
+                        s = s + 1 == size ? 0 : s + 1;
+                        const uint32_t x = t[s];
+                        hit = x == a;
+                        if (hit || x == 0u) break;
+                    }
+                }
+            } else {
+                const uint32_t lh = ((info >> 20) & 31u) - 4u, mask = (1u << lh) - 1u;
+                uint32_t s = lds_hash(lo) >> (32u - lh);
+                for (;;) {
+                    const uint32_t key = v.sHKey[rr.hoff + s];
+                    hit = key == lo + 1u;
+                    if (hit || key == 0u) break;
+                    s = (s + 1) & mask;
+                }
+                if (hit) i = v.sHVal[rr.hoff + s];
+            }
+            if (hit) {
+                if (pl.hits) cnt += pl.closed == kClosedRow ? rr.d - 2u : 1u;
+                else set_pair(v.sE + rr.eoff, (rr.d + 63) >> 6, jl, i, pl.upper);
+            }
+        }
+        wave_lds_sync();
+    };
+
+    constexpr int kUnroll = 4;
+    uint32_t k_done = 0, qn = 0;  // rows started before the tile; queued units
+    for (uint32_t t0 = 0; t0 < total; t0 += kTile) {
+        __syncthreads();
+        if (tid < (int)(kTile / 64)) v.sMark[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kRowsPer; r++) {
+            const uint32_t at = inc[r] - t0;
+            if (un[r] && at < kTile) atomicOr((unsigned long long *)&v.sMark[at >> 6], 1ull << (at & 63u));
+        }
+        __syncthreads();
+        const uint64_t mw = v.sMark[lane];
+        const uint32_t pc = (uint32_t)__popcll(mw), ic = wave_incl_scan(pc);
+        const uint32_t k0 = k_done + ic - pc;
+        k_done += lane_u32(ic, 63);
+        const uint32_t nseg = total - t0 < kTile ? (total - t0 + 63u) >> 6 : kTile / 64;
+        for (uint32_t s0 = wv; s0 < nseg; s0 += kUnroll * (kBlock / 64)) {
+            uint32_t val[kUnroll], aux[kUnroll], info[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; u++) {
+                const uint32_t s = s0 + u * (kBlock / 64);
+                val[u] = aux[u] = info[u] = 0;
+                if (s >= nseg) continue;
+                const uint32_t m0 = lane_u32((uint32_t)mw, s), m1 = lane_u32((uint32_t)(mw >> 32), s);
+                const uint64_t m = (uint64_t)m1 << 32 | m0;
+                const uint32_t k = lane_u32(k0, s) + (m0 & 1u) - 1u + bits_below(m >> 1);
+                const uint32_t e = t0 + s * 64 + lane;
+                if (e >= total) continue;
+                const RowCtx cxt = v.sCtx[k];
+                info[u] = cxt.info;
+                if ((cxt.info >> 9) & 1u) {
+                    const uint64_t hb = cxt.base & ((1ull << kRangeShift) - 1ull);
+                    aux[u] = cxt.aoff + e;
+                    val[u] = g.htab[2 * hb + lookup_slot(v.sA[aux[u]], 2u * (uint32_t)(cxt.base >> kRangeShift))];
+                } else {
+                    val[u] = g.ocol[cxt.base + e];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll; u++) {
+                const uint32_t s = s0 + u * (kBlock / 64);
+                if (s >= nseg) break;
+                const uint32_t e = t0 + s * 64 + lane;
+                bool on = false;
+                uint32_t lo = val[u];
+                if (e < total) {
+                    if ((info[u] >> 9) & 1u) {
+                        on = val[u] != 0u;
+                        lo = aux[u] | (val[u] == v.sA[aux[u]] + 1u ? 1u << 31 : 0u);
+                    } else {
+                        const uint32_t fb = lds_hash(val[u]) >> (32u - ((info[u] >> 20) & 31u));
+                        on = (v.sFlt[((info[u] >> 10) & 1023u) + (fb >> 5)] >> (fb & 31u)) & 1u;
+                    }
+                }
+                const uint64_t m = __ballot(on);
+                if (on) q[qn + bits_below(m)] = (uint64_t)info[u] << 32 | lo;
+                qn += (uint32_t)__popcll(m);
+                if (qn >= 64u) {
+                    qn -= 64u;
+                    settle(qn, 64u);
+                }
+            }
+        }
+    }
+    if (qn) settle(0, qn);
+    __syncthreads();
+    return sumd;
+}
+
+// Processes one LDS batch: build, then the DFS over its items (lds_items).  The
+// plan's level records are in sMisc[M_LEV..].  WALK fixes the walk at compile
+// time where the launch serves one plan (the walks need different registers);
+// kWalkAny picks it per plan.
 enum { kWalkAny = 0, kWalkGroup = 1, kWalkLane = 2, kWalkLaneEmit = 3, kWalkNone = 4 };
 template <int PC, int WALK>
 __device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v,
@@ -820,188 +1119,11 @@ __device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v
                               const KOut &out, uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
 {
     const int tid = threadIdx.x;
-    const int L = pl.L;
-    uint64_t *sE = v.sE;
-    uint64_t *sHBeg = v.sHBeg;
-    RootRec *sRoot = v.sRoot;
-    uint32_t *sA = v.sA, *sPre = v.sPre, *sHKey = v.sHKey, *sMisc = v.sMisc;
-    uint16_t *sHVal = v.sHVal;
-    uint8_t *sJRoot = v.sJRoot;
-    // bitmaps are built only when some level intersects with a bitmap row
-    const bool needE = pl.reads_rows != 0;
     const uint64_t t_build = wall_clock64();
-
-    if (tid < (int)nr) sRoot[tid] = recs[first + tid];
-    __syncthreads();
-    const RootRec last = sRoot[nr - 1];
-    const uint32_t sumd = last.doff + last.d;
-    const uint32_t ew = last.eoff + last.d * ((last.d + 63) >> 6);
-    const uint32_t hsl = last.hoff + hash_slots_dev(last.d);
-    if (needE) {
-        for (uint32_t i = tid; i < ew; i += kBlock) sE[i] = 0;
-        for (uint32_t i = tid; i < hsl; i += kBlock) sHKey[i] = 0;
-    }
-    if (tid == 0) sMisc[M_NEXT] = 0;
-    __syncthreads();
-
-    // rows, hash tables and "higher" ranges of every row vertex.  A thread
-    // holds at most kRowsPer rows; their row entries, then their vertex
-    // records, are loaded together.
-    constexpr int kRowsPer = (int)(LdsBudget::kMaxSumDeg / kBlock);
-    static_assert(LdsBudget::kMaxSumDeg % kBlock == 0, "rows per thread");
-    uint32_t rvx[kRowsPer], rlo[kRowsPer];
-#pragma unroll
-    for (int q = 0; q < kRowsPer; q++) {
-        const uint32_t j = (uint32_t)tid + (uint32_t)q * kBlock;
-        rvx[q] = 0;
-        rlo[q] = 0;
-        if (j < sumd) {
-            uint32_t lo = 0, hi = nr;
-            while (hi - lo > 1) {
-                uint32_t mid = (lo + hi) >> 1;
-                if (sRoot[mid].doff <= j) lo = mid; else hi = mid;
-            }
-            rlo[q] = lo;
-            const RootRec rr = sRoot[lo];
-            rvx[q] = g.ocol[rr.rbeg + (j - rr.doff)];
-        }
-    }
-    VInfo rvi[kRowsPer];
-    if (needE) {
-#pragma unroll
-        for (int q = 0; q < kRowsPer; q++)
-            if ((uint32_t)tid + (uint32_t)q * kBlock < sumd) rvi[q] = g.vinfo[rvx[q]];
-    }
-#pragma unroll
-    for (int q = 0; q < kRowsPer; q++) {
-        const uint32_t j = (uint32_t)tid + (uint32_t)q * kBlock;
-        if (j >= sumd) break;
-        const RootRec rr = sRoot[rlo[q]];
-        const uint32_t jl = j - rr.doff;
-        const uint32_t vx = rvx[q];
-        sA[j] = vx;
-        sJRoot[j] = (uint8_t)rlo[q];
-        if (!needE) continue;
-        const uint32_t H = hash_slots_dev(rr.d);
-        uint32_t s = hash_slot(vx, H);
-        for (;;) {
-            if (atomicCAS(&sHKey[rr.hoff + s], 0u, vx + 1u) == 0u) {
-                sHVal[rr.hoff + s] = (uint16_t)jl;
-                break;
-            }
-            s = (s + 1) & (H - 1);
-        }
-        const VInfo vi = rvi[q];
-        sHBeg[j] = vi.hbeg | ((uint64_t)vi.hlen << kRangeShift);
-        // work units: the range's entries, or the root's neighbours on the
-        // larger-key side of the row (later in ascending rows, earlier in
-        // descending ones) to look up in the range's table
-        sPre[j] = use_search(vi.hlen, rr.d, pl.bin_ratio) ? (g.asc ? rr.d - 1 - jl : jl) : vi.hlen;
-    }
-    __syncthreads();
-    if (needE) {
-        block_excl_scan(sPre, sumd, sMisc + 28);
-        const uint32_t total = sPre[sumd];
-        // bitmap: each adjacent pair (v, w), key(v) < key(w), is found from v.
-        // Every thread takes kChunk consecutive work units: one search for the
-        // row of the first, then the rows advance with the units.  The units'
-        // entries are loaded in a first pass, back to back, and probed in a
-        // second, so a thread waits once for its kChunk loads.
-        constexpr uint32_t kChunk = 8;
-        for (uint32_t e0 = tid * kChunk; e0 < total; e0 += kBlock * kChunk) {
-            uint32_t lo = 0, hi = sumd;  // largest j with sPre[j] <= e0
-            while (hi - lo > 1) {
-                uint32_t mid = (lo + hi) >> 1;
-                if (sPre[mid] <= e0) lo = mid; else hi = mid;
-            }
-            const uint32_t jfirst = lo;
-            const uint32_t e1 = e0 + kChunk < total ? e0 + kChunk : total;
-            // per-row context, refreshed when the units cross into the next row
-            uint32_t j, jn;  // row, first unit of the next row (sPre[sumd] = total)
-            RootRec rr;
-            uint32_t j0, jl, W, H, hl;
-            uint64_t hb;
-            bool srch;
-            auto load_row = [&]() {
-                rr = sRoot[sJRoot[j]];
-                j0 = sPre[j];
-                jl = j - rr.doff;
-                W = (rr.d + 63) >> 6;
-                H = hash_slots_dev(rr.d);
-                const uint64_t hv = sHBeg[j];
-                hb = hv & ((1ull << kRangeShift) - 1ull);
-                hl = (uint32_t)(hv >> kRangeShift);
-                srch = use_search(hl, rr.d, pl.bin_ratio);
-            };
-            auto restart = [&]() {
-                j = jfirst;
-                jn = sPre[j + 1];
-                load_row();
-            };
-            auto seek = [&](uint32_t e) {
-                if (e >= jn) {
-                    do {
-                        j++;
-                        jn = sPre[j + 1];
-                    } while (e >= jn);
-                    load_row();
-                }
-            };
-            uint32_t ent[kChunk];
-            restart();
-#pragma unroll
-            for (uint32_t k = 0; k < kChunk; k++) {
-                const uint32_t e = e0 + k;
-                ent[k] = 0;
-                if (e < e1) {
-                    seek(e);
-                    if (!srch) ent[k] = g.ocol[hb + (e - j0)];
-                }
-            }
-            restart();
-#pragma unroll
-            for (uint32_t k = 0; k < kChunk; k++) {
-                const uint32_t e = e0 + k;
-                if (e >= e1) break;
-                seek(e);
-                const uint32_t off = e - j0;
-                if (srch) {
-                    // neighbour i of the root on the larger-key side of row j:
-                    // is A[i] in A[j]'s larger-key range?  (its lookup table)
-                    const uint32_t i = g.asc ? jl + 1 + off : off;
-                    const uint32_t a = sA[rr.doff + i] + 1u, size = 2 * hl;
-                    const uint32_t *t = g.htab + 2 * hb;
-                    uint32_t s = lookup_slot(a - 1u, size);
-                    for (;;) {
-                        const uint32_t x = t[s];
-                        if (x == a) {
-                            set_pair(sE + rr.eoff, W, jl, i, pl.upper);
-                            break;
-                        }
-                        if (x == 0u) break;
-                        s = s + 1 == size ? 0 : s + 1;
-                    }
-                    continue;
-                }
-                const uint32_t w = ent[k];
-                uint32_t s = hash_slot(w, H);
-                for (;;) {
-                    const uint32_t key = sHKey[rr.hoff + s];
-                    if (key == 0u) break;
-                    if (key == w + 1u) {  // a row holds each vertex once
-                        set_pair(sE + rr.eoff, W, jl, sHVal[rr.hoff + s], pl.upper);
-                        break;
-                    }
-                    s = (s + 1) & (H - 1);
-                }
-            }
-        }
-        __syncthreads();
-    }
-
+    const uint32_t sumd = build_batch(g, pl, v, recs, first, nr, cnt);
     if (tid == 0) prof_add(out, 3, blockIdx.x, t_build);  // staging + bitmap build
 
-    if (L < 3) return;
+    if (pl.hits) return;  // the pairs found are the count
     const uint32_t items = lds_items(pl, v, sumd, cnt);
     if (WALK == kWalkNone || items == 0) {
         __syncthreads();  // the next batch reuses the LDS arrays
@@ -1965,7 +2087,9 @@ static hipError_t launch_lds_lg(int cus, hipStream_t st, const KGraph &g, const 
                                 unsigned long long *cursor, const KOut &out, bool dense)
 {
     constexpr int P = 1 << LG;
-    const LdsLayout lay = make_lds_layout(LG, lds_stack_words(pl, LG), pl.L);
+    LdsNeeds need;
+    need.add(pl, LG);
+    const LdsLayout lay = make_lds_layout(LG, need);
 #define BEEP_RUN(MW, WALK) launch_lds_p<P, MW, WALK>(cus, lay.bytes, st, g, pl, recs, bf, bc, b0, b1, cursor, lay, out)
     if (pl.closed) return dense ? BEEP_RUN(7, kWalkNone) : BEEP_RUN(1, kWalkNone);
     if constexpr (LG <= 3) {
@@ -2050,9 +2174,9 @@ static hipError_t launch_lds_multi_p(int cus, hipStream_t st, const MultiQuery *
 }
 
 hipError_t launch_lds_multi(int cus, hipStream_t st, const MultiQuery *qs, const MultiWork *work,
-                            uint32_t nwork, unsigned long long *cursor, uint32_t stack_words, int levels, int lg)
+                            uint32_t nwork, unsigned long long *cursor, const LdsNeeds &need, int lg)
 {
-    const LdsLayout lay = make_lds_layout(lg, stack_words, levels);
+    const LdsLayout lay = make_lds_layout(lg, need);
     switch (lg) {
 #define BEEP_CASE(LG) \
     case LG: return launch_lds_multi_p<(1 << LG)>(cus, st, qs, work, nwork, cursor, lay);

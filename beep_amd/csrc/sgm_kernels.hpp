@@ -30,9 +30,9 @@ struct KPlan {
     int32_t skip_split;  // skip x_1 < split(u) (sgm_kernelsLD.cuh:60)
     int32_t emit;        // BEEP_EMIT_*
     // LDS bitmap build: a row vertex whose larger-key range is longer than
-    // bin_ratio x the root's degree looks the root's larger-key neighbours up
-    // in the range's lookup table instead of streaming the range (0: always,
-    // ~0u: never)
+    // bin_ratio x the row's partners (pair_partners) looks those up in the
+    // range's lookup table instead of streaming the range (0: always, ~0u:
+    // never)
     uint32_t bin_ratio;
     // Count-only plans whose last level L-1 does not intersect with the row
     // of x_{L-2}: C_{L-1} depends on x_{L-2} only through the exclusion of
@@ -70,6 +70,8 @@ struct KPlan {
     // Count-only plans whose count below x_1 is a function of |C_2| = c and
     // the root's row length d alone (diamond: c (c - 1) / 2); see closed_count.
     int32_t closed;
+    int32_t kept;  // only bitmap rows from the split on are read
+    int32_t hits;  // the LDS build counts the pairs it finds, no bitmap is needed
 };
 
 // KPlan::closed: triangle-like plans (L = 3), or a summed level 3 whose set is
@@ -97,6 +99,22 @@ __host__ __device__ inline uint32_t lds_stack_words(const KPlan &pl, int lg)
     const int group = pl.L > 3 ? pl.L - 3 : 1, lane = lds_lane_walk(pl, lg) ? (pl.L - 4) << lg : 0;
     return (uint32_t)(group > lane ? group : lane);
 }
+
+// What a launch needs of the LDS layout (see make_lds_layout).
+struct LdsNeeds {
+    uint32_t stack_words = 1;
+    int levels = 3;
+    bool rows = false, bitmap = false, walk = false;
+    void add(const KPlan &pl, int lg)
+    {
+        const uint32_t w = lds_stack_words(pl, lg);
+        if (w > stack_words) stack_words = w;
+        if (pl.L > levels) levels = pl.L;
+        rows |= pl.reads_rows != 0;
+        bitmap |= pl.reads_rows && !pl.hits;
+        walk |= !pl.closed;
+    }
+};
 
 // Per-vertex record read when the vertex appears in a root's row: where its
 // bitmap-build scan range starts in ocol and how long it is (one 16-byte

@@ -489,3 +489,21 @@ def test_clique_walk_row_widths(core, k):
         assert r["count"] == o["count"]
         if emit:
             assert (r["hash_sum"], r["hash_xor"]) == (o["hash_sum"], o["hash_xor"])
+
+
+@pytest.mark.parametrize("build", [B.BUILD_AUTO, B.BUILD_SCAN, B.BUILD_SEARCH])
+@pytest.mark.parametrize("core", [3, 64, 65, 130, 300, 512])
+def test_lds_build_row_widths(core, build):
+    """Streamed and looked-up units on rows at the edges of every lane class
+    (several tiles of units for the wide ones), with kept rows only (diamond,
+    w5), all rows (4star's neighbours, wedge-like tails) and counted pairs."""
+    g = _roots_over_core(core, 9)
+    og = oracle_graph(g)
+    for name in ("triangle", "tailed_triangle", "diamond", "4clique", "w5"):
+        for mode in (B.SGM, B.SGC):
+            say("build widths", core, build, name, mode)
+            s, d = P.directed(P.read_mtx_edges(name))
+            pp = B.Prepared(g, B.Plan.from_edges(s, d, mode))
+            pp.upload(0)
+            o = O.Prepared(og, O.plan(s, d, mode)).count(want_hash=False)
+            assert pp.count(build_mode=build)["count"] == o["count"]
