@@ -620,6 +620,7 @@ __device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, ui
             if (on) {
                 const uint32_t x = take();
                 const uint64_t *Ex = E + x * W;
+                const bool end = L == 4 && --left == 0;  // the item's last x_2
                 uint32_t pc = 0;
 #pragma unroll
                 for (int k = 0; k < WT; k++) {
@@ -631,6 +632,10 @@ __device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, ui
                     }
                 }
                 cnt += pc;
+                if (end) {
+#pragma unroll
+                    for (int k = 0; k < WT; k++) S[k] = 0ull;
+                }
             }
         }
     }
