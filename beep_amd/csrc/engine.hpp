@@ -68,7 +68,7 @@ struct DevRoots {
     std::vector<HubRound> rounds;
     uint64_t arena_budget = 0;            // bytes the rounds were cut for
     uint64_t arena_words = 0, arena_slots = 0;
-    uint64_t don_words = 0, don_records = 0;  // upper bounds of the donation ring
+    uint64_t don_words = 0, don_records = 0, don_fine = 0;  // upper bounds of the donation ring
     void release();
 };
 

@@ -306,6 +306,7 @@ void upload(Prep &pp, int device, int p_skip_split, uint64_t arena_budget)
             // donation: at most one slot of W words and ceil(d/16)+1 records per item
             R.don_words += (uint64_t)(r.d - r.jbeg) * W;
             R.don_records += (uint64_t)(r.d - r.jbeg) * ((r.d + 15) / 16 + 1);
+            R.don_fine += (uint64_t)(r.d - r.jbeg) * (r.d + 1);
             hubs.push_back(r);
         }
         if (arena_budget == 0) {
@@ -438,7 +439,10 @@ ScratchNeeds scratch_needs(const Prep &pp, const Plan &p, const beep_opts &o, in
                       hub_wave_words(nlev, std::max<uint32_t>(R.wmax, 1));
     }
     if (hub_donates(p, o, R)) {
+        // records: as many as chunks of 16 x_2 can give; up to 2^18 (6 MB) as
+        // many as single x_2 can.  An item that finds the ring full is walked.
         n.queue_cap = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 22, R.don_records));
+        n.queue_cap = std::max(n.queue_cap, std::min<uint64_t>(1ull << 18, R.don_fine));
         n.slot_cap = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 26, R.don_words));
     }
     if (o.emit == BEEP_EMIT_BUFFER && o.match_cap) n.dbuf_words = o.match_cap * (uint64_t)p.L;
@@ -560,7 +564,11 @@ LaunchCfg make_launch(const Prep &pp, const Plan &p, const beep_opts &o, const S
         c.hq.slot_tail = s.ctr + kCtrSlot;
         c.hq.donated = s.ctr + kCtrDonated;
         c.hq.split_min = o.donate_min ? o.donate_min : 64;
-        c.hq.chunk = c.hq.split_min;
+        // a donated x_2 heads a subtree of the levels below: the deeper the plan,
+        // the fewer of them one wave takes (kp.chunk, as for the LDS batches; with
+        // 64 whatever the depth, W5's hashed matches on 20,000 vertices waited 13
+        // of 17 ms for a hundred records)
+        c.hq.chunk = std::min(c.hq.split_min, std::max(c.kp.chunk, 1u));
     }
     c.lmin = 0;
     if (o.lanes > 0)
