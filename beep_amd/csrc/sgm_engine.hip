@@ -433,17 +433,19 @@ ScratchNeeds scratch_needs(const Prep &pp, const Plan &p, const beep_opts &o, in
         n.hash_slots = R.arena_slots;
     }
     const int nlev = p.L > 3 ? p.L - 3 : 1;
-    if (R.nhubs) {
+    const bool pair5 = hub_pair5(p.L, pair_summed(p, o.emit), std::max<uint32_t>(R.wmax, 1));
+    if (R.nhubs && !pair5) {
         // per wave: nlev stack rows + the row of x_1 (used when they do not fit LDS)
         n.stk_words = (uint64_t)hub_grid_of(R, nlev, pair_summed(p, o.emit), cus) * (kBlock / 64) *
-                      hub_wave_words(nlev, std::max<uint32_t>(R.wmax, 1));
+                      hub_wave_words(nlev, std::max<uint32_t>(R.wmax, 1), pair_summed(p, o.emit));
     }
     if (hub_donates(p, o, R)) {
         // records: as many as chunks of 16 x_2 can give; up to 2^18 (6 MB) as
         // many as single x_2 can.  An item that finds the ring full is walked.
         n.queue_cap = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 22, R.don_records));
         n.queue_cap = std::max(n.queue_cap, std::min<uint64_t>(1ull << 18, R.don_fine));
-        n.slot_cap = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 26, R.don_words));
+        // (records of paired items hold no candidate set)
+        n.slot_cap = pair5 ? 1 : std::max<uint64_t>(1, std::min<uint64_t>(1ull << 26, R.don_words));
     }
     if (o.emit == BEEP_EMIT_BUFFER && o.match_cap) n.dbuf_words = o.match_cap * (uint64_t)p.L;
     if (o.profile) n.prof_words = (uint64_t)kProfPhases * kProfSlots;

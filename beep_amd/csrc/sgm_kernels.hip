@@ -182,8 +182,8 @@ constexpr uint32_t kPairMembers = (1u << kPairSlices) - 1u;
 // A 5-vertex pair plan's hub item of more than kPairSplitWork member-rounds
 // (|C_2| x rounds of 64 words of B) is donated in parts of about
 // kPairChunkWork member-rounds, whole rounds each.
-constexpr uint64_t kPairSplitWork = 1u << 13;
-constexpr uint32_t kPairChunkWork = 1u << 12;
+constexpr uint64_t kPairSplitWork = 1u << 11;
+constexpr uint32_t kPairChunkWork = 1u << 10;
 
 // Compute unit the wave runs on, as a slot below 2048: the XCC (HW_REG_XCC_ID
 // bits 2:0) and, within it, shader engine, shader array and CU (HW_REG_HW_ID
@@ -1405,6 +1405,36 @@ __device__ __forceinline__ uint32_t select_bit(uint64_t w, uint32_t k)
     return (uint32_t)__builtin_ctzll(w);
 }
 
+// Bit-sliced counters of the paired levels: adds a word of weight 2^J.
+template <int J>
+__device__ __forceinline__ void ripple_add(uint64_t *sl, uint64_t c)
+{
+#pragma unroll
+    for (int j = J; j < kPairSlices; j++) {
+        if (c) {
+            const uint64_t t = sl[j] & c;
+            sl[j] ^= c;
+            c = t;
+        }
+    }
+}
+
+// a + b + c = 2 h + l, bit by bit
+__device__ __forceinline__ uint64_t full_add(uint64_t &l, uint64_t b, uint64_t c)
+{
+    const uint64_t u = l ^ b, h = (l & b) | (u & c);
+    l = u ^ c;
+    return h;
+}
+
+// Adds eight words to the slices 0..2; returns the word of weight 8 left over.
+__device__ __forceinline__ uint64_t add8(uint64_t *sl, const uint64_t *c)
+{
+    const uint64_t f0 = full_add(sl[1], full_add(sl[0], c[0], c[1]), full_add(sl[0], c[2], c[3]));
+    const uint64_t f1 = full_add(sl[1], full_add(sl[0], c[4], c[5]), full_add(sl[0], c[6], c[7]));
+    return full_add(sl[2], f0, f1);
+}
+
 // Hub DFS: one wave per (hub, x_1) item; lane i owns words i, i+64, ...
 // The candidate stack (nlev x wmax words per wave) and, when the plan reads
 // it, the bitmap row of x_1 live in LDS (LDSBUF) or, for very wide hubs, in a
@@ -1417,9 +1447,7 @@ __device__ __forceinline__ uint32_t select_bit(uint64_t w, uint32_t k)
 // each a (hub, x_1, slot, [lo, hi)) record appended to the queue with one
 // atomic.  mode 1 (the next launch on the stream) drains the queue: every
 // wave of the grid takes chunks and walks the x_2 in [lo, hi) of its chunk.
-// PAIR compiles in the paired last levels; a 5-vertex pair plan's item is one
-// paired pass, so its records hold ranges [lo, hi) of the pass's positions
-// of B (whole rounds of 64 words) instead of x_2 ranges.
+// PAIR compiles in the paired last levels (5-vertex pair plans: hub_pair5_kernel).
 template <bool LDSBUF, bool PAIR>
 __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g, KPlan pl,
                                                          const HubRec *__restrict__ hubs,
@@ -1446,7 +1474,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
     bool row1 = false;
     for (int l = 2; l < L; l++) row1 |= (sQM[l] & 2u) != 0;
     uint64_t *my;
-    const uint64_t wave_words = hub_wave_words(nlev, wmax);
+    const uint64_t wave_words = hub_wave_words(nlev, wmax, PAIR);
     if (LDSBUF) my = hsm + (uint64_t)wv * wave_words;
     else my = stk + ((uint64_t)blockIdx.x * (kBlock / 64) + wv) * wave_words;
     uint64_t *e1 = my + (uint64_t)nlev * wmax;
@@ -1555,9 +1583,8 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
     };
 
     // Paired last levels (pl.pair), l = L-2 = b: S = C_{l-1} in the stack with
-    // x_1..x_{l-2} fixed, B = level b without its constraints on x_a = x_{l-1},
-    // cut to the positions [plo, phi) (a donated part of an item; words at
-    // multiples of 64).  The three levels add sum over x_b in B of
+    // x_1..x_{l-2} fixed, B = level b without its constraints on x_a = x_{l-1}.
+    // The three levels add sum over x_b in B of
     // C(|S n E[x_b]|, 2).  Returns true when the deadline passed before it was
     // done (a hub of hundreds of thousands of neighbours makes one call long):
     // the item is left with part of its count.
@@ -1568,23 +1595,21 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
     //   sum over p in B of C(c_p, 2)
     // over the rows of S alone.  In each round of 64 words a lane keeps the
     // c_p of its word's 64 positions as bit-sliced counters (slice j = bit j
-    // of every c_p), adds the members' words with a ripple carry, and at the
-    // round's end takes
+    // of every c_p), adds the members' words eight at a time through full
+    // adders, and at the round's end takes
     //   sum_p C(c_p, 2) = sum_j 2^(j-1) (2^j - 1) |sl_j|
     //                     + sum_{i<j} 2^(i+j) |sl_i & sl_j|.
     // Every member row is read once per round where B can hold candidates.
-    // The members come from a list in the next stack row (u32, two rows in
+    // The members come from a list in the next stack row (u32, eight rows in
     // flight) when it holds them, else straight from S's words.  An S with more
     // members than the counters hold takes the walk at the end: B restricted
     // to the union of the members' rows, then C(|S n E[x_b]|, 2) for every x_b
     // in it.
-    auto pair_count = [&](int l, uint32_t plo, uint32_t phi) -> bool {
+    auto pair_count = [&](int l) -> bool {
         uint32_t steps = 0;
         const uint64_t *S = my + (uint64_t)(l - 3) * wmax;
         uint64_t *Bv = my + (uint64_t)(l - 2) * wmax;
-        uint32_t blo = word_lo(l);
-        if ((plo >> 6) > blo) blo = plo >> 6;
-        const uint32_t bhi = phi >= (W << 6) ? W : (phi >> 6);  // B's words: [blo, bhi)
+        const uint32_t blo = word_lo(l), bhi = W;  // B's words: [blo, bhi)
         const uint32_t slo = sWlo[wv][l - 1];
         if (blo >= bhi) return false;
         // B's mask on word w (x_a's constraints left out)
@@ -1607,8 +1632,10 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
             return t;
         };
         {
-            uint32_t *list = (uint32_t *)Bv;
-            const uint32_t cap = 2u * wmax < kPairMembers ? 2u * wmax : kPairMembers;
+            // members: in the next stack row, or, where rows are short, after the rows
+            uint32_t *list = (uint32_t *)(wmax >= kPairListWords ? Bv : my + (uint64_t)(nlev + 1) * wmax);
+            uint32_t cap = 2u * (wmax >= kPairListWords ? wmax : kPairListWords);
+            if (cap > kPairMembers) cap = kPairMembers;
             uint32_t ns = 0;
             for (uint32_t rr = slo >> 6; rr < R; rr++) {
                 const uint32_t w = rr * 64 + lane;
@@ -1632,41 +1659,24 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
                 }
                 const int nb = 32 - __builtin_clz(ns);  // bits of the largest c_p
+                // A row of at most 32 words leaves lanes idle: the wave splits
+                // into G groups of P lanes, each with every G-th member.
+                const uint32_t P = W <= 16u ? 16u : W <= 32u ? 32u : 64u, G = 64u / P;
+                const uint32_t grp = (uint32_t)lane / P;
+                auto member = [&](uint32_t x, uint32_t w) -> uint64_t {
+                    if (G > 1u) return Eh[__umul24(x - rlo, W) + w];
+                    x = (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+                    return Eh[(uint64_t)(x - rlo) * W + w];
+                };
                 for (uint32_t rr = blo >> 6; rr * 64 < bhi; rr++) {
                     if ((++steps & 15u) == 0u && past(dl)) return true;
-                    const uint32_t w = rr * 64 + lane;
+                    const uint32_t w = rr * 64 + ((uint32_t)lane & (P - 1u));
                     const uint64_t bc = (w < bhi && w >= blo) ? b_word(w) : 0ull;
                     if (__ballot(bc != 0ull) == 0ull) continue;
                     uint64_t sl[kPairSlices];
 #pragma unroll
                     for (int j = 0; j < kPairSlices; j++) sl[j] = 0ull;
-                    auto add = [&](uint64_t c) {
-#pragma unroll
-                        for (int j = 0; j < kPairSlices; j++) {
-                            if (c) {
-                                const uint64_t t = sl[j] & c;
-                                sl[j] ^= c;
-                                c = t;
-                            }
-                        }
-                    };
-                    auto word_of = [&](uint32_t s) -> uint64_t {
-                        return bc ? Eh[(uint64_t)(s - rlo) * W + w] & bc : 0ull;
-                    };
-                    if (listed) {
-                        for (uint32_t b0 = 0; b0 < ns; b0 += 64) {
-                            const uint32_t mine = b0 + lane < ns ? list[b0 + lane] : 0u;
-                            const uint32_t nk = ns - b0 < 64u ? ns - b0 : 64u;
-                            uint32_t k = 0;
-                            for (; k + 2 <= nk; k += 2) {  // two member words in flight
-                                const uint64_t r0 = word_of(__builtin_amdgcn_readlane(mine, k));
-                                const uint64_t r1 = word_of(__builtin_amdgcn_readlane(mine, k + 1));
-                                add(r0);
-                                add(r1);
-                            }
-                            for (; k < nk; k++) add(word_of(__builtin_amdgcn_readlane(mine, k)));
-                        }
-                    } else {
+                    if (!listed) {
                         for (uint32_t sr = slo >> 6; sr < R; sr++) {  // S's words, 64 at a time
                             const uint32_t sw = sr * 64 + lane;
                             uint64_t v = (sw < W && sw >= slo) ? S[sw] : 0ull;
@@ -1676,17 +1686,47 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
                                 const int f = __builtin_ctzll(bal);
                                 const uint64_t vf = __shfl(v, f, 64);
                                 if (lane == f) v &= v - 1ull;
-                                add(word_of(((sr * 64 + (uint32_t)f) << 6) + (uint32_t)__builtin_ctzll(vf)));
+                                const uint32_t x = ((sr * 64 + (uint32_t)f) << 6) + (uint32_t)__builtin_ctzll(vf);
+                                ripple_add<0>(sl, bc && grp == 0 ? Eh[(uint64_t)(x - rlo) * W + w] : 0ull);
                             }
                         }
+                    } else if (bc) {
+                        // eight members' words at a time through full adders; what
+                        // overflows the three low slices ripples on
+                        uint32_t m0 = (uint32_t)grp;
+                        for (; m0 + 7u * G < ns; m0 += 8u * G) {
+                            uint64_t c[8];
+#pragma unroll
+                            for (int i = 0; i < 8; i++) c[i] = member(list[m0 + i * G], w);
+                            ripple_add<3>(sl, add8(sl, c));
+                        }
+                        for (; m0 < ns; m0 += G) ripple_add<0>(sl, member(list[m0], w));
+                    }
+                    // groups hold the counters of different members: add them up
+                    for (uint32_t o = P; o < 64u; o <<= 1) {
+                        uint64_t carry = 0;
+#pragma unroll
+                        for (int j = 0; j < kPairSlices; j++)
+                            if (j < nb) {
+                                const uint64_t y = __shfl_xor(sl[j], o, 64), x = sl[j];
+                                sl[j] = x ^ y ^ carry;
+                                carry = (x & y) | (carry & (x ^ y));
+                            }
                     }
                     uint64_t acc = 0;
+                    if (grp == 0) {
 #pragma unroll
-                    for (int j = 1; j < kPairSlices; j++) {
-                        if (j < nb) {
-                            acc += ((1ull << (j - 1)) * ((1ull << j) - 1ull)) * (uint64_t)__popcll(sl[j]);
+                        for (int j = 0; j < kPairSlices; j++) {
+                            if (j < nb) {
+                                sl[j] &= bc;
+                                if (j == 0) continue;
+                                // sum over i < j of 2^i |sl_i & sl_j|, highest i first
+                                uint32_t t = 0;
 #pragma unroll
-                            for (int i = 0; i < j; i++) acc += (uint64_t)__popcll(sl[i] & sl[j]) << (i + j);
+                                for (int i = j - 1; i >= 0; i--) t = (t << 1) + (uint32_t)__popcll(sl[i] & sl[j]);
+                                acc += (uint64_t)t << j;
+                                acc += ((1ull << (j - 1)) * ((1ull << j) - 1ull)) * (uint64_t)__popcll(sl[j]);
+                            }
                         }
                     }
                     cnt += acc;
@@ -1781,9 +1821,8 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
                 pos = xget(l - 1) + 1u;
                 continue;
             }
-            if (PAIR && l == L - 2) {  // levels L-3..L-1 at once; at l = 3 [pos0, hi2) cuts B
-                const bool top = l == 3;
-                if (pair_count(l, top ? pos0 : 0u, top ? hi2 : 0xffffffffu)) break;  // the next claim records the stop
+            if (PAIR && l == L - 2) {  // levels L-3..L-1 at once
+                if (pair_count(l)) break;  // the next claim records the stop
                 if (l == 3) break;
                 --l;
                 pos = xget(l - 1) + 1u;
@@ -1942,49 +1981,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
             }
         }
         c2 = (uint32_t)wave_sum_u64(c2);
-        if (PAIR && L == 5) {
-            // The item is one paired pass over B's words with S = C_2; a long one
-            // donates ranges of B's rounds (the sum splits over B's positions;
-            // B's bounds depend on x_1 only).
-            const uint32_t r0 = word_lo(3) >> 6;
-            const uint32_t nr = R > r0 ? R - r0 : 0u;
-            uint32_t rpc = c2 ? kPairChunkWork / c2 : nr;
-            if (rpc < 1u) rpc = 1u;
-            const uint32_t nc = (nr + rpc - 1u) / rpc;
-            if (hq.q && nc >= 2u && (uint64_t)c2 * nr > kPairSplitWork) {
-                unsigned long long sb = 0;
-                if (lane == 0) sb = atomicAdd(hq.slot_tail, (unsigned long long)W);
-                sb = __shfl(sb, 0, 64);
-                if (sb + W <= hq.slot_cap) {
-                    unsigned long long qb = 0;
-                    if (lane == 0) qb = atomicAdd(hq.tail, (unsigned long long)nc);
-                    qb = __shfl(qb, 0, 64);
-                    if (qb + nc <= hq.cap) {
-                        if (lane == 0) atomicAdd(hq.donated, (unsigned long long)nc);
-                        for (uint32_t rr = 0; rr < R; rr++) {
-                            const uint32_t w = rr * 64 + lane;
-                            if (w < W) hq.slots[sb + w] = my[w];
-                        }
-                        for (uint32_t c = lane; c < nc; c += 64) {
-                            HubChunk *rec = hq.q + qb + c;
-                            rec->hub = hidx;
-                            rec->x1 = jl;
-                            rec->slot = sb;
-                            rec->lo = c ? (r0 + c * rpc) << 12 : 0u;
-                            rec->hi = c + 1u == nc ? (W << 6) : (r0 + (c + 1u) * rpc) << 12;
-                        }
-                        continue;
-                    }
-                    for (uint64_t c = qb + lane; c < qb + nc && c < hq.cap; c += 64) {
-                        hq.q[c].lo = 0;
-                        hq.q[c].hi = 0;
-                    }
-                }
-            }
-            dfs3(0, 0xffffffffu);
-            continue;
-        }
-        if (hq.q && c2 > hq.split_min) {
+        if (hq.q && c2 > hq.split_min && !(PAIR && L == 5)) {  // L = 5: one paired pass, no x_2 to donate
             // donate: publish C_2, then cut it into chunks of hq.chunk candidates
             unsigned long long sb = 0;
             if (lane == 0) sb = atomicAdd(hq.slot_tail, (unsigned long long)W);
@@ -2028,6 +2025,259 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
         dfs3(0, 0xffffffffu);
     }
     flush_acc(out, cnt, hs, hx);
+    if (lane == 0) prof_add(out, 1, wslot, t_start);
+}
+
+// Hub items of 5-vertex plans with paired levels (KPlan::pair, L = 5; W5): with
+// x_1 fixed, S = C_2 and B (the candidates of x_3 without x_2's constraints)
+// follow from x_1 alone, and the item adds sum over p in B of C(c_p, 2),
+// c_p = |{s in S : E[s][p]}| (see hub_dfs_kernel's pair_count, which deeper
+// pair plans use).  No DFS, so a kernel of its own: S goes from the bitmap row
+// straight into a list in LDS, nothing else is staged.
+//
+// The lanes take B's words from the first that can hold a candidate on; when
+// fewer than 64 words are left the wave splits into groups of P lanes, each
+// adding every G-th member, and the groups' counters are added at the end.
+// Eight member words are in flight a lane and go through full adders together.
+//
+// An item is short (35 member reads on average on R-MAT scale 20), so what
+// bounds it is the per-item instructions (2,500 VALU in the DFS kernel before)
+// and the latency of its few dependent loads: the registers are kept to 4 waves
+// per SIMD.  R-MAT scale 20, W5: 20.9 ms in the DFS kernel (items and records),
+// 7.0 ms here.
+//
+// mode 0 walks items and cuts long ones into records of whole rounds (P = 64
+// words each); mode 1 drains the records.
+constexpr uint32_t kPairList = 1024;  // members listed at once, per wave
+__global__ __launch_bounds__(kBlock, 4) void hub_pair5_kernel(KPlan pl, const HubRec *__restrict__ hubs,
+                                                              const uint32_t *__restrict__ hub_of_item, uint64_t i0,
+                                                              uint64_t i1, unsigned long long *cursor,
+                                                              const uint64_t *__restrict__ E, KOut out, HubQueue hq,
+                                                              int mode)
+{
+    __shared__ uint32_t sList[kBlock / 64][kPairList];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    uint32_t *list = sList[wv];
+    const uint32_t wslot = blockIdx.x * (kBlock / 64) + wv;
+    const uint64_t dl = *out.dl, t_start = wall_clock64();
+    // level a = 2 is S, level b = 3 is B without x_2; both see x_1 only
+    const bool s_row = (pl.qmask[2] & 2u) != 0, s_gt = (pl.smask[2] & 2u) != 0;
+    const bool b_row = (pl.qmask[3] & 2u) != 0, b_gt = (pl.smask[3] & 2u) != 0;
+    uint64_t cnt = 0;
+
+    // adds the rounds [r0, r1) of item (h, x1); false: the deadline passed
+    auto item_sum = [&](const HubRec &h, uint32_t x1, uint32_t ns, uint32_t r0, uint32_t r1) -> bool {
+        const uint32_t d = h.d, W = (d + 63) >> 6;
+        const uint64_t *Eh = E + h.eoff;
+        const uint64_t *row1 = Eh + (uint64_t)(x1 - h.rlo) * W;
+        const uint32_t slo = s_gt ? x1 >> 6 : 0u, blo = b_gt ? x1 >> 6 : 0u;
+        const uint32_t left = W - blo;
+        const uint32_t P = left <= 8u ? 8u : left <= 16u ? 16u : left <= 32u ? 32u : 64u, G = 64u / P;
+        const uint32_t grp = (uint32_t)lane / P;
+        const int nb = 32 - __builtin_clz(ns);
+        const bool once = ns <= kPairList;
+        // lists the members of rank [from, from + kPairList)
+        auto fill = [&](uint32_t from) {
+            wave_lds_sync();
+            uint32_t base = 0;
+            for (uint32_t w0 = slo; w0 < W; w0 += 64) {
+                const uint32_t w = w0 + lane;
+                uint64_t v = 0;
+                if (w < W) {
+                    v = (s_row ? row1[w] : valid_mask(w, d)) & ~bit_at(x1, w);
+                    if (s_gt) v &= gt_mask(x1, w);
+                }
+                const uint32_t pc = (uint32_t)__popcll(v), inc = wave_incl_scan(pc);
+                uint32_t at = base + inc - pc - from;  // list slot of the word's first member
+                // words of a few members: a lane lists its own; fuller ones: a
+                // word at a time, one lane per bit
+                uint64_t dense = __ballot(pc > 4u);
+                if (pc <= 4u)
+                    while (v) {
+                        if (at < kPairList) list[at] = (w << 6) + (uint32_t)__builtin_ctzll(v);
+                        at++;
+                        v &= v - 1;
+                    }
+                while (dense) {
+                    const int f = __builtin_ctzll(dense);
+                    dense &= dense - 1;
+                    const uint64_t m = (uint64_t)lane_u32((uint32_t)(v >> 32), f) << 32 | lane_u32((uint32_t)v, f);
+                    const uint32_t slot = lane_u32(at, f) + bits_below(m);
+                    if (((m >> lane) & 1u) && slot < kPairList) list[slot] = ((w0 + (uint32_t)f) << 6) + (uint32_t)lane;
+                }
+                base += lane_u32(inc, 63);
+                if (base >= from + kPairList) break;
+            }
+            wave_lds_sync();
+        };
+        if (once) fill(0);
+        uint32_t steps = 0;
+        for (uint32_t r = r0; r < r1; r++) {
+            if ((++steps & 15u) == 0u && past(dl)) return false;
+            const uint32_t w = blo + r * P + ((uint32_t)lane & (P - 1u));
+            uint64_t bc = 0;
+            if (w < W) {
+                bc = (b_row ? row1[w] : valid_mask(w, d)) & ~bit_at(x1, w);
+                if (b_gt) bc &= gt_mask(x1, w);
+            }
+            if (__ballot(bc != 0ull) == 0ull) continue;
+            uint64_t sl[kPairSlices];
+#pragma unroll
+            for (int j = 0; j < kPairSlices; j++) sl[j] = 0ull;
+            for (uint32_t from = 0; from < ns; from += kPairList) {
+                if (!once) fill(from);
+                const uint32_t n = ns - from < kPairList ? ns - from : kPairList;
+                for (uint32_t m0 = 0; m0 < n; m0 += 8u * G) {
+                    uint64_t c[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const uint32_t m = m0 + i * G + grp;
+                        c[i] = 0;
+                        if (G == 1u) {
+                            if (m < n) {
+                                const uint32_t x = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[m]);
+                                const uint64_t *Ex = Eh + (uint64_t)(x - h.rlo) * W;
+                                if (bc) c[i] = Ex[w];
+                            }
+                        } else if (m < n && bc) {
+                            c[i] = Eh[(uint64_t)(list[m] - h.rlo) * W + w];
+                        }
+                    }
+                    uint64_t over = add8(sl, c);
+#pragma unroll
+                    for (int j = 3; j < kPairSlices; j++)
+                        if (__ballot(over != 0ull) != 0ull) {
+                            const uint64_t t = sl[j] & over;
+                            sl[j] ^= over;
+                            over = t;
+                        }
+                }
+                if (!once && past(dl)) return false;
+            }
+            for (uint32_t o = P; o < 64u; o <<= 1) {
+                uint64_t carry = 0;
+#pragma unroll
+                for (int j = 0; j < kPairSlices; j++)
+                    if (j < nb) {
+                        const uint64_t y = __shfl_xor(sl[j], o, 64), x = sl[j];
+                        sl[j] = x ^ y ^ carry;
+                        carry = (x & y) | (carry & (x ^ y));
+                    }
+            }
+            if (grp != 0u) bc = 0;
+            uint64_t acc = 0;
+            sl[0] &= bc;
+#pragma unroll
+            for (int j = 1; j < kPairSlices; j++)
+                if (j < nb) {
+                    sl[j] &= bc;
+                    uint32_t t = 0;  // sum over i < j of 2^i |sl_i & sl_j|, highest i first
+#pragma unroll
+                    for (int i = j - 1; i >= 0; i--) t = (t << 1) + (uint32_t)__popcll(sl[i] & sl[j]);
+                    acc += (uint64_t)t << j;
+                    acc += ((1ull << (j - 1)) * ((1ull << j) - 1ull)) * (uint64_t)__popcll(sl[j]);
+                }
+            cnt += acc;
+        }
+        return true;
+    };
+    // |S| of item (h, x1)
+    auto members = [&](const HubRec &h, uint32_t x1) -> uint32_t {
+        const uint32_t W = (h.d + 63) >> 6;
+        const uint64_t *row1 = E + h.eoff + (uint64_t)(x1 - h.rlo) * W;
+        uint32_t c = 0;
+        for (uint32_t w = (s_gt ? x1 >> 6 : 0u) + lane; w < W; w += 64) {
+            uint64_t v = (s_row ? row1[w] : valid_mask(w, h.d)) & ~bit_at(x1, w);
+            if (s_gt) v &= gt_mask(x1, w);
+            c += (uint32_t)__popcll(v);
+        }
+        return lane_u32(wave_incl_scan(c), 63);
+    };
+    auto hub = [&](uint32_t i) -> HubRec { return hubs[(uint32_t)__builtin_amdgcn_readfirstlane((int)i)]; };
+    auto first_lane64 = [&](uint64_t v) -> uint64_t {
+        return (uint64_t)lane_u32((uint32_t)(v >> 32), 0) << 32 | lane_u32((uint32_t)v, 0);
+    };
+
+    uint32_t parts = 0;  // lane 0's claim state
+    if (mode == 1) {
+        const uint64_t ntail = *hq.tail, nq = ntail < hq.cap ? ntail : hq.cap;
+        for (;;) {
+            uint64_t c = ~0ull;
+            if (lane == 0) {
+                uint64_t cb = 0, ce = 0;
+                if (past(dl)) mark_stop(out);
+                else if (claim_striped(hq.head, nq, wslot % kStripes, parts, 1, cb, ce)) c = cb;
+            }
+            c = first_lane64(c);
+            if (c >= nq) break;
+            const HubChunk ch = hq.q[c];
+            if (ch.lo >= ch.hi) continue;
+            const HubRec h = hub(ch.hub);
+            const uint32_t x1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ch.x1);
+            const uint32_t ns = members(h, x1);
+            if (ns >= 2u) (void)item_sum(h, x1, ns, ch.lo, ch.hi);
+        }
+        flush_acc(out, cnt, 0, 0);
+        if (lane == 0) prof_add(out, 2, wslot, t_start);
+        return;
+    }
+    constexpr uint32_t kClaim = 4;  // items per cursor claim
+    uint64_t nxt = 0, left = 0;
+    for (;;) {
+        if (left == 0) {
+            uint64_t cb = ~0ull, cc = 0;
+            if (lane == 0) {
+                uint64_t b = 0, n = 0;
+                if (past(dl)) mark_stop(out);
+                else if (claim_striped(cursor, i1 - i0, wslot % kStripes, parts, kClaim, b, n)) {
+                    cb = b;
+                    cc = n;
+                }
+            }
+            cb = first_lane64(cb);
+            cc = first_lane64(cc);
+            if (cb == ~0ull) break;
+            nxt = i0 + cb;
+            left = cc;
+        }
+        const uint64_t item = nxt;
+        nxt += kStripes;
+        left--;
+        const uint32_t hidx = hub_of_item[item];
+        const HubRec h = hub(hidx);
+        const uint32_t x1 = h.jbeg + (uint32_t)(item - h.ioff);
+        const uint32_t ns = members(h, x1);
+        if (ns < 2u) continue;  // no pair
+        const uint32_t words = ((h.d + 63) >> 6) - (b_gt ? x1 >> 6 : 0u);
+        const uint32_t rounds = (words + 63u) >> 6;  // more than one: P = 64
+        uint32_t rpc = kPairChunkWork / ns;
+        if (rpc < 1u) rpc = 1u;
+        const uint32_t nc = (rounds + rpc - 1u) / rpc;
+        if (hq.q && nc >= 2u && (uint64_t)ns * rounds > kPairSplitWork) {
+            uint64_t qb = 0;
+            if (lane == 0) qb = atomicAdd(hq.tail, (unsigned long long)nc);
+            qb = first_lane64(qb);
+            if (qb + nc <= hq.cap) {
+                if (lane == 0) atomicAdd(hq.donated, (unsigned long long)nc);
+                for (uint32_t c = lane; c < nc; c += 64) {
+                    HubChunk *rec = hq.q + qb + c;
+                    rec->hub = hidx;
+                    rec->x1 = x1;
+                    rec->slot = 0;
+                    rec->lo = c * rpc;
+                    rec->hi = c + 1u == nc ? rounds : (c + 1u) * rpc;
+                }
+                continue;
+            }
+            // queue full: neutralise the reserved records that exist, walk inline
+            for (uint64_t c = qb + lane; c < qb + nc && c < hq.cap; c += 64) {
+                hq.q[c].lo = 0;
+                hq.q[c].hi = 0;
+            }
+        }
+        if (!item_sum(h, x1, ns, 0, rounds)) continue;  // the next claim records the stop
+    }
+    flush_acc(out, cnt, 0, 0);
     if (lane == 0) prof_add(out, 1, wslot, t_start);
 }
 
@@ -2208,11 +2458,14 @@ hipError_t launch_hub_encode(int grid, hipStream_t st, const KGraph &g, const Hu
     return hipGetLastError();
 }
 
-// Dynamic LDS of the hub DFS: per wave nlev + 1 rows of wmax words.
-static size_t hub_lds_bytes(int nlev, uint32_t wmax) { return (size_t)(kBlock / 64) * hub_wave_words(nlev, wmax) * 8; }
+// Dynamic LDS of the hub DFS: per wave nlev + 1 rows of wmax words (and a member list).
+static size_t hub_lds_bytes(int nlev, uint32_t wmax, bool pair)
+{
+    return (size_t)(kBlock / 64) * hub_wave_words(nlev, wmax, pair) * 8;
+}
 constexpr size_t kHubLdsMax = 96 * 1024;
 
-bool hub_dfs_in_lds(int nlev, uint32_t wmax) { return hub_lds_bytes(nlev, wmax) <= kHubLdsMax; }
+bool hub_dfs_in_lds(int nlev, uint32_t wmax, bool pair) { return hub_lds_bytes(nlev, wmax, pair) <= kHubLdsMax; }
 
 // one cache per instantiation: [in LDS][pair]
 static LdsLaunchCache &hub_dfs_cache(bool in_lds, bool pair)
@@ -2226,7 +2479,7 @@ static LdsLaunchCache &hub_dfs_cache(bool in_lds, bool pair)
 // registers, hence occupancy, that the other plans keep).
 static const void *hub_dfs_fn(int nlev, uint32_t wmax, bool pair)
 {
-    if (hub_dfs_in_lds(nlev, wmax))
+    if (hub_dfs_in_lds(nlev, wmax, pair))
         return pair ? (const void *)hub_dfs_kernel<true, true> : (const void *)hub_dfs_kernel<true, false>;
     return pair ? (const void *)hub_dfs_kernel<false, true> : (const void *)hub_dfs_kernel<false, false>;
 }
@@ -2236,9 +2489,14 @@ hipError_t launch_hub_dfs(int grid, hipStream_t st, const KGraph &g, const KPlan
                           const uint64_t *E, uint64_t *stk, uint32_t wmax, const KOut &out,
                           const HubQueue &hq, int mode)
 {
+    if (hub_pair5(pl.L, pl.pair != 0, wmax)) {
+        hipLaunchKernelGGL(hub_pair5_kernel, dim3(grid), dim3(kBlock), 0, st, pl, hubs, hoi, i0, i1, cursor, E, out, hq,
+                           mode);
+        return hipGetLastError();
+    }
     const int nlev = pl.L > 3 ? pl.L - 3 : 1;
-    const bool in_lds = hub_dfs_in_lds(nlev, wmax);
-    const size_t lds = in_lds ? hub_lds_bytes(nlev, wmax) : 0;
+    const bool in_lds = hub_dfs_in_lds(nlev, wmax, pl.pair != 0);
+    const size_t lds = in_lds ? hub_lds_bytes(nlev, wmax, pl.pair != 0) : 0;
     const void *fn = hub_dfs_fn(nlev, wmax, pl.pair != 0);
     if (in_lds) (void)hub_dfs_cache(true, pl.pair != 0).get(fn, lds);
     void *args[] = {(void *)&g,  (void *)&pl,     (void *)&hubs, (void *)&hoi, (void *)&i0,
@@ -2249,9 +2507,13 @@ hipError_t launch_hub_dfs(int grid, hipStream_t st, const KGraph &g, const KPlan
 
 int hub_dfs_occupancy(int nlev, uint32_t wmax, bool pair)
 {
+    if (hub_pair5(nlev + 3, pair, wmax)) {
+        static LdsLaunchCache cache;
+        return cache.get((const void *)hub_pair5_kernel, 0);
+    }
     const void *fn = hub_dfs_fn(nlev, wmax, pair);
-    const bool in_lds = hub_dfs_in_lds(nlev, wmax);
-    return hub_dfs_cache(in_lds, pair).get(fn, in_lds ? hub_lds_bytes(nlev, wmax) : 0);
+    const bool in_lds = hub_dfs_in_lds(nlev, wmax, pair);
+    return hub_dfs_cache(in_lds, pair).get(fn, in_lds ? hub_lds_bytes(nlev, wmax, pair) : 0);
 }
 
 }  // namespace beep

@@ -192,11 +192,17 @@ struct HubQueue {
     uint32_t chunk = 0;                       // candidates per record
 };
 
-// Words (u64) of one hub-DFS wave's buffer: nlev candidate-stack rows and the
-// bitmap row of x_1.
-__host__ __device__ inline uint64_t hub_wave_words(int nlev, uint32_t wmax)
+// Hub items of 5-vertex plans with paired levels have a kernel of their own,
+// for hubs of up to 2^20 - 1 neighbours (its counters' range).
+__host__ __device__ inline bool hub_pair5(int L, bool pair, uint32_t wmax) { return pair && L == 5 && wmax < (1u << 14); }
+
+// Words (u64) of one hub-DFS wave's buffer: nlev candidate-stack rows, the
+// bitmap row of x_1 and, for paired levels over rows shorter than it, a list
+// of kPairListWords words of S's members.
+constexpr uint32_t kPairListWords = 256;
+__host__ __device__ inline uint64_t hub_wave_words(int nlev, uint32_t wmax, bool pair)
 {
-    return (uint64_t)(nlev + 1) * wmax;
+    return (uint64_t)(nlev + 1) * wmax + (pair && wmax < kPairListWords ? kPairListWords : 0);
 }
 
 struct KOut {

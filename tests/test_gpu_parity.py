@@ -507,3 +507,28 @@ def test_lds_build_row_widths(core, build):
             pp.upload(0)
             o = O.Prepared(og, O.plan(s, d, mode)).count(want_hash=False)
             assert pp.count(build_mode=build)["count"] == o["count"]
+
+
+@pytest.mark.parametrize("core", [600, 1100, 2200, 4300])
+def test_paired_items_on_wide_hubs(core):
+    """W5 on hubs of 8 to 68 words a row: every split of the wave into groups,
+    rows of more than one round, and member lists past their LDS space."""
+    rng = np.random.default_rng(core)
+    p = min(0.5, 600.0 / core)
+    # one hub over `core` vertices, half of them joined to a dense few
+    u = rng.integers(0, 24, size=int(core * 12 * p))
+    v = rng.integers(0, core, size=len(u))
+    edges = {(int(min(a, b)), int(max(a, b))) for a, b in zip(u, v) if a != b}
+    edges |= {(x, core) for x in range(core)}
+    edges |= {(0, x) for x in range(1, core)}
+    pairs = sorted(edges | {(b, a) for a, b in edges})
+    g = B.Graph.from_edges([x for x, _ in pairs], [y for _, y in pairs])
+    og = oracle_graph(g)
+    s, d = P.directed(P.read_mtx_edges("w5"))
+    for mode in (B.SGM, B.SGC):
+        say("paired wide hubs", core, mode)
+        pp = B.Prepared(g, B.Plan.from_edges(s, d, mode))
+        pp.upload(0)
+        o = O.Prepared(og, O.plan(s, d, mode)).count(want_hash=False)
+        for donate in (True, False):
+            assert pp.count(donate=donate)["count"] == o["count"]
