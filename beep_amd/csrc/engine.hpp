@@ -48,7 +48,8 @@ struct HubRound {
     uint64_t i0, i1;      // global item range (DFS)
     uint64_t ewords;      // bitmap words used
     uint64_t hslots;      // hash slots used
-    uint64_t er0 = 0, er1 = 0;  // its rows with a non-empty scan range: enc_rows[er0, er1)
+    uint64_t er0 = 0, er1 = 0;  // its rows with a non-empty scan range outside slices: enc_rows[er0, er1)
+    uint32_t s0 = 0, s1 = 0;    // its slices
 };
 
 // Read-only device records of one prepared root queue.
@@ -61,7 +62,10 @@ struct DevRoots {
     // per hub row: the part of the row vertex's larger-key range the bitmap
     // build streams (start | length << kRangeShift)
     uint64_t *hub_range = nullptr;
-    uint64_t *enc_rows = nullptr;  // per round, the hub rows whose scan range is not empty
+    uint64_t *enc_rows = nullptr;  // per round, the hub rows whose scan range is not empty and in no slice
+    SliceRec *slices = nullptr;    // per round, heaviest first
+    uint32_t slice_kept = 0;       // most kept rows of a hub in slices
+    bool all_sliced = false;       // every hub row with a scan range is in a slice
     int skip_split = -1;  // plan property the hub items were built for
     uint32_t nhubs = 0;
     uint32_t wmax = 0;
@@ -76,6 +80,7 @@ struct DevRoots {
 struct ScratchNeeds {
     uint64_t arena_words = 0, hash_slots = 0, stk_words = 0;
     uint64_t queue_cap = 0, slot_cap = 0, dbuf_words = 0, prof_words = 0;
+    uint64_t queue_min = 0;  // what queue_cap may be cut to where space is short
     uint64_t bytes() const;
 };
 

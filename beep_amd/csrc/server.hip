@@ -214,6 +214,7 @@ static ScratchNeeds max_needs(const ScratchNeeds &a, const ScratchNeeds &b)
     n.hash_slots = std::max(a.hash_slots, b.hash_slots);
     n.stk_words = std::max(a.stk_words, b.stk_words);
     n.queue_cap = std::max(a.queue_cap, b.queue_cap);
+    n.queue_min = std::max(a.queue_min, b.queue_min);
     n.slot_cap = std::max(a.slot_cap, b.slot_cap);
     n.dbuf_words = std::max(a.dbuf_words, b.dbuf_words);
     n.prof_words = std::max(a.prof_words, b.prof_words);
@@ -426,6 +427,10 @@ void Server::run()
                         }
                     }
                     j.bytes = j.need.bytes();
+                    if (j.bytes > pool_bytes) {  // a short donation ring does
+                        j.need.queue_cap = j.need.queue_min;
+                        j.bytes = j.need.bytes();
+                    }
                     if (j.bytes > pool_bytes)
                         throw Error(BEEP_ENOMEM, "the query's predicted scratch exceeds the server pool");
                 } catch (const Error &e) {

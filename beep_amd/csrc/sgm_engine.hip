@@ -31,12 +31,18 @@ hipError_t launch_hub_hash(int grid, hipStream_t st, const KGraph &g, const HubR
                            const unsigned long long *dl);
 hipError_t launch_hub_encode(int grid, hipStream_t st, const KGraph &g, const HubRec *hubs,
                              const uint32_t *hor, const uint64_t *hrange, const uint64_t *rows, uint64_t nrows,
-                             const uint64_t *kv, uint64_t *E, int upper, const KOut &out);
+                             const uint64_t *kv, uint64_t *E, int upper, int count, const KOut &out);
+hipError_t launch_hub_slices(hipStream_t st, const KGraph &g, const HubRec *hubs, const SliceRec *slices, uint32_t n,
+                             const uint64_t *hrange, uint32_t kmax, uint32_t bin_ratio, uint64_t *E, uint32_t *c2,
+                             uint64_t i0, const KOut &out);
+hipError_t launch_hub_closed(int grid, hipStream_t st, const HubRec *hubs, const uint32_t *hoi, uint64_t i0, uint64_t i1,
+                             const uint32_t *c2, int closed, const KOut &out);
 hipError_t launch_hub_dfs(int grid, hipStream_t st, const KGraph &g, const KPlan &pl, const HubRec *hubs,
                           const uint32_t *hoi, uint64_t i0, uint64_t i1, unsigned long long *cursor,
                           const uint64_t *E, uint64_t *stk, uint32_t wmax, const KOut &out,
                           const HubQueue &hq, int mode);
 int hub_dfs_occupancy(int nlev, uint32_t wmax, bool pair);
+int hub_stack_occupancy(int nlev, uint32_t wmax, bool pair);
 
 template <class T>
 static T *dev_alloc(size_t n)
@@ -70,12 +76,13 @@ Variant::~Variant() { delete dev; }
 void DevRoots::release()
 {
     for (void *p : {(void *)recs, (void *)batch_first, (void *)batch_count, (void *)hubs, (void *)hub_of_row,
-                    (void *)hub_of_item, (void *)hub_range, (void *)enc_rows})
+                    (void *)hub_of_item, (void *)hub_range, (void *)enc_rows, (void *)slices})
         if (p) (void)hipFree(p);
     recs = nullptr;
     batch_first = batch_count = hub_of_row = hub_of_item = nullptr;
     hubs = nullptr;
     hub_range = enc_rows = nullptr;
+    slices = nullptr;
 }
 
 void Lane::create(int dev, int ns)
@@ -344,12 +351,44 @@ void upload(Prep &pp, int device, int p_skip_split, uint64_t arena_budget)
             // the bitmap build streams only rows with a non-empty range (a
             // third of the diamond's hub rows on chunglu1m have none)
             std::vector<uint64_t> rows;
+            std::vector<SliceRec> slices;
             for (auto &r : R.rounds) {
                 r.er0 = rows.size();
-                for (uint64_t g = r.g0; g < r.g1; g++)
-                    if (ranges[g] >> kRangeShift) rows.push_back(g);
+                std::vector<std::pair<uint64_t, SliceRec>> sl;
+                for (uint32_t hi = r.h0; hi < r.h1; hi++) {
+                    const HubRec &h = hubs[hi];
+                    const uint32_t kept = h.d - h.rlo;
+                    if (h.rlo && !pp.upper_rows && kept && kept <= kSliceKept) {
+                        // whole bitmap words (64 rows) up to kSliceRows rows or
+                        // about kSliceUnits entries
+                        for (uint32_t j = 0; j < h.d;) {
+                            uint64_t len = 0;
+                            uint32_t e = j;
+                            while (e < h.d && e - j < kSliceRows) {
+                                const uint32_t to = std::min(e + 64u, h.d);
+                                uint64_t more = 0;
+                                for (uint32_t x = e; x < to; x++) more += ranges[h.joff + x] >> kRangeShift;
+                                if (len && len + more > kSliceUnits) break;
+                                len += more;
+                                e = to;
+                            }
+                            if (len) sl.push_back({len, SliceRec{hi, j, e - j}});
+                            j = e;
+                        }
+                        R.slice_kept = std::max(R.slice_kept, kept);
+                        continue;
+                    }
+                    for (uint64_t g = h.joff; g < h.joff + h.d; g++)
+                        if (ranges[g] >> kRangeShift) rows.push_back(g);
+                }
+                std::stable_sort(sl.begin(), sl.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
+                r.s0 = (uint32_t)slices.size();
+                for (auto &x : sl) slices.push_back(x.second);
+                r.s1 = (uint32_t)slices.size();
                 r.er1 = rows.size();
             }
+            R.all_sliced = rows.empty();
+            if (!slices.empty()) R.slices = dev_upload(slices);
             if (!rows.empty()) R.enc_rows = dev_upload(rows);
             R.hub_range = dev_upload(ranges);
         }
@@ -419,6 +458,13 @@ static bool hub_donates(const Plan &p, const beep_opts &o, const DevRoots &R)
     return o.donate && R.nhubs && p.L >= 4 && !(p.L == 4 && tail_summed(p, o.emit));
 }
 
+// Count-only runs whose count follows from |C_2| of the kept rows (whole rows:
+// no bound on x_2), with every hub in slices: the slices count pairs per item.
+static bool hub_counted(const KPlan &kp, const DevRoots &R)
+{
+    return kp.closed && !kp.hits && !(kp.smask[2] & 2u) && R.all_sliced;
+}
+
 static int hub_grid_of(const DevRoots &R, int nlev, bool pair, int cus)
 {
     return hub_dfs_occupancy(nlev, std::max<uint32_t>(R.wmax, 1), pair) * cus;
@@ -428,24 +474,26 @@ ScratchNeeds scratch_needs(const Prep &pp, const Plan &p, const beep_opts &o, in
 {
     const DevRoots &R = pp.dev->roots;
     ScratchNeeds n;
+    // (counted hubs keep their item counters where the bitmaps would be; the
+    // sizes do not depend on which kernels a run takes)
     if (R.nhubs && pp.uses_bitmap) {
         n.arena_words = R.arena_words;
         n.hash_slots = R.arena_slots;
     }
     const int nlev = p.L > 3 ? p.L - 3 : 1;
-    const bool pair5 = hub_pair5(p.L, pair_summed(p, o.emit), std::max<uint32_t>(R.wmax, 1));
-    if (R.nhubs && !pair5) {
+    if (R.nhubs) {
         // per wave: nlev stack rows + the row of x_1 (used when they do not fit LDS)
-        n.stk_words = (uint64_t)hub_grid_of(R, nlev, pair_summed(p, o.emit), cus) * (kBlock / 64) *
-                      hub_wave_words(nlev, std::max<uint32_t>(R.wmax, 1), pair_summed(p, o.emit));
+        const uint32_t wmax = std::max<uint32_t>(R.wmax, 1);
+        n.stk_words = (uint64_t)hub_stack_occupancy(nlev, wmax, pair_summed(p, o.emit)) * cus * (kBlock / 64) *
+                      hub_wave_words(nlev, wmax, false);
     }
     if (hub_donates(p, o, R)) {
-        // records: as many as chunks of 16 x_2 can give; up to 2^18 (6 MB) as
-        // many as single x_2 can.  An item that finds the ring full is walked.
-        n.queue_cap = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 22, R.don_records));
-        n.queue_cap = std::max(n.queue_cap, std::min<uint64_t>(1ull << 18, R.don_fine));
-        // (records of paired items hold no candidate set)
-        n.slot_cap = pair5 ? 1 : std::max<uint64_t>(1, std::min<uint64_t>(1ull << 26, R.don_words));
+        // records: as many as chunks of 16 x_2 can give; where there is room for
+        // them, up to 2^18 (6 MB) as many as single x_2 can.  An item that finds
+        // the ring full is walked.
+        n.queue_min = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 22, R.don_records));
+        n.queue_cap = std::max(n.queue_min, std::min<uint64_t>(1ull << 18, R.don_fine));
+        n.slot_cap = std::max<uint64_t>(1, std::min<uint64_t>(1ull << 26, R.don_words));
     }
     if (o.emit == BEEP_EMIT_BUFFER && o.match_cap) n.dbuf_words = o.match_cap * (uint64_t)p.L;
     if (o.profile) n.prof_words = (uint64_t)kProfPhases * kProfSlots;
@@ -598,15 +646,33 @@ void enqueue_hubs(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStrea
         const HubRound &r = R.rounds[ri];
         const uint64_t rows = r.g1 - r.g0;
         if (pp.uses_bitmap) {
-            HIP_CHECK(launch_fill_zero(s.arena, r.ewords * 8, st, c.out.dl));
-            HIP_CHECK(launch_fill_zero(s.kv, r.hslots * 8, st, c.out.dl));
-            int g1 = (int)std::min<uint64_t>((rows + kBlock - 1) / kBlock, (uint64_t)cus * 16);
-            HIP_CHECK(launch_hub_hash(std::max(g1, 1), st, c.kg, R.hubs, R.hub_of_row, r.g0, r.g1, s.kv, c.out.dl));
-            const uint64_t nenc = r.er1 - r.er0;
-            int g2 = (int)std::min<uint64_t>((nenc + 255) / 256, (uint64_t)cus * 16);
-            if (nenc)
+            const uint64_t nenc = r.er1 - r.er0, items = r.i1 - r.i0;
+            auto slices = [&](uint32_t *c2) {
+                if (r.s1 > r.s0)
+                    HIP_CHECK(launch_hub_slices(st, c.kg, R.hubs, R.slices + r.s0, r.s1 - r.s0, R.hub_range,
+                                                R.slice_kept, c.kp.bin_ratio, s.arena, c2, r.i0, c.out));
+            };
+            if (hub_counted(c.kp, R)) {
+                if (items == 0) continue;
+                HIP_CHECK(launch_fill_zero(s.arena, items * 4, st, c.out.dl));
+                slices((uint32_t *)s.arena);
+                const int g4 = (int)std::min<uint64_t>((items + kBlock - 1) / kBlock, (uint64_t)cus * 4);
+                HIP_CHECK(launch_hub_closed(g4, st, R.hubs, R.hub_of_item, r.i0, r.i1, (uint32_t *)s.arena,
+                                            c.kp.closed, c.out));
+                continue;
+            }
+            if (!c.kp.hits) HIP_CHECK(launch_fill_zero(s.arena, r.ewords * 8, st, c.out.dl));
+            if (nenc) {
+                HIP_CHECK(launch_fill_zero(s.kv, r.hslots * 8, st, c.out.dl));
+                int g1 = (int)std::min<uint64_t>((rows + kBlock - 1) / kBlock, (uint64_t)cus * 16);
+                HIP_CHECK(launch_hub_hash(std::max(g1, 1), st, c.kg, R.hubs, R.hub_of_row, r.g0, r.g1, s.kv, c.out.dl));
+                int g2 = (int)std::min<uint64_t>((nenc + 255) / 256, (uint64_t)cus * 16);
                 HIP_CHECK(launch_hub_encode(std::max(g2, 1), st, c.kg, R.hubs, R.hub_of_row, R.hub_range,
-                                            R.enc_rows + r.er0, nenc, s.kv, s.arena, c.kp.upper, c.out));
+                                            R.enc_rows + r.er0, nenc, s.kv, s.arena, c.kp.upper,
+                                            c.kp.hits ? c.kp.closed : 0, c.out));
+            }
+            if (c.kp.hits) continue;  // the pairs found are the count
+            slices(nullptr);
         }
         unsigned long long *cur = s.ctr + kCtrHub + (uint64_t)(ri % 64) * kCurWords;
         if (ri >= 64) HIP_CHECK(launch_fill_zero(cur, kCurWords * 8, st));

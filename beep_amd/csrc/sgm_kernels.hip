@@ -301,7 +301,7 @@ __device__ __forceinline__ void emit_word(const KOut &out, const KPlan &pl, int 
 // Context of a row of an LDS batch that has build units (see find_pairs):
 // streamed rows: unit e is ocol[base + e]; looked-up rows: unit e looks the row
 // entry aoff + e up in the range whose hbeg | hlen << kRangeShift is `base`.
-struct RowCtx {
+struct alignas(16) RowCtx {
     uint64_t base;
     uint32_t aoff;
     uint32_t info;  // row (9 bits) | looked up << 9 | filter word << 10 (10) | filter bits' log2 << 20
@@ -856,28 +856,213 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
 // full-rate multiply; the 32-bit one runs at a quarter of the rate).
 __device__ __forceinline__ uint32_t lds_hash(uint32_t v) { return __umul24(v, 0x9E3779u); }
 
-// Stages a batch -- its roots, row vertices and each row's root -- and builds
-// the roots' bitmaps (or counts their pairs, KPlan::hits).  Returns the number
-// of rows.
+// Table of 2^lh slots (key + 1, value) with a filter of 16 bits per slot.
+__device__ __forceinline__ void table_add(uint32_t *key, uint16_t *val, uint32_t *flt, uint32_t lh, uint32_t vx,
+                                          uint32_t value)
+{
+    const uint32_t h = lds_hash(vx), mask = (1u << lh) - 1u;
+    uint32_t s = h >> (32u - lh);
+    while (atomicCAS(&key[s], 0u, vx + 1u) != 0u) s = (s + 1) & mask;
+    val[s] = (uint16_t)value;
+    const uint32_t fb = h >> (28u - lh);
+    atomicOr(&flt[fb >> 5], 1u << (fb & 31u));
+}
+
+__device__ __forceinline__ bool table_find(const uint32_t *key, const uint16_t *val, uint32_t lh, uint32_t vx,
+                                           uint32_t &value)
+{
+    const uint32_t mask = (1u << lh) - 1u;
+    uint32_t s = lds_hash(vx) >> (32u - lh);
+    bool hit;
+    for (;;) {  // one exit: two of them cost the wave a third of the search's time
+        const uint32_t k = key[s];
+        hit = k == vx + 1u;
+        if (hit || k == 0u) break;
+        s = (s + 1) & mask;
+    }
+    if (hit) value = val[s];
+    return hit;
+}
+
+// Whether w is in v's larger-key range, by the range's table past w's first slot.
+__device__ __forceinline__ bool later_slot(const KGraph &g, uint32_t v, uint32_t w)
+{
+    const VInfo vi = g.vinfo[v];
+    const uint32_t size = 2 * vi.hlen;
+    const uint32_t *t = g.htab + 2 * vi.hbeg;
+    uint32_t s = lookup_slot(w, size);
+    bool hit;
+    for (;;) {
+        s = s + 1 == size ? 0 : s + 1;
+        const uint32_t x = t[s];
+        hit = x == w + 1u;
+        if (hit || x == 0u) break;
+    }
+    return hit;
+}
+
+// LDS of the pair search: row contexts, row-start marks, the waves' queues, the
+// filters and the vertices that looked-up units name.
+struct UnitView {
+    RowCtx *ctx;
+    uint64_t *mark, *q;
+    const uint32_t *flt, *A, *key;
+};
+
+// Finds adjacent pairs (v, w), key(v) < key(w), from v, for up to N * kBlock
+// rows (thread t has rows t, t + kBlock, ...; un[q] units and context cx[q]
+// each, base and aoff relative to the row's first unit).  A row's work units
+// are the entries of v's larger-key range, each tested against a table of
+// wanted vertices, or, where that range is longer than kLookupRatio times the
+// vertices it can pair with, those vertices, each looked up in the range's
+// table.  settle(lo, info) is called for units that are probably a pair, 64 a
+// wave at a time: info is the row's, lo the entry, or for looked-up units the
+// index of the wanted vertex with bit 31 set when its first slot held it.
 //
-// Each adjacent pair (v, w) of a root's row, key(v) < key(w), is found from v.
-// Row v's work units are the entries of v's larger-key range, each tested
-// against the root's row, or, where that range is longer than kLookupRatio
-// times the entries v can pair with, those entries, each looked up in the
-// range's table.  What bounds it is instruction issue (a wave64 VALU
-// instruction takes a SIMD four cycles), so the units cost as few as possible:
+// What bounds it is instruction issue (a wave64 VALU instruction takes a SIMD
+// four cycles), so a unit costs as little as possible:
 //  * all rows' units are numbered through and a wave takes 64 consecutive ones,
 //    one a lane.  A unit's row is the number of row starts at or before it,
 //    one 64-bit mark word and one count per 64 units and a mask-and-count per
 //    lane; the row's context is one 16-byte LDS read;
-//  * a streamed entry is first tested against a filter of 16 to 32 bits per row
-//    entry.  The few per cent that pass (and the looked-up slots that are taken)
-//    go to a queue per wave, which is worked off 64 at a time: the exact probe
-//    and the bit setting run with full waves;
+//  * a streamed entry is first tested against a filter of 16 to 32 bits per
+//    wanted vertex.  The few per cent that pass (and the looked-up slots that
+//    are taken) go to a queue per wave, so the exact probe and what a pair does
+//    run with full waves;
 //  * four loads a lane are in flight.
 // Before, each thread took 8 consecutive units and reloaded the row's context
 // wherever one of 64 lanes crossed into another row, and every lane waited for
-// the longest probe: 216 lane instructions per unit (4-clique, 1.1M vertices).
+// the longest probe: 216 lane instructions per unit (4-clique on 1.1M vertices,
+// 362 us; now 257 us).
+//  * where a pair only counts (`count`), those that a first slot settles -- most
+//    -- are counted on the spot and never queued.
+template <int N, class Settle>
+__device__ __forceinline__ void find_pairs(const KGraph &g, const UnitView &u, const uint32_t (&un)[N],
+                                           RowCtx (&cx)[N], uint32_t rows, bool count, uint64_t &cnt, Settle &&settle)
+{
+    uint32_t counted = 0;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    uint32_t at[N];
+    uint64_t act[N];
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        at[r] = 0;
+        act[r] = 0;
+        if ((uint32_t)r * kBlock >= rows) continue;
+        at[r] = wave_incl_scan(un[r]);
+        act[r] = __ballot(un[r] != 0);
+        if (lane == 63)
+            u.mark[16 + r * (kBlock / 64) + wv] = (uint64_t)at[r] | (uint64_t)__popcll(act[r]) << 32;
+    }
+    __syncthreads();
+    uint32_t total = 0, nrows = 0;  // units; rows that have any
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        if ((uint32_t)r * kBlock >= rows) continue;
+        uint32_t ub = total, rb = nrows;
+        for (int w = 0; w < kBlock / 64; w++) {
+            const uint64_t t = u.mark[16 + r * (kBlock / 64) + w];
+            if (w < wv) {
+                ub += (uint32_t)t;
+                rb += (uint32_t)(t >> 32);
+            }
+            total += (uint32_t)t;
+            nrows += (uint32_t)(t >> 32);
+        }
+        at[r] = ub + at[r] - un[r];  // the row's first unit
+        if (un[r]) {
+            cx[r].aoff -= at[r];
+            if (!((cx[r].info >> 9) & 1u)) cx[r].base -= at[r];
+            u.ctx[rb + bits_below(act[r])] = cx[r];
+        }
+    }
+    uint64_t *q = u.q + wv * kQueue;
+    auto flush = [&](uint32_t from, uint32_t n) {
+        wave_lds_sync();
+        if ((uint32_t)lane < n) settle((uint32_t)q[from + lane], (uint32_t)(q[from + lane] >> 32));
+        wave_lds_sync();
+    };
+    constexpr int kUnroll = 4;
+    uint32_t k_done = 0, qn = 0;  // rows started before the tile; queued units
+    for (uint32_t t0 = 0; t0 < total; t0 += kTile) {
+        __syncthreads();
+        if (tid < (int)(kTile / 64)) u.mark[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+            const uint32_t o = at[r] - t0;
+            if (un[r] && o < kTile) atomicOr((unsigned long long *)&u.mark[o >> 6], 1ull << (o & 63u));
+        }
+        __syncthreads();
+        const uint64_t mw = u.mark[lane];
+        const uint32_t pc = (uint32_t)__popcll(mw), ic = wave_incl_scan(pc);
+        const uint32_t k0 = k_done + ic - pc;
+        k_done += lane_u32(ic, 63);
+        const uint32_t nseg = total - t0 < kTile ? (total - t0 + 63u) >> 6 : kTile / 64;
+        for (uint32_t s0 = wv; s0 < nseg; s0 += kUnroll * (kBlock / 64)) {
+            uint32_t val[kUnroll], aux[kUnroll], info[kUnroll];
+#pragma unroll
+            for (int i = 0; i < kUnroll; i++) {
+                const uint32_t s = s0 + i * (kBlock / 64);
+                val[i] = aux[i] = info[i] = 0;
+                if (s >= nseg) continue;
+                const uint32_t m0 = lane_u32((uint32_t)mw, s), m1 = lane_u32((uint32_t)(mw >> 32), s);
+                const uint64_t m = (uint64_t)m1 << 32 | m0;
+                const uint32_t k = lane_u32(k0, s) + (m0 & 1u) - 1u + bits_below(m >> 1);
+                const uint32_t e = t0 + s * 64 + lane;
+                if (e >= total) continue;
+                const RowCtx c = u.ctx[k];
+                info[i] = c.info;
+                if ((c.info >> 9) & 1u) {
+                    const uint64_t hb = c.base & ((1ull << kRangeShift) - 1ull);
+                    aux[i] = c.aoff + e;
+                    val[i] = g.htab[2 * hb + lookup_slot(u.A[aux[i]], 2u * (uint32_t)(c.base >> kRangeShift))];
+                } else {
+                    val[i] = g.ocol[c.base + e];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kUnroll; i++) {
+                const uint32_t s = s0 + i * (kBlock / 64);
+                if (s >= nseg) break;
+                const uint32_t e = t0 + s * 64 + lane;
+                bool on = false;
+                uint32_t lo = val[i];
+                if (e < total) {
+                    if ((info[i] >> 9) & 1u) {
+                        on = val[i] != 0u;
+                        lo = aux[i] | (val[i] == u.A[aux[i]] + 1u ? 1u << 31 : 0u);
+                    } else {
+                        const uint32_t fb = lds_hash(val[i]) >> (32u - ((info[i] >> 20) & 31u));
+                        on = (u.flt[((info[i] >> 10) & 1023u) + (fb >> 5)] >> (fb & 31u)) & 1u;
+                    }
+                }
+                if (count && on) {
+                    const uint32_t lh = ((info[i] >> 20) & 31u) - 4u;
+                    const uint32_t slot = 2u * ((info[i] >> 10) & 1023u) + (lds_hash(val[i]) >> (32u - lh));
+                    const bool sure = (info[i] >> 9) & 1u ? (lo >> 31) != 0u : u.key[slot] == val[i] + 1u;
+                    counted += sure ? 1u : 0u;
+                    on = !sure;
+                }
+                const uint64_t m = __ballot(on);
+                if (on) q[qn + bits_below(m)] = (uint64_t)info[i] << 32 | lo;
+                qn += (uint32_t)__popcll(m);
+                if (qn >= 64u) {
+                    qn -= 64u;
+                    flush(qn, 64u);
+                }
+            }
+        }
+    }
+    if (qn) flush(0, qn);
+    cnt += counted;
+    __syncthreads();
+}
+
+// Stages a batch -- its roots, row vertices and each row's root -- and builds
+// the roots' bitmaps (or counts their pairs, KPlan::hits).  Returns the number
+// of rows.
+template <bool MAY_COUNT>
 __device__ uint32_t build_batch(const KGraph &g, const KPlan &pl, const LdsView &v, const RootRec *__restrict__ recs,
                                 uint32_t first, uint32_t nr, uint64_t &cnt)
 {
@@ -934,26 +1119,17 @@ __device__ uint32_t build_batch(const KGraph &g, const KPlan &pl, const LdsView 
 #pragma unroll
     for (int q = 0; q < kRowsPer; q++)
         if ((uint32_t)tid + (uint32_t)q * kBlock < sumd) rvi[q] = g.vinfo[rvx[q]];
-    uint32_t un[kRowsPer], inc[kRowsPer];
-    uint64_t act[kRowsPer];
+    uint32_t un[kRowsPer];
     RowCtx cx[kRowsPer];
 #pragma unroll
     for (int q = 0; q < kRowsPer; q++) {
         const uint32_t j = (uint32_t)tid + (uint32_t)q * kBlock;
-        un[q] = inc[q] = 0;
-        act[q] = 0;
-        if ((uint32_t)q * kBlock >= sumd) continue;
+        un[q] = 0;
         if (j < sumd) {
             const RootRec rr = v.sRoot[rro[q]];
             const uint32_t jl = j - rr.doff, vx = rvx[q], lh = lds_hash_log2(rr.d);
-            const uint32_t H = 1u << lh, h = lds_hash(vx);
-            if (!pl.kept || jl >= rr.split) {  // only kept entries are looked for
-                uint32_t s = h >> (32u - lh);
-                while (atomicCAS(&v.sHKey[rr.hoff + s], 0u, vx + 1u) != 0u) s = (s + 1) & (H - 1);
-                v.sHVal[rr.hoff + s] = (uint16_t)jl;
-                const uint32_t fb = h >> (28u - lh);  // 16 H filter bits
-                atomicOr(&v.sFlt[(rr.hoff >> 1) + (fb >> 5)], 1u << (fb & 31u));
-            }
+            // only kept entries are looked for
+            if (!pl.kept || jl >= rr.split) table_add(v.sHKey + rr.hoff, v.sHVal + rr.hoff, v.sFlt + (rr.hoff >> 1), lh, vx, jl);
             // x_1..x_{L-1} are distinct row entries: shorter rows hold no tuple
             const uint32_t c = rr.d + 1u < (uint32_t)pl.L
                                    ? 0u : pair_partners(jl, rr.d, rr.split, g.asc, pl.kept, pl.upper);
@@ -966,150 +1142,26 @@ __device__ uint32_t build_batch(const KGraph &g, const KPlan &pl, const LdsView 
                 cx[q].info = j | (look ? 1u << 9 : 0u) | (rr.hoff >> 1) << 10 | (lh + 4u) << 20;
             }
         }
-        inc[q] = wave_incl_scan(un[q]);
-        act[q] = __ballot(un[q] != 0);
-        if (lane == 63) {
-            v.sMark[16 + q * (kBlock / 64) + wv] = (uint64_t)inc[q] | (uint64_t)__popcll(act[q]) << 32;
-        }
     }
-    __syncthreads();
-    uint32_t total = 0, rows_before = 0;
-#pragma unroll
-    for (int q = 0; q < kRowsPer; q++) {
-        if ((uint32_t)q * kBlock >= sumd) continue;
-        uint32_t ub = total, rb = rows_before;
-        for (int w = 0; w < kBlock / 64; w++) {
-            const uint64_t t = v.sMark[16 + q * (kBlock / 64) + w];
-            if (w < wv) {
-                ub += (uint32_t)t;
-                rb += (uint32_t)(t >> 32);
-            }
-            total += (uint32_t)t;
-            rows_before += (uint32_t)(t >> 32);
+    const UnitView uv{v.sCtx, v.sMark, v.sQ, v.sFlt, v.sA, v.sHKey};
+    find_pairs(g, uv, un, cx, sumd, MAY_COUNT && pl.hits && pl.closed == kClosedC, cnt, [&](uint32_t lo, uint32_t info) {
+        const uint32_t j = info & 511u;
+        const RootRec rr = v.sRoot[v.sJRoot[j]];
+        const uint32_t jl = j - rr.doff;
+        uint32_t i = 0;
+        bool hit;
+        if ((info >> 9) & 1u) {
+            const uint32_t p = lo & 0x7fffffffu;
+            i = p - rr.doff;
+            hit = (lo >> 31) || later_slot(g, v.sA[j], v.sA[p]);
+        } else {
+            hit = table_find(v.sHKey + rr.hoff, v.sHVal + rr.hoff, ((info >> 20) & 31u) - 4u, lo, i);
         }
-        if (un[q]) {
-            const uint32_t start = ub + inc[q] - un[q];
-            cx[q].aoff -= start;
-            if (!((cx[q].info >> 9) & 1u)) cx[q].base -= start;
-            v.sCtx[rb + bits_below(act[q])] = cx[q];
+        if (hit) {
+            if (MAY_COUNT && pl.hits) cnt += pl.closed == kClosedRow ? rr.d - 2u : 1u;
+            else set_pair(v.sE + rr.eoff, (rr.d + 63) >> 6, jl, i, pl.upper);
         }
-        inc[q] = ub + inc[q] - un[q];  // the row's first unit
-    }
-
-    // exact probe of 64 queued units (lanes below n), and what a pair does
-    uint64_t *q = v.sQ + wv * kQueue;
-    auto settle = [&](uint32_t from, uint32_t n) {
-        wave_lds_sync();
-        if ((uint32_t)lane < n) {
-            const uint64_t ent = q[from + lane];
-            const uint32_t lo = (uint32_t)ent, info = (uint32_t)(ent >> 32);
-            const uint32_t j = info & 511u;
-            const RootRec rr = v.sRoot[v.sJRoot[j]];
-            const uint32_t jl = j - rr.doff;
-            uint32_t i = 0;
-            bool hit = false;
-            if ((info >> 9) & 1u) {  // looked up: lo = the partner's row, top bit = found in its first slot
-                const uint32_t p = lo & 0x7fffffffu;
-                i = p - rr.doff;
-                hit = (lo >> 31) != 0;
-                if (!hit) {
-                    const VInfo vi = g.vinfo[v.sA[j]];
-                    const uint32_t a = v.sA[p] + 1u, size = 2 * vi.hlen;
-                    const uint32_t *t = g.htab + 2 * vi.hbeg;
-                    uint32_t s = lookup_slot(a - 1u, size);
-                    for (;;) {
-                        s = s + 1 == size ? 0 : s + 1;
-                        const uint32_t x = t[s];
-                        hit = x == a;
-                        if (hit || x == 0u) break;
-                    }
-                }
-            } else {
-                const uint32_t lh = ((info >> 20) & 31u) - 4u, mask = (1u << lh) - 1u;
-                uint32_t s = lds_hash(lo) >> (32u - lh);
-                for (;;) {
-                    const uint32_t key = v.sHKey[rr.hoff + s];
-                    hit = key == lo + 1u;
-                    if (hit || key == 0u) break;
-                    s = (s + 1) & mask;
-                }
-                if (hit) i = v.sHVal[rr.hoff + s];
-            }
-            if (hit) {
-                if (pl.hits) cnt += pl.closed == kClosedRow ? rr.d - 2u : 1u;
-                else set_pair(v.sE + rr.eoff, (rr.d + 63) >> 6, jl, i, pl.upper);
-            }
-        }
-        wave_lds_sync();
-    };
-
-    constexpr int kUnroll = 4;
-    uint32_t k_done = 0, qn = 0;  // rows started before the tile; queued units
-    for (uint32_t t0 = 0; t0 < total; t0 += kTile) {
-        __syncthreads();
-        if (tid < (int)(kTile / 64)) v.sMark[tid] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kRowsPer; r++) {
-            const uint32_t at = inc[r] - t0;
-            if (un[r] && at < kTile) atomicOr((unsigned long long *)&v.sMark[at >> 6], 1ull << (at & 63u));
-        }
-        __syncthreads();
-        const uint64_t mw = v.sMark[lane];
-        const uint32_t pc = (uint32_t)__popcll(mw), ic = wave_incl_scan(pc);
-        const uint32_t k0 = k_done + ic - pc;
-        k_done += lane_u32(ic, 63);
-        const uint32_t nseg = total - t0 < kTile ? (total - t0 + 63u) >> 6 : kTile / 64;
-        for (uint32_t s0 = wv; s0 < nseg; s0 += kUnroll * (kBlock / 64)) {
-            uint32_t val[kUnroll], aux[kUnroll], info[kUnroll];
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const uint32_t s = s0 + u * (kBlock / 64);
-                val[u] = aux[u] = info[u] = 0;
-                if (s >= nseg) continue;
-                const uint32_t m0 = lane_u32((uint32_t)mw, s), m1 = lane_u32((uint32_t)(mw >> 32), s);
-                const uint64_t m = (uint64_t)m1 << 32 | m0;
-                const uint32_t k = lane_u32(k0, s) + (m0 & 1u) - 1u + bits_below(m >> 1);
-                const uint32_t e = t0 + s * 64 + lane;
-                if (e >= total) continue;
-                const RowCtx cxt = v.sCtx[k];
-                info[u] = cxt.info;
-                if ((cxt.info >> 9) & 1u) {
-                    const uint64_t hb = cxt.base & ((1ull << kRangeShift) - 1ull);
-                    aux[u] = cxt.aoff + e;
-                    val[u] = g.htab[2 * hb + lookup_slot(v.sA[aux[u]], 2u * (uint32_t)(cxt.base >> kRangeShift))];
-                } else {
-                    val[u] = g.ocol[cxt.base + e];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const uint32_t s = s0 + u * (kBlock / 64);
-                if (s >= nseg) break;
-                const uint32_t e = t0 + s * 64 + lane;
-                bool on = false;
-                uint32_t lo = val[u];
-                if (e < total) {
-                    if ((info[u] >> 9) & 1u) {
-                        on = val[u] != 0u;
-                        lo = aux[u] | (val[u] == v.sA[aux[u]] + 1u ? 1u << 31 : 0u);
-                    } else {
-                        const uint32_t fb = lds_hash(val[u]) >> (32u - ((info[u] >> 20) & 31u));
-                        on = (v.sFlt[((info[u] >> 10) & 1023u) + (fb >> 5)] >> (fb & 31u)) & 1u;
-                    }
-                }
-                const uint64_t m = __ballot(on);
-                if (on) q[qn + bits_below(m)] = (uint64_t)info[u] << 32 | lo;
-                qn += (uint32_t)__popcll(m);
-                if (qn >= 64u) {
-                    qn -= 64u;
-                    settle(qn, 64u);
-                }
-            }
-        }
-    }
-    if (qn) settle(0, qn);
-    __syncthreads();
+    });
     return sumd;
 }
 
@@ -1125,7 +1177,8 @@ __device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v
 {
     const int tid = threadIdx.x;
     const uint64_t t_build = wall_clock64();
-    const uint32_t sumd = build_batch(g, pl, v, recs, first, nr, cnt);
+    constexpr bool kMayCount = WALK == kWalkAny || WALK == kWalkNone;
+    const uint32_t sumd = build_batch<kMayCount>(g, pl, v, recs, first, nr, cnt);
     if (tid == 0) prof_add(out, 3, blockIdx.x, t_build);  // staging + bitmap build
 
     if (pl.hits) return;  // the pairs found are the count
@@ -1262,7 +1315,7 @@ __global__ __launch_bounds__(kBlock) void hub_encode_kernel(KGraph g, const HubR
                                                             const uint64_t *__restrict__ hub_range,
                                                             const uint64_t *__restrict__ rows, uint64_t nrows,
                                                             const uint64_t *__restrict__ kv,
-                                                            uint64_t *E, int upper, KOut out)
+                                                            uint64_t *E, int upper, int count, KOut out)
 {
     __shared__ uint64_t sBeg[kBlock];
     __shared__ uint32_t sPre[kBlock];
@@ -1272,6 +1325,8 @@ __global__ __launch_bounds__(kBlock) void hub_encode_kernel(KGraph g, const HubR
     const uint64_t nchunks = (nrows + 63) / 64;
     const uint64_t wstride = (uint64_t)gridDim.x * (kBlock / 64);
     const uint64_t dl = *out.dl;
+    const uint64_t t_start = wall_clock64();
+    uint64_t cnt = 0;  // count: KPlan::closed of a plan whose pairs are counted, no bitmap (KPlan::hits)
     for (uint64_t c = blockIdx.x * (uint64_t)(kBlock / 64) + wv; c < nchunks; c += wstride) {
         if (past(dl)) {  // the bitmap stays incomplete; the DFS that follows stops at once
             if (lane == 0) mark_stop(out);
@@ -1360,6 +1415,10 @@ __global__ __launch_bounds__(kBlock) void hub_encode_kernel(KGraph g, const HubR
                     if (key == 0u) break;
                     if (key == wv2 + 1u) {
                         const uint32_t i = (uint32_t)(slot >> 32);
+                        if (count) {
+                            cnt += count == kClosedRow ? h.d - 2u : 1u;
+                            break;
+                        }
                         // upper plans keep the bit in the row of the smaller index only
                         const bool fwd = !upper || i > jl, mir = !upper || jl > i;
                         if (fwd && jl >= h.rlo)
@@ -1377,6 +1436,159 @@ __global__ __launch_bounds__(kBlock) void hub_encode_kernel(KGraph g, const HubR
         }
         __builtin_amdgcn_wave_barrier();
     }
+    if (count) {
+        flush_acc(out, cnt, 0, 0);
+        if (lane == 0) prof_add(out, 1, blockIdx.x * (kBlock / 64) + wv, t_start);
+    }
+}
+
+// Slices of hubs with few kept rows (K <= kSliceKept): a workgroup takes up to
+// kSliceRows consecutive row vertices of a hub, holds the kept vertices' table
+// in LDS and finds the slice's pairs as the LDS batches do (find_pairs).  Every
+// pair has a kept endpoint.
+//   CLOSED: the plan's count follows from |C_2| of each kept x_1 (KPlan::closed):
+//     the pairs are counted per kept row, in LDS, and added to c2 (one counter
+//     per hub item, cleared before) at the end.  No bitmap is built or read.
+//   else the kept rows' words of the slice's columns are built in LDS, 256
+//     columns at a time, and stored: the slice alone holds them, but for columns
+//     of kept rows, whose words also take the bits set from the kept row's own
+//     side (atomics, on zeroed words).
+// The grid-wide hub_encode_kernel probed a table in HBM and set bits by HBM
+// atomics, 64 bytes of write traffic each: diamond on 1.1M vertices 356 us alone
+// for 8.5 M entries.  Slices come heaviest first (listed so at upload).
+constexpr int kSliceWords = kBlock / 64;
+struct SliceLayout {
+    uint32_t oCtx, oQ, oMark, oKey, oFlt, oA, oE, oVal, bytes;
+};
+__host__ inline SliceLayout make_slice_layout(uint32_t kmax, bool closed)
+{
+    const uint32_t hs = lds_hash_slots(kmax);
+    SliceLayout L{};
+    uint32_t o = 0;
+    L.oE = o;    o += closed ? align_up(kmax * 4, 16) : kmax * kSliceWords * 8;
+    L.oCtx = o;  o += kBlock * (uint32_t)sizeof(RowCtx);
+    L.oQ = o;    o += (kBlock / 64) * kQueue * 8;
+    L.oMark = o; o += kTile / 8;
+    L.oKey = o;  o += hs * 4;
+    L.oFlt = o;  o += hs / 2 * 4;
+    L.oA = o;    o += kmax * 4;
+    L.oVal = o;  o += hs * 2;
+    L.bytes = align_up(o, 16);
+    return L;
+}
+
+template <bool CLOSED>
+__global__ __launch_bounds__(kBlock) void hub_slice_kernel(KGraph g, const HubRec *__restrict__ hubs,
+                                                           const SliceRec *__restrict__ slices,
+                                                           const uint64_t *__restrict__ hub_range,
+                                                           uint32_t bin_ratio, uint64_t *E, uint32_t *c2, uint64_t i0,
+                                                           SliceLayout lay, KOut out)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    uint64_t *sE = (uint64_t *)(smem + lay.oE);
+    uint32_t *sCnt = (uint32_t *)(smem + lay.oE);
+    uint32_t *sKey = (uint32_t *)(smem + lay.oKey), *sFlt = (uint32_t *)(smem + lay.oFlt);
+    uint32_t *sA = (uint32_t *)(smem + lay.oA);
+    uint16_t *sVal = (uint16_t *)(smem + lay.oVal);
+    const UnitView uv{(RowCtx *)(smem + lay.oCtx), (uint64_t *)(smem + lay.oMark), (uint64_t *)(smem + lay.oQ), sFlt,
+                      sA, sKey};
+    const int tid = threadIdx.x;
+    if (past(*out.dl)) {  // what follows stops at once
+        if (tid == 0) mark_stop(out);
+        return;
+    }
+    const uint64_t t_start = wall_clock64();
+    const SliceRec sl = slices[blockIdx.x];
+    const HubRec h = hubs[sl.hub];
+    const uint32_t d = h.d, rlo = h.rlo, K = d - rlo, W = (d + 63) >> 6, lh = lds_hash_log2(K);
+    for (uint32_t i = tid; i < (1u << lh); i += kBlock) sKey[i] = 0;
+    for (uint32_t i = tid; i < (1u << lh) / 2; i += kBlock) sFlt[i] = 0;
+    if (CLOSED)
+        for (uint32_t i = tid; i < K; i += kBlock) sCnt[i] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < K; i += kBlock) {
+        const uint32_t v = g.ocol[h.rbeg + rlo + i];
+        sA[i] = v;
+        table_add(sKey, sVal, sFlt, lh, v, i);
+    }
+    for (uint32_t r0 = sl.row0; r0 < sl.row0 + sl.rows; r0 += kBlock) {
+        const uint32_t rows = sl.row0 + sl.rows - r0 < (uint32_t)kBlock ? sl.row0 + sl.rows - r0 : (uint32_t)kBlock;
+        if (!CLOSED)
+            for (uint32_t i = tid; i < K * kSliceWords; i += kBlock) sE[i] = 0;
+        uint32_t un[1] = {0};
+        RowCtx cx[1];
+        if (tid < (int)rows) {
+            const uint32_t j = r0 + tid;
+            const uint64_t rg = hub_range[h.joff + j];
+            const uint32_t len = (uint32_t)(rg >> kRangeShift);
+            const uint32_t c = j < rlo ? K : d - 1u - j;  // kept rows it can pair with
+            if (len && c) {
+                const bool look = (uint64_t)len > (uint64_t)c * bin_ratio;
+                un[0] = look ? c : len;
+                cx[0].base = rg & ((1ull << kRangeShift) - 1ull);
+                if (look) {
+                    const VInfo vi = g.vinfo[g.ocol[h.rbeg + j]];
+                    cx[0].base = vi.hbeg | ((uint64_t)vi.hlen << kRangeShift);
+                }
+                cx[0].aoff = K - c;
+                cx[0].info = (uint32_t)tid | (look ? 1u << 9 : 0u) | (lh + 4u) << 20;
+            }
+        }
+        __syncthreads();
+        uint64_t none = 0;
+        find_pairs(g, uv, un, cx, rows, false, none, [&](uint32_t lo, uint32_t info) {
+            const uint32_t row = info & 511u, j = r0 + row;
+            uint32_t i = 0;
+            bool hit;
+            if ((info >> 9) & 1u) {
+                i = lo & 0x7fffffffu;
+                hit = (lo >> 31) || later_slot(g, g.ocol[h.rbeg + j], sA[i]);
+            } else {
+                hit = table_find(sKey, sVal, lh, lo, i);
+            }
+            if (!hit) return;
+            if (CLOSED) {
+                atomicAdd(&sCnt[i], 1u);
+                if (j >= rlo) atomicAdd(&sCnt[j - rlo], 1u);
+            } else {
+                atomicOr((unsigned long long *)&sE[i * kSliceWords + (row >> 6)], 1ull << (row & 63u));
+                if (j >= rlo) {
+                    const uint32_t ci = i + rlo;
+                    atomicOr((unsigned long long *)&E[h.eoff + (uint64_t)(j - rlo) * W + (ci >> 6)], 1ull << (ci & 63u));
+                }
+            }
+        });
+        if (!CLOSED) {
+            const uint32_t w0 = r0 >> 6, nw = (rows + 63u) >> 6;
+            for (uint32_t x = tid; x < K * kSliceWords; x += kBlock) {
+                const uint32_t w = x % kSliceWords;
+                if (w >= nw) continue;
+                uint64_t *to = &E[h.eoff + (uint64_t)(x / kSliceWords) * W + w0 + w];
+                const uint64_t val = sE[x];
+                if (w0 + w < (rlo >> 6)) *to = val;
+                else if (val) atomicOr((unsigned long long *)to, val);
+            }
+            __syncthreads();
+        }
+    }
+    if (CLOSED)
+        for (uint32_t i = tid; i < K; i += kBlock)
+            if (sCnt[i]) atomicAdd(&c2[h.ioff - i0 + i], sCnt[i]);
+    if (tid == 0) prof_add(out, 1, blockIdx.x, t_start);
+}
+
+// Sums closed_count over the items' |C_2| counters.
+__global__ __launch_bounds__(kBlock) void hub_closed_kernel(const HubRec *__restrict__ hubs,
+                                                            const uint32_t *__restrict__ hub_of_item, uint64_t i0,
+                                                            uint64_t i1, const uint32_t *__restrict__ c2, int closed,
+                                                            KOut out)
+{
+    uint64_t cnt = 0;
+    for (uint64_t i = i0 + blockIdx.x * (uint64_t)kBlock + threadIdx.x; i < i1; i += (uint64_t)gridDim.x * kBlock) {
+        const uint32_t c = c2[i - i0];
+        if (c) cnt += closed_count(closed, c, hubs[hub_of_item[i]].d);
+    }
+    flush_acc(out, cnt, 0, 0);
 }
 
 // Copies a W-word row (HBM) into a wave's buffer, lane i taking words i,
@@ -2451,10 +2663,36 @@ hipError_t launch_hub_hash(int grid, hipStream_t st, const KGraph &g, const HubR
 
 hipError_t launch_hub_encode(int grid, hipStream_t st, const KGraph &g, const HubRec *hubs,
                              const uint32_t *hor, const uint64_t *hrange, const uint64_t *rows, uint64_t nrows,
-                             const uint64_t *kv, uint64_t *E, int upper, const KOut &out)
+                             const uint64_t *kv, uint64_t *E, int upper, int count, const KOut &out)
 {
     hipLaunchKernelGGL(hub_encode_kernel, dim3(grid), dim3(kBlock), 0, st, g, hubs, hor, hrange, rows, nrows, kv, E,
-                       upper, out);
+                       upper, count, out);
+    return hipGetLastError();
+}
+
+// c2 set: count the slices' pairs per item (CLOSED); else build bitmap words in E.
+hipError_t launch_hub_slices(hipStream_t st, const KGraph &g, const HubRec *hubs, const SliceRec *slices, uint32_t n,
+                             const uint64_t *hrange, uint32_t kmax, uint32_t bin_ratio, uint64_t *E, uint32_t *c2,
+                             uint64_t i0, const KOut &out)
+{
+    const SliceLayout lay = make_slice_layout(kmax, c2 != nullptr);
+    static LdsLaunchCache cache[2];
+    if (c2) {
+        (void)cache[1].get((const void *)hub_slice_kernel<true>, lay.bytes);
+        hipLaunchKernelGGL((hub_slice_kernel<true>), dim3(n), dim3(kBlock), lay.bytes, st, g, hubs, slices, hrange,
+                           bin_ratio, E, c2, i0, lay, out);
+    } else {
+        (void)cache[0].get((const void *)hub_slice_kernel<false>, lay.bytes);
+        hipLaunchKernelGGL((hub_slice_kernel<false>), dim3(n), dim3(kBlock), lay.bytes, st, g, hubs, slices, hrange,
+                           bin_ratio, E, c2, i0, lay, out);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_hub_closed(int grid, hipStream_t st, const HubRec *hubs, const uint32_t *hoi, uint64_t i0, uint64_t i1,
+                             const uint32_t *c2, int closed, const KOut &out)
+{
+    hipLaunchKernelGGL(hub_closed_kernel, dim3(grid), dim3(kBlock), 0, st, hubs, hoi, i0, i1, c2, closed, out);
     return hipGetLastError();
 }
 
@@ -2514,6 +2752,15 @@ int hub_dfs_occupancy(int nlev, uint32_t wmax, bool pair)
     const void *fn = hub_dfs_fn(nlev, wmax, pair);
     const bool in_lds = hub_dfs_in_lds(nlev, wmax, pair);
     return hub_dfs_cache(in_lds, pair).get(fn, in_lds ? hub_lds_bytes(nlev, wmax, pair) : 0);
+}
+
+// Workgroups per CU the HBM stacks are sized for: those of the DFS kernel with
+// the stack rows alone in LDS.
+int hub_stack_occupancy(int nlev, uint32_t wmax, bool pair)
+{
+    const size_t lds = hub_lds_bytes(nlev, wmax, false);
+    const bool in_lds = lds <= kHubLdsMax;
+    return hub_dfs_cache(in_lds, pair).get(hub_dfs_fn(nlev, wmax, pair), in_lds ? lds : 0);
 }
 
 }  // namespace beep

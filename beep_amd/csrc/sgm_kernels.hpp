@@ -169,6 +169,15 @@ struct HubRec {
     uint32_t rlo;    // first bitmap row kept (rows below are never read)
 };
 
+// Rows [row0, row0 + rows) of a hub's bitmap build, for hubs with at most
+// kSliceKept kept rows (of those that keep rows from the split on only, with
+// both bits of every pair): their vertices fit an LDS table.
+struct SliceRec {
+    uint32_t hub, row0, rows;
+};
+constexpr uint32_t kSliceKept = 1024, kSliceRows = 512;
+constexpr uint64_t kSliceUnits = 3072;
+
 // Donated level-2 subtree of a hub item: x_2 in C_2 n [lo, hi), with C_2
 // published at slots[slot, slot + W).
 struct HubChunk {

@@ -532,3 +532,42 @@ def test_paired_items_on_wide_hubs(core):
         o = O.Prepared(og, O.plan(s, d, mode)).count(want_hash=False)
         for donate in (True, False):
             assert pp.count(donate=donate)["count"] == o["count"]
+
+
+@pytest.mark.parametrize("kept,low", [(1, 512), (2, 640), (64, 1300), (257, 500), (257, 1300), (1024, 500), (1030, 500)])
+def test_hub_slices_kept_rows(kept, low):
+    """Hubs adjacent to `kept` vertices of larger key and `low` of smaller: the
+    slice build up to its largest table (1,024 kept rows) and the grid-wide
+    build past it, counting (diamond), with bitmaps (its hashed matches) and
+    counted pairs over all rows (tailed triangle)."""
+    rng = np.random.default_rng(kept * 7 + low)
+    hub = kept + low
+    leaves = hub + 9  # every kept vertex outgrows the hub by these; they form a cycle
+    c, x = np.divmod(np.arange(kept * 6), 6)[0], rng.integers(0, hub, kept * 6)
+    lf = hub + 1 + np.arange(leaves)
+    lo = kept + np.arange(low)  # so do the smaller ones: nothing is peeled
+    u = np.concatenate([np.arange(hub), c, np.repeat(np.arange(kept), leaves), lf, lo])
+    v = np.concatenate([np.full(hub, hub), x, np.tile(lf, kept), np.roll(lf, 1), np.roll(lo, 1)])
+    key = np.unique(np.concatenate([u, v])[np.r_[u != v, u != v]] * (1 << 32)
+                    + np.concatenate([v, u])[np.r_[u != v, u != v]])
+    g = B.Graph.from_edges(key >> 32, key & 0xFFFFFFFF)
+    og = oracle_graph(g)
+    for name, emit in (("diamond", B.EMIT_NONE), ("diamond", B.EMIT_HASH), ("tailed_triangle", B.EMIT_NONE)):
+        if emit and kept > 300:
+            continue
+        say("hub slices", kept, low, name, emit)
+        s, d = P.directed(P.read_mtx_edges(name))
+        full = B.Prepared(g, B.Plan.from_edges(s, d, B.SGM))
+        of = O.Prepared(og, O.plan(s, d, B.SGM))
+        roots = full.arrays()["roots"]
+        ranks = [i for i, r in enumerate(roots.tolist()) if r == hub]
+        assert ranks
+        pp = full.subset(ranks)
+        assert pp.arrays()["n_hub_roots"] == 1
+        pp.upload(0)
+        o = of.count_ranks(ranks, want_hash=emit != B.EMIT_NONE)
+        for build in (B.BUILD_AUTO, B.BUILD_SCAN, B.BUILD_SEARCH):
+            r = pp.count(emit=emit, build_mode=build)
+            assert r["count"] == o["count"]
+            if emit:
+                assert (r["hash_sum"], r["hash_xor"]) == (o["hash_sum"], o["hash_xor"])
