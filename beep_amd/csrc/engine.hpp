@@ -21,17 +21,21 @@ namespace beep {
 // Counter words of one launch sequence (u64), in 128-byte lines of kLine
 // words.  Read back after the run (kCtrWords): the kStripes accumulator
 // stripes (kCtrAcc; see KOut::acc), then one line with the donation tail,
-// slot tail and donated count, the deadlines of the hub and the LDS kernels
-// and the stop flag.  Cleared but not read back: striped work cursors
-// (kCurWords each) of the hub rounds (64), the donation drain and the LDS
-// lane classes (32).
+// slot tail and donated count, the deadlines of the hub and the LDS kernels,
+// the stop flag and the sequence's start and end times.  Cleared but not read
+// back: striped work cursors (kCurWords each) of the hub rounds (64), the
+// donation drain and the LDS lane classes (31), and the stamps (KOut::stamp),
+// whose maxima follow the read-back words in the host's record (kRecWords).
 constexpr int kCtrAcc = 0;
 constexpr int kCtrQTail = kStripes * kLine, kCtrSlot = kCtrQTail + 1, kCtrDonated = kCtrQTail + 2,
-              kCtrDeadline = kCtrQTail + 3, kCtrStop = kCtrQTail + 5;
+              kCtrDeadline = kCtrQTail + 3, kCtrStop = kCtrQTail + 5, kCtrT0 = kCtrQTail + 6,
+              kCtrTEnd = kCtrQTail + 7;
 constexpr int kCtrWords = (kStripes + 1) * kLine;
 constexpr int kCurWords = kStripes * kLine;
 constexpr int kCtrHub = kCtrWords, kCtrHead = kCtrHub + 64 * kCurWords, kCtrLds = kCtrHead + kCurWords,
-              kCtrTotal = kCtrLds + 32 * kCurWords;
+              kCtrStamp = kCtrLds + 31 * kCurWords, kCtrTotal = kCtrStamp + kCurWords;
+static_assert(kCurWords >= kStripes * kLine, "stamps fill a cursor's words");
+constexpr int kRecWords = kCtrWords + kStampWords;
 
 // HBM copy of a variant: oriented rows and per-vertex records.
 struct DevGraph {
@@ -107,15 +111,10 @@ struct Lane {
     int nside = 0;
     hipStream_t main = nullptr;
     hipStream_t side[kMaxSide] = {};
-    hipEvent_t ev[4] = {};  // start, hubs done, all done, counters copied
+    hipEvent_t fork = nullptr, done = nullptr;  // main: counters cleared; everything done
     hipEvent_t side_done[kMaxSide] = {};
-    // start and end of each LDS lane class's launch (recorded on its stream
-    // right before and after it) and its lane class
-    static constexpr int kMaxClasses = 32;
-    hipEvent_t cls_start[kMaxClasses] = {};
-    hipEvent_t cls_done[kMaxClasses] = {};
-    uint8_t cls_lg[kMaxClasses] = {};
-    int ncls = 0;
+    static constexpr int kMaxClasses = 31;
+    unsigned long long *rec = nullptr;  // the run's record (kRecWords), pinned
     void create(int device, int nside);
     ~Lane();
 };
@@ -165,20 +164,17 @@ ScratchNeeds scratch_needs(const Prep &pp, const Plan &p, const beep_opts &o, in
 // lds_deadline_ms < 0: the LDS kernels share o.deadline_ms
 LaunchCfg make_launch(const Prep &pp, const Plan &p, const beep_opts &o, const Scratch &s, int cus,
                       double lds_deadline_ms = -1.0);
-// clear counters + deadline, LDS classes on the side streams and hub rounds on
-// main, join, counters -> host_ctr; records lane.ev[0..3].
-void enqueue_query(const Prep &pp, const LaunchCfg &c, const Scratch &s, Lane &lane,
-                   unsigned long long *host_ctr);
+// clear counters + deadline, LDS classes and hub rounds on main and the side
+// streams, join, record -> lane.rec; records lane.done at the end.
+void enqueue_query(const Prep &pp, const LaunchCfg &c, const Scratch &s, Lane &lane);
+hipError_t launch_end_sequence(const unsigned long long *ctr, uint32_t n, uint32_t t_end, const unsigned long long *stamp,
+                               unsigned long long *rec, hipStream_t st);
 void enqueue_hubs(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStream_t st);
-// LDS lane classes, one launch each, round-robin over nst streams; with
-// cls_done, the end of class i's launch is recorded in cls_done[i] and its
-// lane class in cls_lg[i].  Returns the number of classes.
-int enqueue_lds_classes(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStream_t *streams, int nst,
-                        hipEvent_t *cls_done = nullptr, uint8_t *cls_lg = nullptr);
-// Device time of each lane class's launch (ms, by lane class) from a lane's
-// events, and of the whole LDS phase (ev[0] to the last class's end).
-void class_times(const Lane &lane, double *t_by_lg);
-double lds_phase_ms(const Lane &lane);
+// LDS lane classes, one launch each, on one stream.
+void enqueue_lds_classes(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStream_t st);
+// Device times of a run from its record (ms): t_enum_ms, t_hub_ms and t_lds_ms
+// from the first kernel's start, and each lane class's launch.
+void fill_times(const unsigned long long *rec, int device, beep_result &res);
 void fill_result(const beep_opts &o, const unsigned long long *acc, beep_result &res);
 // Balance figures from the busy-time accumulators (kProfPhases x kProfSlots).
 void fill_profile(const unsigned long long *prof, beep_result &res);

@@ -92,7 +92,7 @@ void count_noalloc(Prep &pp, const Plan &p, const beep_opts &o, void *stream, be
     unsigned long long acc[kCtrWords];
     const auto t0 = std::chrono::steady_clock::now();
     HIP_CHECK(launch_begin_sequence(s.ctr, kCtrTotal, kCtrDeadline, c.deadline_ticks, c.deadline_ticks_lds, st));
-    enqueue_lds_classes(pp, c, s, &st, 1);
+    enqueue_lds_classes(pp, c, s, st);
     enqueue_hubs(pp, c, s, st);
     HIP_CHECK(hipMemcpyAsync(acc, s.ctr, sizeof(unsigned long long) * kCtrWords, hipMemcpyDeviceToHost, st));
     HIP_CHECK(hipStreamSynchronize(st));

@@ -121,7 +121,6 @@ struct Server {
     };
     struct Slot {
         Lane lane;
-        unsigned long long *host_ctr = nullptr;
         bool busy = false;
         bool busy_pilot = false;  // its launch sequence is a pilot
         Job job;
@@ -241,11 +240,11 @@ void Server::launch(Slot &sl)
     if (j.piloting) {
         const beep_opts po = pilot_opts(j.opts);
         sl.c = make_launch(*j.pilot, j.plan, po, sl.s, cus, kPilotSlack * budget_ms / stride);
-        enqueue_query(*j.pilot, sl.c, sl.s, sl.lane, sl.host_ctr);
+        enqueue_query(*j.pilot, sl.c, sl.s, sl.lane);
         running_pilots++;
     } else {
         sl.c = make_launch(*j.pp, j.plan, j.opts, sl.s, cus);
-        enqueue_query(*j.pp, sl.c, sl.s, sl.lane, sl.host_ctr);
+        enqueue_query(*j.pp, sl.c, sl.s, sl.lane);
         running_full++;
         j.charged_ms = j.predicted_ms > 0 ? j.predicted_ms : 0;
         running_pred += j.charged_ms;
@@ -279,13 +278,10 @@ void Server::finish(Slot &sl, int status, const std::string &err)
     d.predicted_ms = j.predicted_ms;
     if (status == 0) {
         try {
-            fill_result(j.opts, sl.host_ctr, d.result);
-            float t_all = 0, t_hub = 0;
-            HIP_CHECK(hipEventElapsedTime(&t_all, sl.lane.ev[0], sl.lane.ev[3]));
-            HIP_CHECK(hipEventElapsedTime(&t_hub, sl.lane.ev[0], sl.lane.ev[1]));
-            d.result.t_enum_ms = t_all;
-            d.result.t_hub_ms = t_hub;
-            d.result.t_lds_ms = lds_phase_ms(sl.lane);
+            fill_result(j.opts, sl.lane.rec, d.result);
+            fill_times(sl.lane.rec, device, d.result);
+            // per-class times are beep_count's
+            for (double &t : d.result.t_lds_class_ms) t = 0;
             if (sl.c.out.buf && j.opts.match_buf && d.result.n_written) {
                 HIP_CHECK(hipMemcpyAsync(j.opts.match_buf, sl.c.out.buf,
                                          d.result.n_written * (uint64_t)j.plan.L * sizeof(uint32_t),
@@ -351,23 +347,19 @@ void Server::run()
         for (auto &sp : slots) {
             Slot &sl = *sp;
             if (!sl.busy) continue;
-            const hipError_t q = hipEventQuery(sl.lane.ev[3]);
+            const hipError_t q = hipEventQuery(sl.lane.done);
             if (q == hipErrorNotReady) continue;
             progress = true;
             if (q == hipSuccess && sl.job.piloting) {
                 // pilot done: predict, then refuse or run the query on the same lane
                 running_pilots--;
                 sl.busy_pilot = false;
-                float t_hub = 0, t_lds = 0;
-                bool ok = hipEventElapsedTime(&t_hub, sl.lane.ev[0], sl.lane.ev[1]) == hipSuccess;
-                for (int i = 0; ok && i < sl.lane.ncls; i++) {
-                    float t = 0;
-                    ok = hipEventElapsedTime(&t, sl.lane.ev[0], sl.lane.cls_done[i]) == hipSuccess;
-                    t_lds = std::max(t_lds, t);
-                }
+                beep_result pr{};
+                fill_times(sl.lane.rec, device, pr);
+                const double t_hub = pr.t_hub_ms, t_lds = pr.t_lds_ms;
                 // hub and LDS phases run side by side; each scales by its own stride
-                const double t = std::max((double)t_hub * hub_sample_stride(stride) / stride, (double)t_lds);
-                const bool stopped = sl.host_ctr[kCtrStop] != 0;
+                const double t = std::max(t_hub * hub_sample_stride(stride) / stride, t_lds);
+                const bool stopped = sl.lane.rec[kCtrStop] != 0;
                 // the pilot shared the GPU with the other running queries: its
                 // time over the average number of busy lanes estimates it alone
                 uint64_t busy_now = 1;
@@ -376,7 +368,7 @@ void Server::run()
                     busy_now = std::max<uint64_t>(st.running, 1);
                 }
                 const double share = 0.5 * (double)(sl.job.busy_at_pilot + busy_now);
-                const double pred = (stopped || !ok) ? INFINITY : (double)t * stride / share;
+                const double pred = stopped ? INFINITY : (double)t * stride / share;
                 predicted[sl.job.sig] = pred;
                 sl.job.predicted_ms = pred;
                 sl.job.piloting = false;
@@ -500,8 +492,6 @@ Server::~Server()
     cv_in.notify_all();
     if (worker.joinable()) worker.join();
     (void)hipSetDevice(device);
-    for (auto &sp : slots)
-        if (sp->host_ctr) (void)hipHostFree(sp->host_ctr);
     slots.clear();
     rootq.clear();
     variants.clear();
@@ -534,7 +524,6 @@ Server *server_create(const Graph *g, const beep_server_opts &o)
     for (int i = 0; i < o.lanes; i++) {
         auto sl = std::make_unique<Server::Slot>();
         sl->lane.create(o.device, 1);
-        HIP_CHECK(hipHostMalloc((void **)&sl->host_ctr, sizeof(unsigned long long) * kCtrWords));
         s->slots.push_back(std::move(sl));
     }
     Server *raw = s.get();

@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 
 #include "engine.hpp"
@@ -92,26 +93,23 @@ void Lane::create(int dev, int ns)
     nside = std::max(1, std::min(ns, kMaxSide));
     HIP_CHECK(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
     for (int i = 0; i < nside; i++) HIP_CHECK(hipStreamCreateWithFlags(&side[i], hipStreamNonBlocking));
-    for (auto &e : ev) HIP_CHECK(hipEventCreate(&e));
-    for (int i = 0; i < nside; i++) HIP_CHECK(hipEventCreate(&side_done[i]));
-    for (auto &e : cls_done) HIP_CHECK(hipEventCreate(&e));
-    for (auto &e : cls_start) HIP_CHECK(hipEventCreate(&e));
+    HIP_CHECK(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+    HIP_CHECK(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    for (int i = 0; i < nside; i++) HIP_CHECK(hipEventCreateWithFlags(&side_done[i], hipEventDisableTiming));
+    HIP_CHECK(hipHostMalloc((void **)&rec, sizeof(unsigned long long) * kRecWords));
 }
 
 Lane::~Lane()
 {
     if (device >= 0) (void)hipSetDevice(device);
-    for (auto &e : ev)
+    for (auto e : {fork, done})
         if (e) (void)hipEventDestroy(e);
     for (auto &e : side_done)
-        if (e) (void)hipEventDestroy(e);
-    for (auto &e : cls_start)
-        if (e) (void)hipEventDestroy(e);
-    for (auto &e : cls_done)
         if (e) (void)hipEventDestroy(e);
     for (auto &s : side)
         if (s) (void)hipStreamDestroy(s);
     if (main) (void)hipStreamDestroy(main);
+    if (rec) (void)hipHostFree(rec);
 }
 
 DevPrep::~DevPrep()
@@ -135,9 +133,14 @@ int device_cus(int device)
 
 uint64_t wall_clock_khz(int device)
 {
-    int khz = 0;
+    static std::atomic<int> known[64];  // by device, 0: not asked yet
+    const bool keep = device >= 0 && device < 64;
+    int khz = keep ? known[device].load(std::memory_order_relaxed) : 0;
+    if (khz > 0) return (uint64_t)khz;
     HIP_CHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
-    return khz > 0 ? (uint64_t)khz : 100000ull;
+    if (khz <= 0) khz = 100000;
+    if (keep) known[device].store(khz, std::memory_order_relaxed);
+    return (uint64_t)khz;
 }
 
 static void upload_variant(Variant &V, int device)
@@ -233,6 +236,11 @@ static std::vector<uint64_t> hub_scan_ranges(const Variant &V, const std::vector
 
 void upload(Prep &pp, int device, int p_skip_split, uint64_t arena_budget)
 {
+    if (pp.dev && pp.dev->device == device && pp.dev->roots.skip_split == p_skip_split && pp.var->dev &&
+        (arena_budget == 0 || pp.dev->roots.arena_budget == arena_budget)) {
+        HIP_CHECK(hipSetDevice(device));
+        return;
+    }
     int ndev = 0;
     HIP_CHECK(hipGetDeviceCount(&ndev));
     if (device < 0 || device >= ndev) throw Error(BEEP_EDEVICE, "no such HIP device");
@@ -597,7 +605,7 @@ LaunchCfg make_launch(const Prep &pp, const Plan &p, const beep_opts &o, const S
     LaunchCfg c{};
     const bool buf = o.emit == BEEP_EMIT_BUFFER && o.match_cap && s.dbuf;
     c.out = KOut{s.ctr + kCtrAcc, buf ? s.dbuf : nullptr, buf ? o.match_cap : 0, s.ctr + kCtrDeadline,
-                 s.ctr + kCtrStop, s.prof};
+                 s.ctr + kCtrStop, s.ctr + kCtrStamp, s.prof};
     c.kp = make_kplan(p, o.emit != BEEP_EMIT_NONE ? 1 : 0, o.build_mode);
     c.kg = KGraph{V.dev->ocol, V.dev->vinfo, V.dev->htab, V.asc};
     c.nlev = p.L > 3 ? p.L - 3 : 1;
@@ -692,11 +700,10 @@ void enqueue_hubs(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStrea
     }
 }
 
-// LDS lane classes, one launch each, round-robin over the given streams.
-int enqueue_lds_classes(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStream_t *streams, int nst,
-                        hipEvent_t *cls_done, uint8_t *cls_lg)
+// LDS lane classes, one launch each.
+void enqueue_lds_classes(const Prep &pp, const LaunchCfg &c, const Scratch &s, hipStream_t st)
 {
-    if (c.kp.L < 3) return 0;
+    if (c.kp.L < 3) return;
     const DevRoots &R = pp.dev->roots;
     uint32_t b = 0;
     int cls = 0;
@@ -704,39 +711,28 @@ int enqueue_lds_classes(const Prep &pp, const LaunchCfg &c, const Scratch &s, hi
         int lg = std::max<int>(pp.batch_lanes_log2[b], c.lmin);
         uint32_t e = b + 1;
         while (e < R.nbatches && std::max<int>(pp.batch_lanes_log2[e], c.lmin) == lg) e++;
-        if (cls >= 32) throw Error(BEEP_ERANGE, "too many lane classes");
+        if (cls >= Lane::kMaxClasses) throw Error(BEEP_ERANGE, "too many lane classes");
         unsigned long long *cur = s.ctr + kCtrLds + (uint64_t)cls * kCurWords;
-        HIP_CHECK(launch_lds_batches(lg, pp.dev->cus, streams[cls % nst], c.kg, c.kp, R.recs, R.batch_first,
-                                     R.batch_count, b, e, cur, c.out));
-        if (cls_done) {
-            HIP_CHECK(hipEventRecord(cls_done[cls], streams[cls % nst]));
-            cls_lg[cls] = (uint8_t)lg;
-        }
+        HIP_CHECK(launch_lds_batches(lg, pp.dev->cus, st, c.kg, c.kp, R.recs, R.batch_first, R.batch_count, b, e, cur,
+                                     c.out));
         b = e;
         cls++;
     }
-    return cls;
 }
 
-void class_times(const Lane &lane, double *t_by_lg)
+void fill_times(const unsigned long long *rec, int device, beep_result &res)
 {
-    for (int i = 0; i < 8; i++) t_by_lg[i] = 0;
-    for (int i = 0; i < lane.ncls; i++) {
-        float t = 0;
-        HIP_CHECK(hipEventElapsedTime(&t, lane.cls_start[i], lane.cls_done[i]));
-        if (lane.cls_lg[i] < 8) t_by_lg[lane.cls_lg[i]] += t;
+    const double khz = (double)wall_clock_khz(device);
+    const unsigned long long t0 = rec[kCtrT0], *st = rec + kCtrWords;
+    auto ms = [&](unsigned long long a, unsigned long long b) { return b > a ? (double)(b - a) / khz : 0.0; };
+    res.t_enum_ms = ms(t0, rec[kCtrTEnd]);
+    res.t_hub_ms = ms(t0, st[kStampHub]);
+    res.t_lds_ms = 0;
+    for (int lg = 0; lg < 8; lg++) {
+        const bool ran = lg <= 6 && st[kStampEnd + lg];
+        res.t_lds_class_ms[lg] = ran ? ms(st[kStampStart + lg], st[kStampEnd + lg]) : 0.0;
+        if (ran) res.t_lds_ms = std::max(res.t_lds_ms, ms(t0, st[kStampEnd + lg]));
     }
-}
-
-double lds_phase_ms(const Lane &lane)
-{
-    float tmax = 0;
-    for (int i = 0; i < lane.ncls; i++) {
-        float t = 0;
-        HIP_CHECK(hipEventElapsedTime(&t, lane.ev[0], lane.cls_done[i]));
-        tmax = std::max(tmax, t);
-    }
-    return tmax;
 }
 
 // Lane classes of a query: [batch begin, end) and lane class, with the bitmap
@@ -765,12 +761,13 @@ static std::vector<LdsClass> lds_classes(const Prep &pp, const LaunchCfg &c)
     return out;
 }
 
-void enqueue_query(const Prep &pp, const LaunchCfg &c, const Scratch &s, Lane &lane, unsigned long long *host_ctr)
+void enqueue_query(const Prep &pp, const LaunchCfg &c, const Scratch &s, Lane &lane)
 {
     hipStream_t st = lane.main;
     HIP_CHECK(launch_begin_sequence(s.ctr, kCtrTotal, kCtrDeadline, c.deadline_ticks, c.deadline_ticks_lds, st));
     if (s.prof) HIP_CHECK(launch_fill_zero(s.prof, s.cap.prof_words * 8, st));
-    HIP_CHECK(hipEventRecord(lane.ev[0], st));
+    // Times come from stamps that the kernels write (KOut::stamp): an event on
+    // either side of every launch cost the host and the queues about 10 us each.
     // With hub roots, the heaviest LDS lane class starts on the main stream at
     // once (a wait on another stream's event costs tens of microseconds); the
     // hub rounds, the longest chain of dependent kernels, are queued next, on
@@ -795,49 +792,39 @@ void enqueue_query(const Prep &pp, const LaunchCfg &c, const Scratch &s, Lane &l
     const int nstreams = 1 + lane.nside;
     std::vector<bool> waited(nstreams, false);
     waited[0] = true;
+    bool forked = false;
+    if (hubs || order.size() > 1) {  // before anything else is queued on main
+        HIP_CHECK(hipEventRecord(lane.fork, st));
+        forked = true;
+    }
     auto side_stream = [&](int k) -> hipStream_t {
         if (!waited[k]) {
-            HIP_CHECK(hipStreamWaitEvent(lane.side[k - 1], lane.ev[0], 0));
+            HIP_CHECK(hipStreamWaitEvent(lane.side[k - 1], lane.fork, 0));
             waited[k] = true;
         }
         return lane.side[k - 1];
     };
-    lane.ncls = 0;
-    hipStream_t hs = nullptr;
     for (size_t n = 0; n < order.size(); n++) {
         const LdsClass &lc = cls[order[n]];
         // class n >= 1 on side stream first_side + n - 1 while there is one
         const int first_side = hubs ? 2 : 1;
         const int k = n > 0 && first_side + (int)n - 1 < nstreams ? first_side + (int)n - 1 : 0;
         hipStream_t sk = k == 0 ? st : side_stream(k);
-        const int i = lane.ncls++;
         unsigned long long *cur = s.ctr + kCtrLds + (uint64_t)order[n] * kCurWords;
         // without hub kernels beside them, the classes take the registers
         // for 7 workgroups per CU
-        HIP_CHECK(hipEventRecord(lane.cls_start[i], sk));
         HIP_CHECK(launch_lds_batches(lc.lg, pp.dev->cus, sk, c.kg, c.kp, R.recs, R.batch_first, R.batch_count,
                                      lc.b0, lc.b1, cur, c.out, !hubs));
-        HIP_CHECK(hipEventRecord(lane.cls_done[i], sk));
-        lane.cls_lg[i] = (uint8_t)lc.lg;
-        if (n == 0) {
-            hs = side_stream(1);
-            if (hubs) enqueue_hubs(pp, c, s, hs);
-            HIP_CHECK(hipEventRecord(lane.ev[1], hs));
-        }
+        if (n == 0 && hubs) enqueue_hubs(pp, c, s, side_stream(1));
     }
-    if (!hs) {
-        hs = side_stream(1);
-        if (hubs) enqueue_hubs(pp, c, s, hs);
-        HIP_CHECK(hipEventRecord(lane.ev[1], hs));
-    }
-    for (int k = 1; k < nstreams; k++)
+    if (order.empty() && hubs) enqueue_hubs(pp, c, s, side_stream(1));
+    for (int k = 1; forked && k < nstreams; k++)
         if (waited[k]) {
             HIP_CHECK(hipEventRecord(lane.side_done[k - 1], lane.side[k - 1]));
             HIP_CHECK(hipStreamWaitEvent(st, lane.side_done[k - 1], 0));
         }
-    HIP_CHECK(hipEventRecord(lane.ev[2], st));
-    HIP_CHECK(hipMemcpyAsync(host_ctr, s.ctr, sizeof(unsigned long long) * kCtrWords, hipMemcpyDeviceToHost, st));
-    HIP_CHECK(hipEventRecord(lane.ev[3], st));
+    HIP_CHECK(launch_end_sequence(s.ctr, kCtrWords, kCtrTEnd, s.ctr + kCtrStamp, lane.rec, st));
+    HIP_CHECK(hipEventRecord(lane.done, st));
 }
 
 void fill_result(const beep_opts &o, const unsigned long long *acc, beep_result &res)
@@ -919,17 +906,10 @@ void count_on_device(Prep &pp, const Plan &p, const beep_opts &o, beep_result &r
     own_scratch(d, scratch_needs(pp, p, o, d.cus));
     d.lane.create(d.device, Lane::kMaxSide);
     const LaunchCfg c = make_launch(pp, p, o, d.scratch, d.cus);
-    unsigned long long acc[kCtrWords];
-    enqueue_query(pp, c, d.scratch, d.lane, acc);
+    enqueue_query(pp, c, d.scratch, d.lane);
     HIP_CHECK(hipStreamSynchronize(d.lane.main));
-    float t_all = 0, t_hub = 0;
-    HIP_CHECK(hipEventElapsedTime(&t_all, d.lane.ev[0], d.lane.ev[3]));
-    HIP_CHECK(hipEventElapsedTime(&t_hub, d.lane.ev[0], d.lane.ev[1]));
-    fill_result(o, acc, res);
-    res.t_enum_ms = t_all;
-    res.t_hub_ms = t_hub;
-    res.t_lds_ms = lds_phase_ms(d.lane);
-    class_times(d.lane, res.t_lds_class_ms);
+    fill_result(o, d.lane.rec, res);
+    fill_times(d.lane.rec, d.device, res);
     if (c.out.buf && o.match_buf && res.n_written)
         HIP_CHECK(hipMemcpy(o.match_buf, c.out.buf, res.n_written * (uint64_t)p.L * sizeof(uint32_t),
                             hipMemcpyDeviceToHost));
@@ -971,6 +951,7 @@ struct Batch {
     hipEvent_t fork = nullptr, t0 = nullptr, t1 = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    unsigned long long *rec = nullptr;  // one record (kRecWords) per query, pinned
     ~Batch()
     {
         if (device >= 0) (void)hipSetDevice(device);
@@ -987,6 +968,7 @@ struct Batch {
         for (auto s : branch)
             if (s) (void)hipStreamDestroy(s);
         if (s0) (void)hipStreamDestroy(s0);
+        if (rec) (void)hipHostFree(rec);
     }
 };
 
@@ -1052,6 +1034,7 @@ Batch *batch_create(Prep *const *preps, const Plan *const *plans, const beep_opt
         b->dwork = dev_upload(w);
         b->nwork = (uint32_t)w.size();
         b->cursor = dev_alloc<unsigned long long>(kCurWords * std::max<size_t>(1, b->cls_lg.size()));
+        HIP_CHECK(hipHostMalloc((void **)&b->rec, sizeof(unsigned long long) * kRecWords * n));
         HIP_CHECK(hipStreamCreateWithFlags(&b->s0, hipStreamNonBlocking));
         b->branch.resize(n + b->cls_lg.size() + 1);
         b->done.resize(n + b->cls_lg.size() + 1);
@@ -1100,6 +1083,9 @@ static void batch_capture(Batch &b)
         HIP_CHECK(hipEventRecord(b.done[n + k], sk));
     }
     for (int i = 0; i < n + ncls; i++) HIP_CHECK(hipStreamWaitEvent(b.s0, b.done[i], 0));
+    for (int i = 0; i < n; i++)
+        HIP_CHECK(launch_end_sequence(b.scr[i].ctr, kCtrWords, kCtrTEnd, b.scr[i].ctr + kCtrStamp,
+                                      b.rec + (size_t)i * kRecWords, b.s0));
     HIP_CHECK(hipStreamEndCapture(b.s0, &b.graph));
     HIP_CHECK(hipGraphInstantiate(&b.exec, b.graph, nullptr, nullptr, 0));
 }
@@ -1115,17 +1101,13 @@ void batch_run(Batch &b, beep_result *res, double *t_ms)
     HIP_CHECK(hipGraphLaunch(b.exec, b.s0));
     HIP_CHECK(hipEventRecord(b.t1, b.s0));
     const int n = (int)b.preps.size();
-    std::vector<unsigned long long> acc((size_t)n * kCtrWords);
-    for (int i = 0; i < n; i++)
-        HIP_CHECK(hipMemcpyAsync(acc.data() + (size_t)i * kCtrWords, b.scr[i].ctr,
-                                 sizeof(unsigned long long) * kCtrWords, hipMemcpyDeviceToHost, b.s0));
     HIP_CHECK(hipStreamSynchronize(b.s0));
     float t = 0;
     HIP_CHECK(hipEventElapsedTime(&t, b.t0, b.t1));
     for (int i = 0; i < n; i++) {
         if (res) {
             memset(&res[i], 0, sizeof(beep_result));
-            fill_result(b.opts[i], acc.data() + (size_t)i * kCtrWords, res[i]);
+            fill_result(b.opts[i], b.rec + (size_t)i * kRecWords, res[i]);
             res[i].t_enum_ms = t;
         }
     }

@@ -206,6 +206,13 @@ __device__ __forceinline__ void prof_add(const KOut &out, int phase, uint32_t sl
     }
 }
 
+// Stamps the end of a workgroup (one thread calls it).
+__device__ __forceinline__ void stamp_end(const KOut &out, int word)
+{
+    if (out.stamp)
+        atomicMax(&out.stamp[(blockIdx.x % kStripes) * kLine + word], (unsigned long long)wall_clock64());
+}
+
 // Flushes per-lane accumulators: one atomic per wave and counter, into the
 // wave's stripe.
 __device__ __forceinline__ void flush_acc(const KOut &out, uint64_t cnt, uint64_t hs, uint64_t hx)
@@ -1215,6 +1222,8 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
     uint64_t cnt = 0, hs = 0, hx = 0;
     const uint64_t dl = out.dl[1];
     const uint64_t t_start = wall_clock64();
+    constexpr int kLg = P == 64 ? 6 : P == 32 ? 5 : P == 16 ? 4 : P == 8 ? 3 : P >> 1;
+    if (out.stamp && blockIdx.x == 0 && tid == 0) out.stamp[kStampStart + kLg] = t_start;
     uint32_t parts = 0;  // thread 0's claim state
     for (;;) {
         if (tid == 0) {
@@ -1234,7 +1243,10 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
         process_batch<P, WALK>(g, pl, v, recs, batch_first[b], batch_count[b], out, dl, cnt, hs, hx);
     }
     flush_acc(out, cnt, hs, hx);
-    if (tid == 0) prof_add(out, 0, blockIdx.x, t_start);
+    if (tid == 0) {
+        prof_add(out, 0, blockIdx.x, t_start);
+        stamp_end(out, kStampEnd + kLg);
+    }
 }
 
 // One persistent launch over the LDS batches of several prepared queries.
@@ -1440,6 +1452,7 @@ __global__ __launch_bounds__(kBlock) void hub_encode_kernel(KGraph g, const HubR
         flush_acc(out, cnt, 0, 0);
         if (lane == 0) prof_add(out, 1, blockIdx.x * (kBlock / 64) + wv, t_start);
     }
+    if (tid == 0) stamp_end(out, kStampHub);
 }
 
 // Slices of hubs with few kept rows (K <= kSliceKept): a workgroup takes up to
@@ -1574,7 +1587,10 @@ __global__ __launch_bounds__(kBlock) void hub_slice_kernel(KGraph g, const HubRe
     if (CLOSED)
         for (uint32_t i = tid; i < K; i += kBlock)
             if (sCnt[i]) atomicAdd(&c2[h.ioff - i0 + i], sCnt[i]);
-    if (tid == 0) prof_add(out, 1, blockIdx.x, t_start);
+    if (tid == 0) {
+        prof_add(out, 1, blockIdx.x, t_start);
+        stamp_end(out, kStampHub);
+    }
 }
 
 // Sums closed_count over the items' |C_2| counters.
@@ -1589,6 +1605,7 @@ __global__ __launch_bounds__(kBlock) void hub_closed_kernel(const HubRec *__rest
         if (c) cnt += closed_count(closed, c, hubs[hub_of_item[i]].d);
     }
     flush_acc(out, cnt, 0, 0);
+    if (threadIdx.x == 0) stamp_end(out, kStampHub);
 }
 
 // Copies a W-word row (HBM) into a wave's buffer, lane i taking words i,
@@ -2126,6 +2143,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
         }
         flush_acc(out, cnt, hs, hx);
         if (lane == 0) prof_add(out, 2, wslot, t_start);
+        if (threadIdx.x == 0) stamp_end(out, kStampHub);
         return;
     }
 
@@ -2238,6 +2256,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
     }
     flush_acc(out, cnt, hs, hx);
     if (lane == 0) prof_add(out, 1, wslot, t_start);
+    if (threadIdx.x == 0) stamp_end(out, kStampHub);
 }
 
 // Hub items of 5-vertex plans with paired levels (KPlan::pair, L = 5; W5): with
@@ -2431,6 +2450,7 @@ __global__ __launch_bounds__(kBlock, 4) void hub_pair5_kernel(KPlan pl, const Hu
         }
         flush_acc(out, cnt, 0, 0);
         if (lane == 0) prof_add(out, 2, wslot, t_start);
+        if (threadIdx.x == 0) stamp_end(out, kStampHub);
         return;
     }
     constexpr uint32_t kClaim = 4;  // items per cursor claim
@@ -2491,6 +2511,7 @@ __global__ __launch_bounds__(kBlock, 4) void hub_pair5_kernel(KPlan pl, const Hu
     }
     flush_acc(out, cnt, 0, 0);
     if (lane == 0) prof_add(out, 1, wslot, t_start);
+    if (threadIdx.x == 0) stamp_end(out, kStampHub);
 }
 
 // ------------------------------------------------------------ launchers
@@ -2614,8 +2635,35 @@ __global__ void begin_sequence_kernel(unsigned long long *ctr, uint64_t n, uint6
             const uint64_t t = i == dl ? ticks_hub : ticks_lds;
             v = t ? (unsigned long long)wall_clock64() + t : ~0ull;
         }
+        if (i == dl + 3) v = (unsigned long long)wall_clock64();  // the sequence's start
         ctr[i] = v;
     }
+}
+
+// Last kernel of a launch sequence: copies the n result words to the record in
+// host memory, with the time now as word t_end, followed by the stamps' maxima
+// over their stripes.  (A copy command waits for the kernels on a queue of its
+// own and took 15 to 20 us from the last kernel's end to the host.)
+__global__ void end_sequence_kernel(const unsigned long long *ctr, uint32_t n, uint32_t t_end,
+                                    const unsigned long long *stamp, unsigned long long *rec)
+{
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+        rec[i] = i == t_end ? (unsigned long long)wall_clock64() : ctr[i];
+    if (threadIdx.x < (uint32_t)kStampWords) {
+        unsigned long long m = 0;
+        for (int s = 0; s < kStripes; s++) {
+            const unsigned long long x = stamp[s * kLine + threadIdx.x];
+            m = x > m ? x : m;
+        }
+        rec[n + threadIdx.x] = m;
+    }
+}
+
+hipError_t launch_end_sequence(const unsigned long long *ctr, uint32_t n, uint32_t t_end, const unsigned long long *stamp,
+                               unsigned long long *rec, hipStream_t st)
+{
+    hipLaunchKernelGGL(end_sequence_kernel, dim3(1), dim3(kBlock), 0, st, ctr, n, t_end, stamp, rec);
+    return hipGetLastError();
 }
 
 hipError_t launch_begin_sequence(unsigned long long *ctr, uint64_t n, uint64_t dl, uint64_t ticks_hub,

@@ -226,6 +226,10 @@ struct KOut {
     // DFS once theirs has passed, and set *stop.
     const unsigned long long *dl = nullptr;
     unsigned long long *stop = nullptr;
+    // kStripes lines of wall_clock64() stamps, cleared before: latest end of a hub
+    // kernel (kStampHub), of lane class lg's launch (kStampEnd + lg), and in
+    // stripe 0 the class's start (kStampStart + lg); or null.
+    unsigned long long *stamp = nullptr;
     // Optional busy-time accumulators (wall_clock64 ticks), kProfPhases x
     // kProfSlots: phase 0 LDS workgroups, 1 hub waves on their own items, 2 hub
     // waves on donated subtrees, 3 the LDS workgroups' staging and bitmap
@@ -233,6 +237,9 @@ struct KOut {
     // phases 0-2 by compute unit (slot = XCC, shader engine, array, CU).
     unsigned long long *prof = nullptr;
 };
+
+// Words of a stamp stripe (KOut::stamp).
+constexpr int kStampHub = 0, kStampEnd = 1, kStampStart = 8, kStampWords = 15;
 
 constexpr int kProfSlots = 4096, kProfPhases = 5, kProfCuPhase = 4;
 
