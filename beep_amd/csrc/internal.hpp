@@ -1,6 +1,7 @@
 // internal.hpp -- host-side data structures shared by the libbeep sources.
 #pragma once
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <cstring>
@@ -55,6 +56,37 @@ void parallel_for(size_t n, F &&f, size_t grain = 1 << 14)
     for (unsigned t = 1; t < T; ++t) th.emplace_back(worker);
     worker();
     for (auto &x : th) x.join();
+}
+
+// Dynamic parallel loop over the rows [v0, v1) of a CSR (rp: row starts) in
+// chunks of about equal entries + rows: degree-sorted or power-law graphs put
+// half of their entries into a few thousand neighbouring rows, which a chunk of
+// a fixed number of rows gave to one thread (orientation of 200,000 vertices:
+// most of 13.5 ms, with 16 threads).
+template <class F>
+void parallel_rows(const std::vector<uint64_t> &rp, size_t v0, size_t v1, F &&f)
+{
+    if (v0 >= v1) return;
+    auto pos = [&](size_t v) { return rp[v] - rp[v0] + (v - v0); };
+    const uint64_t total = pos(v1);
+    // (a chunk is worth starting a thread for)
+    const uint64_t per = std::max<uint64_t>(1 << 15, total / ((uint64_t)host_threads() * 8) + 1);
+    const size_t chunks = (size_t)((total + per - 1) / per);
+    auto bound = [&](size_t c) {  // first row at or past position c * per
+        if (c >= chunks) return v1;
+        size_t lo = v0, hi = v1;
+        while (lo < hi) {
+            const size_t mid = (lo + hi) / 2;
+            if (pos(mid) < (uint64_t)c * per) lo = mid + 1; else hi = mid;
+        }
+        return lo;
+    };
+    parallel_for(chunks, [&](size_t b, size_t e) {
+        for (size_t c = b; c < e; c++) {
+            const size_t x = bound(c), y = bound(c + 1);
+            if (x < y) f(x, y);
+        }
+    }, 1);
 }
 
 // ---------------------------------------------------------------- graph

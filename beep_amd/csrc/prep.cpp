@@ -74,7 +74,7 @@ int peel(const Graph &g, int min_qdeg, std::vector<uint64_t> &rp, std::vector<ui
             }
         }, 256);
         std::vector<uint64_t> nrp(n + 1, 0);
-        parallel_for(n, [&](size_t b, size_t e) {
+        parallel_rows(rp, 0, n, [&](size_t b, size_t e) {
             for (size_t v = b; v < e; v++) {
                 uint64_t c = 0;
                 for (uint64_t x = rp[v]; x < rp[v + 1]; x++) c += keep[x];
@@ -83,7 +83,7 @@ int peel(const Graph &g, int min_qdeg, std::vector<uint64_t> &rp, std::vector<ui
         });
         for (uint32_t v = 0; v < n; v++) nrp[v + 1] += nrp[v];
         std::vector<uint32_t> ncol(nrp[n]);
-        parallel_for(n, [&](size_t b, size_t e) {
+        parallel_rows(rp, 0, n, [&](size_t b, size_t e) {
             for (size_t v = b; v < e; v++) {
                 uint64_t o = nrp[v];
                 for (uint64_t x = rp[v]; x < rp[v + 1]; x++)
@@ -136,12 +136,12 @@ std::shared_ptr<Variant> make_variant(const Graph &g, int min_qdeg, int asc_flag
     const uint32_t nslices = V.m > (1ull << 30) ? 16 : 1;
     for (uint32_t sl = 0; sl < nslices; sl++) {
     const size_t s0 = (size_t)n * sl / nslices, s1 = (size_t)n * (sl + 1) / nslices;
-    parallel_for(s1 - s0, [&](size_t b, size_t e) {
+    parallel_rows(rp, s0, s1, [&](size_t b, size_t e) {
         // rows are sorted on 64-bit keys (degree, or its complement for desc
         // rows, above the id): the order of the comparison on (deg, id)
         // without a degree lookup per comparison
         std::vector<uint64_t> key;
-        for (size_t u = s0 + b; u < s0 + e; u++) {
+        for (size_t u = b; u < e; u++) {
             const uint64_t rb = rp[u], re = rp[u + 1];
             const uint32_t du = deg[u];
             uint32_t lo = 0, hc = 0;
@@ -161,7 +161,7 @@ std::shared_ptr<Variant> make_variant(const Graph &g, int min_qdeg, int asc_flag
             // degrees followed by equal degrees with smaller ids.
             V.hlen[u] = asc ? du - lo : hc;
         }
-    }, 4096);
+    });
     if (nslices > 1) progress("orientation: rows %zu..%zu done", s0, s1);
     }
     uint32_t maxd = 0;
@@ -260,7 +260,7 @@ void build_work(Prep &pp_, const Plan &p, uint32_t sample_stride)
             for (uint64_t x = rp[u]; x < rp[u + 1]; x++) acc += 4ull * (deg(V.col[x]) + 2);
         }
         bytes.fetch_add(acc);
-    }, 1024);
+    }, pp->roots.size() > 4096 ? 64 : 1024);  // roots come heaviest first
     pp->alg_bytes = bytes.load();
     // Work list.  With above_split plans a root keeps only its suffix of
     // larger keys (asc rows), which drops the skipped x_1 < split items and
@@ -393,7 +393,7 @@ void class_figures(Prep &pp)
         bu[bi] = units;
         bb[bi] = bytes;
     }
-    }, 256);
+    }, pp.batches.size() > 1024 ? 64 : 256);
     for (size_t bi = 0; bi < pp.batches.size(); bi++) {
         const int lg = pp.batch_lanes_log2[bi];
         pp.cls_roots[lg] += pp.batches[bi].count;

@@ -169,7 +169,7 @@ static void upload_variant(Variant &V, int device)
             // lookup tables: vertex v's larger-key range [hbeg, hbeg + hlen)
             // in the 2 hlen slots at 2 hbeg, linear probing (KGraph::htab)
             std::vector<uint32_t> ht(2 * V.m, 0u);
-            parallel_for(V.n, [&](size_t b, size_t e2) {
+            parallel_rows(V.rowptr, 0, V.n, [&](size_t b, size_t e2) {
                 for (size_t v = b; v < e2; v++) {
                     const uint64_t hb = vi[v].hbeg, hl = vi[v].hlen;
                     const uint32_t size = (uint32_t)(2 * hl);
@@ -181,7 +181,7 @@ static void upload_variant(Variant &V, int device)
                         t[s] = w + 1;
                     }
                 }
-            }, 1024);
+            });
             dg->htab = dev_upload(ht);
         }
         progress("variant uploaded (%llu entries)", (unsigned long long)V.m);
