@@ -564,19 +564,23 @@ static KPlan make_kplan(const Plan &p, int emit, int build_mode)
     k.nested = p.upper_rows && p.L >= 4 ? 1 : 0;
     for (int l = 2; l < p.L; l++) {
         if (p.qmask[l]) k.reads_rows = 1;
-        // a summed last level leaves its constraint on x_{L-2} to the sum
-        const bool summed = k.tail && l == p.L - 1;
-        const LevelWork w = reduce_level(p, l, p.qmask[l], summed ? p.smask[l] & ~(1u << (l - 1)) : p.smask[l],
-                                         summed ? l - 1 : l);
-        k.lev[l] = w.rq | w.rs << 16;
-        k.lev[kMaxLevels + l] = w.rx | w.base << 16;
+        const LevelWork w = reduce_level(p, l, p.qmask[l], p.smask[l], l);
         if (w.rq != 1u << (l - 1) || w.rs || w.rx || (l > 2 && (int)w.base != l - 1)) k.nested = 0;
+        const bool last = l == p.L - 1 && p.L >= 4;
+        const uint32_t own = 1u << (l - 1);
+        const LevelWork f = last ? reduce_level(p, l, p.qmask[l] & ~own, p.smask[l] & ~own, l - 1) : w;
+        k.lev[l] = f.rq | f.rs << 16;
+        k.lev[kMaxLevels + l] = f.rx | f.base << 16;
+        if (last) {
+            k.leaf_row = (p.qmask[l] & own) ? 1 : 0;
+            k.leaf_gt = (p.smask[l] & own) ? 1 : 0;
+            k.leaf_x = !k.leaf_row && !k.leaf_gt;  // no row holds its own vertex
+        }
     }
-    k.tail_gt = k.tail && ((p.smask[p.L - 1] >> (p.L - 2)) & 1u) ? 1 : 0;
     if (emit == BEEP_EMIT_NONE && p.L == 3) k.closed = kClosedC;
     if (k.tail && p.L == 4) {
-        if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 2u << 16) k.closed = k.tail_gt ? kClosedPairs : kClosedOrdered;
-        if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 1u << 1 && !k.tail_gt) k.closed = kClosedRow;
+        if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 2u << 16) k.closed = k.leaf_gt ? kClosedPairs : kClosedOrdered;
+        if (k.lev[3] == 0 && k.lev[kMaxLevels + 3] == 1u << 1 && !k.leaf_gt) k.closed = kClosedRow;
     }
     k.kept = p.rows_above_split;
     // every pair found is one candidate x_2 of its smaller index, and the count

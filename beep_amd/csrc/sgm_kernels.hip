@@ -730,7 +730,7 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
                 if (lx >= o) fin += y;
             }
             const uint32_t ftot = __shfl(fin, P - 1, P);
-            if (pl.tail_gt) return (uint64_t)sc * (ftot - fin) + pairs_in_word(S, F);
+            if (pl.leaf_gt) return (uint64_t)sc * (ftot - fin) + pairs_in_word(S, F);
             return (uint64_t)sc * ftot - (uint64_t)__popcll(S & F);
         };
 
@@ -810,6 +810,7 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
         }
         int l = 3;
         uint32_t pos = 0;
+        uint64_t F = 0, hpre = 0;  // last level: what x_{L-2} does not change
         for (;;) {
             if (++spins == kClockEvery) {
                 spins = 0;
@@ -829,6 +830,13 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
                 pos = (uint32_t)xget(l - 1) + 1u;
                 continue;
             }
+            if (l == L - 1 && pos == 0u) {
+                F = own ? level_word(l) : 0ull;
+                if (pl.emit) {
+                    hpre = hash_step(hash_seed(L), 0, rr.u);
+                    for (int q = 1; q < l - 1; q++) hpre = hash_step(hpre, q, A[xget(q)]);
+                }
+            }
             uint64_t vv = l == 3 ? x2s : own ? sStk[(l - 3) * kBlock + tid] : 0ull;
             const uint32_t pw = pos >> 6;
             if (w < pw) vv = 0ull;
@@ -845,12 +853,17 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
             const uint64_t vf = __shfl(vv, f, P);
             const uint32_t xi = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
             sX[(l - 1) * kBlock + tid] = (uint16_t)xi;
-            const uint64_t t = own ? level_word(l) : 0ull;
             if (l == L - 1) {
+                uint64_t t = F;
+                if (pl.leaf_row && t) t &= E[xi * W + w];
+                if (pl.leaf_gt) t &= gt_mask(xi, w);
+                if (pl.leaf_x) t &= ~bit_at(xi, w);
                 cnt += (uint64_t)__popcll(t);
-                if (pl.emit && t) emit_word(out, pl, l, rr.u, A, t, w, xget, hs, hx);
+                if (pl.emit && t)
+                    emit_bits(out, l, rr.u, A, hash_step(hpre, l - 1, A[xi]), t, w, xget, hs, hx);
                 pos = xi + 1u;
             } else {
+                const uint64_t t = own ? level_word(l) : 0ull;
                 sStk[(l - 2) * kBlock + tid] = t;
                 ++l;
                 pos = 0;
@@ -1690,12 +1703,13 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
     extern __shared__ __align__(16) uint64_t hsm[];
     __shared__ uint32_t sX[kBlock / 64][kMaxLevels];
     __shared__ uint32_t sWlo[kBlock / 64][kMaxLevels];
-    __shared__ uint32_t sQM[kMaxLevels], sSM[kMaxLevels];
+    __shared__ uint32_t sQM[kMaxLevels], sSM[kMaxLevels], sLev[2 * kMaxLevels];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     if (tid < kMaxLevels) {
         sQM[tid] = pl.qmask[tid];
         sSM[tid] = pl.smask[tid];
     }
+    if (tid < 2 * kMaxLevels) sLev[tid] = pl.lev[tid];
     __syncthreads();
     const int L = pl.L;
     const int nlev = L > 3 ? L - 3 : 1;
@@ -1731,27 +1745,41 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
         }
         return lo;
     };
-    // The masks go first, then the rows (x_1's from LDS first), and a lane
-    // whose word is already empty loads no further row word.
+    // C_l (for l = L-1 >= 3: without x_{l-1}'s constraints, KPlan::lev) from its
+    // base level's set.  The masks go first, then the rows (x_1's from LDS
+    // first), and a lane whose word is already empty loads no further row word.
     auto level_word = [&](int l, uint32_t w) -> uint64_t {
-        uint64_t t = valid_mask(w, d);
-        for (int s = 1; s < l; s++) t &= ~bit_at(xget(s), w);
-        uint32_t sm = sSM[l];
-        while (sm) {
-            const int s = __builtin_ctz(sm);
-            sm &= sm - 1;
+        const uint32_t a = sLev[l], b = sLev[kMaxLevels + l], base = b >> 16;
+        uint64_t t = !base ? valid_mask(w, d) : w >= sWlo[wv][base] ? my[(uint64_t)(base - 2) * wmax + w] : 0ull;
+        uint32_t m = b & 0xffffu;
+        while (m) {
+            const int s = __builtin_ctz(m);
+            m &= m - 1;
+            t &= ~bit_at(xget(s), w);
+        }
+        m = a >> 16;
+        while (m) {
+            const int s = __builtin_ctz(m);
+            m &= m - 1;
             t &= gt_mask(xget(s), w);
         }
-        uint32_t qm = sQM[l];
-        if (row1 && (qm & 2u)) {
+        m = a & 0xffffu;
+        if (row1 && (m & 2u)) {
             t &= e1[w];
-            qm &= ~2u;
+            m &= ~2u;
         }
-        while (qm && t) {
-            const int q = __builtin_ctz(qm);
-            qm &= qm - 1;
+        while (m && t) {
+            const int q = __builtin_ctz(m);
+            m &= m - 1;
             t &= Eh[(uint64_t)(xget(q) - rlo) * W + w];
         }
+        return t;
+    };
+    // x_{L-2} = x's part of the last level
+    auto leaf_word = [&](uint64_t t, uint32_t x, uint32_t w) -> uint64_t {
+        if (pl.leaf_gt) t &= gt_mask(x, w);
+        if (pl.leaf_x) t &= ~bit_at(x, w);
+        if (pl.leaf_row && t) t &= Eh[(uint64_t)(x - rlo) * W + w];
         return t;
     };
 
@@ -1761,7 +1789,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
     //   sum_x |F n (x, inf)| = |S||F| - sum_w (|S_w| |F_{<=w}| - pairs_w(S, F))
     //   sum_x |F \ {x}|      = |S||F| - |S n F|
     // (words below both S's and F's first word add nothing to either).
-    const bool tail_gt = pl.tail && ((sSM[L - 1] >> (L - 2)) & 1u);
+    const bool tail_gt = pl.tail && pl.leaf_gt;
     auto tail_count = [&](int l, uint32_t pos0, uint32_t hi2) {
         const int lv = l - 1;
         const uint32_t wl = sWlo[wv][l - 1];
@@ -1782,23 +1810,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
             uint64_t S = 0, F = 0;
             if (w < W && w >= w0) {
                 if (w >= ws) S = my[(uint64_t)(l - 3) * wmax + w] & ~lt_mask(pos0, w) & lt_mask(hi2, w);
-                if (w >= fl) {
-                    F = valid_mask(w, d);
-                    uint32_t qm = sQM[l];
-                    while (qm && F) {  // lanes whose word is already empty load nothing
-                        const int q = __builtin_ctz(qm);
-                        qm &= qm - 1;
-                        if (q == 1 && row1) F &= e1[w];
-                        else F &= Eh[(uint64_t)(xget(q) - rlo) * W + w];
-                    }
-                    for (int s = 1; s < lv; s++) F &= ~bit_at(xget(s), w);
-                    uint32_t sm = sSM[l] & ~(1u << lv);
-                    while (sm) {
-                        const int s = __builtin_ctz(sm);
-                        sm &= sm - 1;
-                        F &= gt_mask(xget(s), w);
-                    }
-                }
+                if (w >= fl) F = level_word(l, w);
             }
             const uint32_t sc = (uint32_t)__popcll(S);
             const uint32_t fin = wave_incl_scan((uint32_t)__popcll(F)) + carry;
@@ -2039,7 +2051,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
         int l = 3;
         uint32_t pos = pos0;
         for (;;) {
-            if (++spins == kClockEvery) {
+            if (++spins >= kClockEvery) {
                 spins = 0;
                 if (past(dl)) break;  // the next claim records the stop
             }
@@ -2052,6 +2064,62 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
             }
             if (PAIR && l == L - 2) {  // levels L-3..L-1 at once
                 if (pair_count(l)) break;  // the next claim records the stop
+                if (l == 3) break;
+                --l;
+                pos = xget(l - 1) + 1u;
+                continue;
+            }
+            if (l == L - 1 && R == 1u) {
+                // Rows of at most 64 words: the whole last level here, F once, four
+                // x_{L-2}'s rows in flight (each is a dependent load from L2 or
+                // beyond: W5's hashed matches on hubs of 865 waited 1.5 us a row)
+                const uint32_t w = lane, lo = sWlo[wv][l - 1];
+                uint64_t v = (w < W && w >= lo) ? my[(uint64_t)(l - 3) * wmax + w] & ~lt_mask(pos, w) : 0ull;
+                if (l == 3) v &= lt_mask(hi2, w);
+                const uint64_t F = w < W ? level_word(l, w) : 0ull;
+                uint64_t hpre = 0;
+                if (pl.emit) {
+                    hpre = hash_step(hash_seed(L), 0, u);
+                    for (int q = 1; q < l - 1; q++) hpre = hash_step(hpre, q, A[xget(q)]);
+                }
+                for (;;) {
+                    uint32_t x[4];
+                    uint64_t t[4];
+                    int n = 0;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const uint64_t bal = __ballot(v != 0ull);
+                        x[k] = 0;
+                        if (bal) {
+                            const int f = __builtin_ctzll(bal);
+                            const uint64_t vf = (uint64_t)lane_u32((uint32_t)(v >> 32), f) << 32 | lane_u32((uint32_t)v, f);
+                            x[k] = ((uint32_t)f << 6) + (uint32_t)__builtin_ctzll(vf);
+                            if (lane == f) v &= v - 1ull;
+                            n++;
+                        }
+                    }
+                    if (n == 0) break;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) t[k] = k < n ? leaf_word(F, x[k], w) : 0ull;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        if (k >= n) break;
+                        cnt += (uint64_t)__popcll(t[k]);
+                        if (pl.emit) {
+                            if (out.buf) {
+                                if (lane == 0) sX[wv][l - 1] = x[k];
+                                wave_lds_sync();
+                            }
+                            if (t[k])
+                                emit_bits(out, l, u, A, hash_step(hpre, l - 1, A[x[k]]), t[k], w, xget, hs, hx);
+                        }
+                    }
+                    spins += 4;
+                    if (spins >= kClockEvery) {
+                        spins = 0;
+                        if (past(dl)) break;  // the next claim records the stop
+                    }
+                }
                 if (l == 3) break;
                 --l;
                 pos = xget(l - 1) + 1u;
@@ -2088,7 +2156,7 @@ __global__ __launch_bounds__(kBlock, PAIR ? 3 : 1) void hub_dfs_kernel(KGraph g,
                     const uint32_t w = rr * 64 + lane;
                     if (w >= W) break;
                     if (w < lo) continue;
-                    const uint64_t t = level_word(l, w);
+                    const uint64_t t = leaf_word(level_word(l, w), xi, w);
                     cnt += (uint64_t)__popcll(t);
                     if (pl.emit && t) emit_word(out, pl, l, u, A, t, w, xget, hs, hx);
                 }

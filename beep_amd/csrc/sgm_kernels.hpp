@@ -58,15 +58,18 @@ struct KPlan {
     // What is left to do for level l when the walk starts from an earlier
     // level's set: C_l = C_base with the rows rq, the bounds rs and the
     // exclusions rx applied (base 0: from all of [0, d)).  lev[l] holds
-    // rq | rs << 16, lev[kMaxLevels + l] holds rx | base << 16.
+    // rq | rs << 16, lev[kMaxLevels + l] holds rx | base << 16.  For the last
+    // level (L >= 4) they leave x_{L-2}'s constraints out: the rest, F, is the
+    // same for every x_{L-2}, and leaf_row, leaf_gt and leaf_x say whether
+    // x_{L-2} adds its row, the bound and its exclusion.
     uint32_t lev[2 * kMaxLevels];
+    int32_t leaf_row, leaf_gt, leaf_x;
     // Every level is C_l = C_{l-1} n E[x_{l-1}] over bitmaps without mirrored
     // bits (cliques): one row per step, no bounds, no exclusions.
     int32_t nested;
     // x_2 candidates of one DFS item of the LDS batches (see lds_items).
     uint32_t chunk;
     int32_t reads_rows;  // some level intersects with a bitmap row
-    int32_t tail_gt;     // tail: L-2 is in smask[L-1]
     // Count-only plans whose count below x_1 is a function of |C_2| = c and
     // the root's row length d alone (diamond: c (c - 1) / 2); see closed_count.
     int32_t closed;

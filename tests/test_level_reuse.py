@@ -66,6 +66,10 @@ def test_reduced_levels_give_the_full_levels_sets(seed):
                     E[i][j] = 1
                     E[j][i] = 0 if p.upper_rows else 1
         red = [None, None] + [reduce_level(p, l, qm, sm, above, qm[l], sm[l], l) for l in range(2, L)]
+        # the last level: without x_{L-2}'s constraints, which are applied on top
+        leaf_row, leaf_gt = L - 2 in qm[L - 1], L - 2 in sm[L - 1]
+        if L >= 4:
+            red[L - 1] = reduce_level(p, L - 1, qm, sm, above, qm[L - 1] - {L - 2}, sm[L - 1] - {L - 2}, L - 2)
 
         def full(l, x):
             return {i for i in range(d) if i not in x[1:l] and all(E[x[q]][i] for q in qm[l])
@@ -78,6 +82,10 @@ def test_reduced_levels_give_the_full_levels_sets(seed):
             base, rq, rs, rx = red[l]
             got = {i for i in (sets[base] if base else range(d)) if all(E[x[q]][i] for q in rq)
                    and all(i > x[s] for s in rs) and all(i != x[t] for t in rx)}
+            if l == L - 1 and L >= 4:
+                y = x[L - 2]
+                got = {i for i in got if (not leaf_row or E[y][i]) and (not leaf_gt or i > y)
+                       and (leaf_row or leaf_gt or i != y)}
             assert got == want, (name, l, x)
             if l == L - 1:
                 return
