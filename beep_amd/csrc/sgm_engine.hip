@@ -589,6 +589,7 @@ static KPlan make_kplan(const Plan &p, int emit, int build_mode)
     // levels an item walks below x_2: none (one pass over the row's words, or
     // the count itself), one, two, or more
     const int walked = p.L - (k.tail ? 1 : 0) - (k.pair ? 2 : 0) - 3;
+    k.deep = walked >= 2;
     k.chunk = walked <= 0 ? kNoSplit : walked == 1 ? 16u : walked == 2 ? 8u : 2u;
     // an emitted tuple costs its two 64-bit mixes in the lane that found it
     // (4-clique on 1.1M vertices, hashed: 535 us with 64, 427 with 16, 381 with 4)

@@ -28,6 +28,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "internal.hpp"
@@ -422,6 +423,12 @@ __device__ __forceinline__ LdsView lds_view(unsigned char *smem, const LdsLayout
     return v;
 }
 
+// The items a workgroup takes of a batch: those congruent to part modulo parts
+// (see lds_batch_kernel).
+struct Share {
+    uint32_t part, parts;
+};
+
 // Rows whose index range holds item e: the largest j with pre[j] <= e (pre
 // ascends, pre[n] > e).
 __device__ __forceinline__ uint32_t find_row(const uint32_t *pre, uint32_t n, uint32_t e)
@@ -499,8 +506,8 @@ __device__ uint32_t lds_items(const KPlan &pl, const LdsView &v, uint32_t sumd, 
 // that still have work are out of candidates: the two phases' instructions are
 // then paid by at least half of the lanes they serve.
 template <int WT, bool EMIT>
-__device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uint32_t items, const KOut &out,
-                            uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
+__device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uint32_t items, Share sh,
+                            const KOut &out, uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
 {
     const int tid = threadIdx.x;
     const int L = pl.L;
@@ -552,7 +559,7 @@ __device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, ui
                 const uint32_t rank = bits_below(m);
                 uint32_t first = 0;
                 if (rank == 0) first = atomicAdd(&v.sMisc[M_NEXT], (uint32_t)__popcll(m));
-                const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + rank;
+                const uint32_t item = ((uint32_t)__builtin_amdgcn_readfirstlane((int)first) + rank) * sh.parts + sh.part;
                 if (item >= items) {
                     live = false;
 #pragma unroll
@@ -652,8 +659,8 @@ __device__ void clique_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, ui
 // i of every set, the next candidate is one ballot over the group's words, and
 // the sets of the levels above are kept in the thread's LDS stack.
 template <int P>
-__device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uint32_t items, const KOut &out,
-                           uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
+__device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uint32_t items, Share sh,
+                           const KOut &out, uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
 {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -672,7 +679,7 @@ __device__ void group_walk(const KPlan &pl, const LdsView &v, uint32_t sumd, uin
                 item = 0xffffffffu;
                 mark_stop(out);
             } else {
-                item = atomicAdd(&sMisc[M_NEXT], 1u);
+                item = atomicAdd(&sMisc[M_NEXT], 1u) * sh.parts + sh.part;
             }
         }
         item = __shfl(item, 0, P);
@@ -1192,7 +1199,7 @@ __device__ uint32_t build_batch(const KGraph &g, const KPlan &pl, const LdsView 
 enum { kWalkAny = 0, kWalkGroup = 1, kWalkLane = 2, kWalkLaneEmit = 3, kWalkNone = 4 };
 template <int PC, int WALK>
 __device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v,
-                              const RootRec *__restrict__ recs, uint32_t first, uint32_t nr,
+                              const RootRec *__restrict__ recs, uint32_t first, uint32_t nr, Share sh,
                               const KOut &out, uint64_t dl, uint64_t &cnt, uint64_t &hs, uint64_t &hx)
 {
     const int tid = threadIdx.x;
@@ -1210,12 +1217,16 @@ __device__ void process_batch(const KGraph &g, const KPlan &pl, const LdsView &v
     constexpr int WT = PC <= 8 ? PC : 1, kLg = WT == 8 ? 3 : WT >> 1;
     const int walk = WALK != kWalkAny ? WALK
                      : PC <= 8 && lds_lane_walk(pl, kLg) ? (pl.emit ? kWalkLaneEmit : kWalkLane) : kWalkGroup;
-    if (PC <= 8 && walk == kWalkLane) clique_walk<WT, false>(pl, v, sumd, items, out, dl, cnt, hs, hx);
-    else if (PC <= 8 && walk == kWalkLaneEmit) clique_walk<WT, true>(pl, v, sumd, items, out, dl, cnt, hs, hx);
-    else group_walk<PC>(pl, v, sumd, items, out, dl, cnt, hs, hx);
+    if (PC <= 8 && walk == kWalkLane) clique_walk<WT, false>(pl, v, sumd, items, sh, out, dl, cnt, hs, hx);
+    else if (PC <= 8 && walk == kWalkLaneEmit) clique_walk<WT, true>(pl, v, sumd, items, sh, out, dl, cnt, hs, hx);
+    else group_walk<PC>(pl, v, sumd, items, sh, out, dl, cnt, hs, hx);
     __syncthreads();
 }
 
+// A class of few batches leaves CUs idle while its workgroups walk deep plans
+// (W5's hashed matches on 20,000 vertices: 16 batches of the widest class, 3.2
+// of 3.4 ms).  Each of its batches is then taken by `parts` workgroups, which
+// all build it and walk every parts-th item.
 // MinWaves > 1: the compiler keeps the registers to that many waves per SIMD
 // (7 workgroups per CU instead of 5 for the narrow classes, at the cost of a
 // few bytes of spill); used when no hub kernels of the query share the CUs.
@@ -1224,7 +1235,7 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
                                                            const RootRec *__restrict__ recs,
                                                            const uint32_t *__restrict__ batch_first,
                                                            const uint32_t *__restrict__ batch_count,
-                                                           uint32_t b0, uint32_t b1,
+                                                           uint32_t b0, uint32_t b1, uint32_t parts,
                                                            unsigned long long *cursor, LdsLayout lay,
                                                            KOut out)
 {
@@ -1237,23 +1248,25 @@ __global__ __launch_bounds__(kBlock, MinWaves) void lds_batch_kernel(KGraph g, K
     const uint64_t t_start = wall_clock64();
     constexpr int kLg = P == 64 ? 6 : P == 32 ? 5 : P == 16 ? 4 : P == 8 ? 3 : P >> 1;
     if (out.stamp && blockIdx.x == 0 && tid == 0) out.stamp[kStampStart + kLg] = t_start;
-    uint32_t parts = 0;  // thread 0's claim state
+    uint32_t seen = 0;  // thread 0's claim state
     for (;;) {
         if (tid == 0) {
             uint64_t bb = 0, be = 0;
             if (past(dl)) {
-                v.sMisc[M_BATCH] = b1;
+                v.sMisc[M_BATCH] = ~0u;
                 mark_stop(out);
-            } else if (claim_striped(cursor, b1 - b0, blockIdx.x % kStripes, parts, 1, bb, be)) {
-                v.sMisc[M_BATCH] = b0 + (uint32_t)bb;
+            } else if (claim_striped(cursor, (uint64_t)(b1 - b0) * parts, blockIdx.x % kStripes, seen, 1, bb, be)) {
+                v.sMisc[M_BATCH] = (uint32_t)bb;
             } else {
-                v.sMisc[M_BATCH] = b1;
+                v.sMisc[M_BATCH] = ~0u;
             }
         }
         __syncthreads();
-        const uint32_t b = v.sMisc[M_BATCH];
-        if (b >= b1) break;
-        process_batch<P, WALK>(g, pl, v, recs, batch_first[b], batch_count[b], out, dl, cnt, hs, hx);
+        const uint32_t t = v.sMisc[M_BATCH];
+        if (t == ~0u) break;
+        const uint32_t b = b0 + t / parts;
+        process_batch<P, WALK>(g, pl, v, recs, batch_first[b], batch_count[b], Share{t % parts, parts}, out, dl, cnt, hs,
+                               hx);
     }
     flush_acc(out, cnt, hs, hx);
     if (tid == 0) {
@@ -1293,8 +1306,8 @@ __global__ __launch_bounds__(kBlock) void lds_multi_kernel(const MultiQuery *__r
         uint64_t cnt = 0, hs = 0, hx = 0;
         const uint64_t dl = q.out.dl[1];
         const uint64_t t_start = wall_clock64();
-        process_batch<P, kWalkAny>(q.g, pl, v, q.recs, q.batch_first[w.batch], q.batch_count[w.batch], q.out, dl, cnt, hs,
-                         hx);
+        process_batch<P, kWalkAny>(q.g, pl, v, q.recs, q.batch_first[w.batch], q.batch_count[w.batch], Share{0, 1}, q.out,
+                                   dl, cnt, hs, hx);
         flush_acc(q.out, cnt, hs, hx);
         if (tid == 0) prof_add(q.out, 0, blockIdx.x, t_start);
     }
@@ -2614,6 +2627,7 @@ struct LdsLaunchCache {
 };
 
 constexpr int kBesideHubs = 3;
+constexpr uint32_t kMaxParts = 16;
 
 template <int P, int MinWaves, int WALK>
 static hipError_t launch_lds_p(int cus, size_t lds, hipStream_t st, const KGraph &g, const KPlan &pl,
@@ -2629,10 +2643,12 @@ static hipError_t launch_lds_p(int cus, size_t lds, hipStream_t st, const KGraph
     // 826 with 6.
     if (MinWaves == 1 && occ > kBesideHubs) occ = kBesideHubs;
     int grid = occ * cus;
-    if ((uint32_t)grid > b1 - b0) grid = (int)(b1 - b0);
+    uint32_t parts = 1;
+    if (pl.deep && WALK != kWalkNone) parts = std::min(kMaxParts, std::max(1u, (uint32_t)grid / (b1 - b0)));
+    if ((uint64_t)grid > (uint64_t)(b1 - b0) * parts) grid = (int)((b1 - b0) * parts);
     if (grid < 1) grid = 1;
     hipLaunchKernelGGL((lds_batch_kernel<P, MinWaves, WALK>), dim3(grid), dim3(kBlock), lds, st, g, pl, recs, bf,
-                       bc, b0, b1, cursor, lay, out);
+                       bc, b0, b1, parts, cursor, lay, out);
     return hipGetLastError();
 }
 

@@ -69,6 +69,7 @@ struct KPlan {
     int32_t nested;
     // x_2 candidates of one DFS item of the LDS batches (see lds_items).
     uint32_t chunk;
+    int32_t deep;        // two or more levels are walked below x_2
     int32_t reads_rows;  // some level intersects with a bitmap row
     // Count-only plans whose count below x_1 is a function of |C_2| = c and
     // the root's row length d alone (diamond: c (c - 1) / 2); see closed_count.
