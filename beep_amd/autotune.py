@@ -4,7 +4,7 @@ Sweeps, per prepared query, the minimum DFS group width (``lanes``: automatic
 from the bitmap width, or 4 / 8 / 16 lanes) and the donation threshold of hub
 items (|C_2| above which a level-2 subtree is donated), then, with the best of
 those, the LDS bitmap build (automatic, range streaming only, neighbour search
-only); each setting is timed with the library's HIP events and the fastest is
+only); each setting is timed by the library's device times and the fastest is
 kept.  Results can be cached in a JSON file keyed by graph shape and query.
 """
 import json

@@ -7,18 +7,19 @@
 //
 // Here the same enumeration is organised for wave64:
 //  * bitmap words are 64 bits; a DFS group is P lanes of one wave (P = 1..64,
-//    lane i of a group owns words i, i+P, ...), the next candidate is found
-//    with one wave ballot over the group's words and one ds_bpermute;
+//    lane i of a group owns word i), the next candidate is found with one wave
+//    ballot over the group's words; cliques are walked one lane an item;
 //  * roots whose bitmap fits are packed into LDS batches: a workgroup stages
 //    the rows, an LDS hash (vertex -> row index) and the bitmaps, then its
-//    groups claim (root, x_1) items from an LDS counter;
-//  * the bitmap is built by streaming, for every row vertex v, only the part
-//    of v's oriented row that holds neighbours with a larger (degree, id) key
-//    and probing the hash -- each adjacent pair inside N(u) is found once and
-//    both bits are set -- instead of d^2/2 binary searches; when that part is
-//    long next to the root's degree, the root's neighbours on v's larger-key
-//    side are looked up in a hash table of it instead (one load each);
-//  * roots too large for LDS ("hubs") keep bitmap + hash in an HBM arena built
+//    lanes or groups claim items -- an x_1 with some of its x_2 -- from an LDS
+//    counter; counts that follow from |C_2| need no walk;
+//  * a root's adjacent pairs are found once each, from the endpoint with the
+//    smaller (degree, id) key: by streaming the part of its oriented row that
+//    holds larger keys, or, when that part is long next to what it can pair
+//    with, by looking those vertices up in a hash table of it (one load each)
+//    -- instead of d^2/2 binary searches;
+//  * roots too large for LDS ("hubs") keep their bitmap in an HBM arena, built
+//    by workgroups that each own a slice of a hub where few rows are kept, else
 //    by grid-wide kernels, and every wave of the grid takes (hub, x_1) items,
 //    so one hub is shared by the whole GPU.
 //

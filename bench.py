@@ -9,12 +9,12 @@ sequence in sgm mode (counting, no tuple output -- the reference's sgm).
 Reported:
   value        matches/s = (count_4clique + count_diamond) / device time
   roofline     the dominant kernel, lds_batch_kernel<1, *> (LDS batches of
-               roots with at most 64 row entries; its two occupancy
-               instantiations are one kernel here): the bytes its launches must read
+               roots with at most 64 row entries; its instantiations
+               are one kernel here): the bytes its launches must read
                at least once (root records and rows, the row vertices' records
                and bitmap-build scan ranges; computed on the host per lane
-               class) over its device time, measured with HIP events on the
-               stream it runs on, against the 8 TB/s HBM peak.  "traffic" is
+               class) over its device time, from the device-clock stamps of
+               its first and last workgroups, against the 8 TB/s HBM peak.  "traffic" is
                its measured HBM bytes per step (committed rocprofv3
                FETCH_SIZE / WRITE_SIZE summary); "b_alg_per_step" is
                sum over roots of 4(d(u)+2) + sum over neighbours 4(d(v)+2)

@@ -167,7 +167,7 @@ typedef struct {
     uint32_t q0_head_larger; /* neighbours of Q0[0] with a larger (degree, id) key */
     /* Per lane class lg (LDS batches of roots with at most 64 << lg row
      * entries; one lds_batch_kernel launch each): roots, bitmap-build work
-     * units (scan-range entries streamed, or root neighbours looked up) and
+     * units (scan-range entries streamed, or row entries looked up) and
      * the bytes the launch must read at least once (root records and rows,
      * row-vertex records and scan ranges, batch arrays). */
     uint64_t lds_class_roots[8], lds_class_units[8], lds_class_bytes[8];
@@ -203,23 +203,24 @@ typedef struct {
                                such as W5: ranges of the paired pass instead) */
     uint32_t donate_min;    /* donation threshold: min |C_2| of a donated subtree
                                (not used by the paired-pass ranges) */
-    int timing;             /* 1 = record HIP events around the enumeration */
+    int timing;             /* kept for callers; times always come from the device clock */
     double deadline_ms;     /* > 0: stop the enumeration this long after it starts on
                                the device; the result is then partial and marked stopped */
     int profile;            /* 1 = busy-time balance of workgroups / waves (beep_count) */
-    int build_mode;         /* BEEP_BUILD_*: how LDS bitmaps find adjacent row pairs */
+    int build_mode;         /* BEEP_BUILD_*: how LDS bitmaps and hub slices find adjacent
+                               row pairs */
 } beep_opts;
 
-#define BEEP_BUILD_AUTO 0   /* stream ranges, look up the root's neighbours when a
-                               range is over 32x the root's degree */
+#define BEEP_BUILD_AUTO 0   /* stream ranges, look the entries a row can pair with up
+                               when its range is over 4x as long */
 #define BEEP_BUILD_SCAN 1   /* always stream the row vertices' larger-key ranges */
-#define BEEP_BUILD_SEARCH 2 /* always binary-search the root's neighbours */
+#define BEEP_BUILD_SEARCH 2 /* always look the entries up in the ranges' tables */
 
 typedef struct {
     uint64_t count;         /* "------------- Counter = N" */
     uint64_t hash_sum, hash_xor;
     uint64_t n_emitted, n_written;
-    double t_enum_ms;       /* first enumeration launch -> counter readback */
+    double t_enum_ms;       /* first enumeration kernel -> result record written */
     double t_hub_ms, t_lds_ms; /* device time of the hub and LDS phases */
     uint64_t donations;     /* subtrees donated through the ring */
     uint64_t stopped;       /* 1: the deadline passed; counts are partial */
