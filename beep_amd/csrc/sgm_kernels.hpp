@@ -175,7 +175,9 @@ struct HubRec {
 
 // Rows [row0, row0 + rows) of a hub's bitmap build, for hubs with at most
 // kSliceKept kept rows (of those that keep rows from the split on only, with
-// both bits of every pair): their vertices fit an LDS table.
+// both bits of every pair): their vertices fit an LDS table. A limit of 512 or
+// 2,048 rows measures the same (diamond on 1.1M vertices 359 us, a served mix
+// of ten queries 4.35 ms).
 struct SliceRec {
     uint32_t hub, row0, rows;
 };
